@@ -55,6 +55,18 @@ __device__ __forceinline__ void global_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// Publishes everything this workgroup stored before its last global_barrier(): the L2 writeback
+// of an agent-scope release, the wait for it, then the flag.  The wait is written out: after the
+// barrier's own wait the compiler takes nothing to be outstanding and puts none between the
+// writeback and the flag's store of a release atomic, so that the flag could pass a line still on
+// its way to memory and a consumer on another XCD read that line's old contents.
+__device__ __forceinline__ void publish_flag(uint32_t *flag, uint32_t value)
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Load of data that another workgroup published (a flag release after its stores): an
 // agent-scope atomic load is served from the coherence point, so it cannot hit a stale line
 // in this CU's L1 or this XCD's L2.  (One thread's acquire after the flag invalidates the

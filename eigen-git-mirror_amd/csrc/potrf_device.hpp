@@ -511,7 +511,7 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
             publish_lower_tiles(smem, Wp);
         }
         global_barrier();  // every wave's stores of the image have reached L2
-        if (tid == 0) __hip_atomic_store(flag, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) publish_flag(flag, epoch);
         if (f < 0) lds_to_block(smem, Ck, lda, bs);  // read by later launches only
         return;
     }

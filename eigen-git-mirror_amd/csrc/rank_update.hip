@@ -252,9 +252,7 @@ __global__ __launch_bounds__(64) void rank_update_kernel(double *__restrict__ L,
     if (!GIVENS && l == 0) bbeta[ib] = beta;
     // publish: the wave's stores (coefficients, beta) complete before the flag
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    if (l == 0)
-        __hip_atomic_store(flags + ib, kRuDone | (failed ? kRuFail : 0u) | (uint32_t)ncol, __ATOMIC_RELEASE,
-                           __HIP_MEMORY_SCOPE_AGENT);
+    if (l == 0) publish_flag(flags + ib, kRuDone | (failed ? kRuFail : 0u) | (uint32_t)ncol);
 }
 
 __global__ __launch_bounds__(256) void ru_reset_kernel(uint32_t *flags, int nblk, int *ticket, int *info)

@@ -188,3 +188,32 @@ def test_batched_argument_errors(dev):
     assert L.mi_dpotrf_batched_async(h.ptr, b"L", 8, 2, p, 8, 64, vp(None)) == -8
     assert L.mi_dpotrf_batched_async(h.ptr, b"L", 8, 0, p, 8, 64, q) == 0
     torch.cuda.synchronize()
+
+
+def test_batched_factor_repeats_bit_for_bit(dev):
+    """A batch of several rounds of workgroups (256 systems of four blocks), factored many times
+    with three inputs in turn over the same workspace: the panel images that the row roles read
+    must be the ones published for this factorization, never a line of an earlier one's."""
+    n, batch = 512, 256
+    gen = torch.Generator(device=dev).manual_seed(3)
+    x = [torch.randn(batch, n, 8, dtype=torch.float64, device=dev, generator=gen) for _ in range(3)]
+    mats = []
+    for xi in x:
+        k = torch.zeros(batch, n, n, dtype=torch.float64, device=dev)
+        for j in range(8):
+            k += (xi[:, :, None, j] - xi[:, None, :, j]) ** 2
+        k = torch.exp(-k / 4.5)
+        k.diagonal(dim1=1, dim2=2).add_(1e-2)
+        mats.append(k)
+    h = mi_llt.Handle().bind_stream()
+    info = torch.zeros(batch, dtype=torch.int32, device=dev)
+    first, differ = {}, torch.zeros((), dtype=torch.int64, device=dev)
+    for it in range(600):
+        a = mi_llt.colmajor_batched(mats[it % 3])
+        mi_llt.potrf_batched_async_(a, info, handle=h)
+        if it < 3:
+            first[it] = a
+        else:
+            differ += (a != first[it % 3]).sum() + (info != 0).sum()
+    assert int(differ) == 0
+    assert h.status() == 0
