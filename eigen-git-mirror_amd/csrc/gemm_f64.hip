@@ -86,59 +86,98 @@ void launch_lower_to_upper(const T *W, int64_t ldw, int64_t n, T *A, int64_t lda
 template void launch_lower_to_upper<double>(const double *, int64_t, int64_t, double *, int64_t, hipStream_t);
 template void launch_lower_to_upper<float>(const float *, int64_t, int64_t, float *, int64_t, hipStream_t);
 
-// Symmetric L1 norm (LLT.h:442-453).  For lower storage column c sums |A(i,c)|, i >= c
-// (col(c).tail) plus |A(c,j)|, j < c (row(c).head); upper storage mirrors it.  The column
-// part is a workgroup reduction per column (coalesced), the row part one thread per c
-// (coalesced across threads); both in a fixed order, so the result is deterministic.
-__global__ __launch_bounds__(256) void sy_colpart_kernel(const double *__restrict__ A, int64_t lda, int64_t n,
-                                                         bool upper, double *__restrict__ colsum)
+// Symmetric L1 norm (LLT.h:442-453): the largest column sum of |A| of the symmetric matrix, from
+// one triangle, each stored element read once.  A workgroup takes a 64 x 64 tile (ti, tj) of the
+// stored triangle (of its lower mirror: ti >= tj) and writes its sums along both directions:
+// part[tj][64 ti + i] gets what the tile adds to the columns 64 ti.. of the symmetric matrix,
+// part[ti][64 tj + j] what it adds to 64 tj.., and a diagonal tile both together -- so column c
+// receives exactly one value per tile index u, part[u][c], added in that order by the second
+// kernel (deterministic).  Bound by the read of the triangle (a thread's 16 loads go out
+// together); n = 1024 took 228 us and n = 4001 950 us with one thread walking each row.
+template <typename T>
+__global__ __launch_bounds__(256) void sy_l1_tile_kernel(const T *__restrict__ A, int64_t lda, int64_t n, bool upper,
+                                                         double *__restrict__ part, double *__restrict__ out)
 {
-    __shared__ double red[256];
-    const int64_t c = blockIdx.x;
-    const int64_t lo = upper ? 0 : c, hi = upper ? c : n;
-    double s = 0.0;
-    for (int64_t i = lo + threadIdx.x; i < hi; i += 256) s += fabs(A[i + c * lda]);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    __shared__ double t[64][65];  // |element| at [second index in storage order][row in storage]
+    __shared__ double red[2][4][64];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *out = 0.0;  // the second kernel's atomic maximum starts here
+    int ti, tj;
+    lower_tile((int)blockIdx.x, ti, tj);
+    // storage rows r0.. (contiguous), storage columns c0..
+    const int64_t r0 = 64 * (int64_t)(upper ? tj : ti), c0 = 64 * (int64_t)(upper ? ti : tj);
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    double v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const int64_t r = r0 + tx, c = c0 + 16 * ty + q;
+        const bool in = r < n && c < n && (upper ? r <= c : r >= c);
+        const double x = (double)A[(in ? r : 0) + (in ? c : 0) * lda];
+        v[q] = in ? fabs(x) : 0.0;
     }
-    if (threadIdx.x == 0) colsum[c] = red[0];
-}
-
-__global__ __launch_bounds__(256) void sy_rowpart_kernel(const double *__restrict__ A, int64_t lda, int64_t n,
-                                                         bool upper, double *__restrict__ colsum)
-{
-    const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const int64_t lo = upper ? c : 0, hi = upper ? n : c;
+    // along the storage rows: this thread's 16 columns, then the four waves in order
     double s = 0.0;
-    for (int64_t j = lo; j < hi; ++j) s += fabs(A[c + j * lda]);
-    colsum[c] += s;
-}
-
-__global__ __launch_bounds__(256) void max_reduce_kernel(const double *__restrict__ v, int64_t n, double *out)
-{
-    __shared__ double red[256];
-    double m = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += 256) m = fmax(m, v[i]);
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + s]);
-        __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        t[16 * ty + q][tx] = v[q];
+        // a diagonal tile's column sums below take the diagonal element; the row sums skip it
+        s += (ti == tj && tx == 16 * ty + q) ? 0.0 : v[q];
     }
-    if (threadIdx.x == 0) *out = red[0];
+    red[0][ty][tx] = s;
+    __syncthreads();
+    // along the storage columns: thread (column tx, quarter ty of the rows)
+    s = 0.0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) s += t[tx][16 * ty + q];
+    red[1][ty][tx] = s;
+    __syncthreads();
+    if (ty < 2) {
+        const double a = (red[ty][0][tx] + red[ty][1][tx]) + (red[ty][2][tx] + red[ty][3][tx]);
+        if (ti == tj) {
+            red[ty][0][tx] = a;
+        } else {
+            // ty 0: sums of storage rows r0 + tx; ty 1: of storage columns c0 + tx
+            const int64_t c = (ty == 0 ? r0 : c0) + tx;
+            const int u = ty == 0 ? (int)(c0 / 64) : (int)(r0 / 64);
+            if (c < n) part[(int64_t)u * n + c] = a;
+        }
+    }
+    if (ti != tj) return;
+    __syncthreads();
+    if (ty == 0 && r0 + tx < n) part[(int64_t)ti * n + r0 + tx] = red[0][0][tx] + red[1][0][tx];
 }
 
-void launch_sy_l1norm(const double *A, int64_t lda, int64_t n, bool upper, double *colsum, double *out,
-                      hipStream_t s)
+// Column sums (64 columns per workgroup, four interleaved quarters of the tile index) and
+// their maximum: non-negative doubles order as their bit patterns, and a NaN sum is skipped, as
+// the reference's `if (abs_col_sum > m_l1_norm)` skips it.
+__global__ __launch_bounds__(256) void sy_l1_max_kernel(const double *__restrict__ part, int64_t n, double *out)
 {
-    hipLaunchKernelGGL(sy_colpart_kernel, dim3((unsigned)n), dim3(256), 0, s, A, lda, n, upper, colsum);
-    hipLaunchKernelGGL(sy_rowpart_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, A, lda, n, upper,
-                       colsum);
-    hipLaunchKernelGGL(max_reduce_kernel, dim3(1), dim3(256), 0, s, colsum, n, out);
+    __shared__ double red[4][64];
+    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+    const int64_t c = 64 * (int64_t)blockIdx.x + tx;
+    const int T = (int)((n + 63) / 64);
+    double s = 0.0;
+#pragma unroll 4
+    for (int u = ty; u < T; u += 4) s += part[(int64_t)u * n + (c < n ? c : n - 1)];
+    red[ty][tx] = s;
+    __syncthreads();
+    if (ty != 0) return;
+    double a = (red[0][tx] + red[1][tx]) + (red[2][tx] + red[3][tx]);
+    a = c < n && a == a ? a : 0.0;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) a = fmax(a, __shfl_xor(a, d));
+    if (tx == 0) atomicMax((unsigned long long *)out, (unsigned long long)__double_as_longlong(a));
 }
+
+int64_t l1norm_scratch_doubles(int64_t n) { return n * ((n + 63) / 64); }
+
+template <typename T>
+void launch_sy_l1norm(const T *A, int64_t lda, int64_t n, bool upper, double *part, double *out, hipStream_t s)
+{
+    const unsigned nt = (unsigned)((n + 63) / 64);
+    hipLaunchKernelGGL(sy_l1_tile_kernel<T>, dim3(nt * (nt + 1) / 2), dim3(256), 0, s, A, lda, n, upper, part, out);
+    hipLaunchKernelGGL(sy_l1_max_kernel, dim3(nt), dim3(256), 0, s, part, n, out);
+}
+template void launch_sy_l1norm<double>(const double *, int64_t, int64_t, bool, double *, double *, hipStream_t);
+template void launch_sy_l1norm<float>(const float *, int64_t, int64_t, bool, double *, double *, hipStream_t);
 
 }  // namespace mi

@@ -60,6 +60,7 @@ def lib() -> ctypes.CDLL:
         L.mi_dpotrs.argtypes = [_VP, ctypes.c_char, _I64, _I64, _VP, _I64, _VP, _I64]
         L.mi_dposv_async.argtypes = [_VP, ctypes.c_char, _I64, _I64, _VP, _I64, _VP, _I64, _VP]
         L.mi_dsy_l1norm.argtypes = [_VP, ctypes.c_char, _I64, _VP, _I64, _VP]
+        L.mi_ssy_l1norm.argtypes = [_VP, ctypes.c_char, _I64, _VP, _I64, _VP]
         L.mi_llt_trace.argtypes = [_VP, _INT]
         L.mi_llt_trace_read.argtypes = [_VP, _INT, ctypes.POINTER(ctypes.c_double),
                                         ctypes.POINTER(ctypes.c_double), ctypes.POINTER(_I64)]
@@ -114,7 +115,7 @@ def lib() -> ctypes.CDLL:
         L.dpotrs_.argtypes = [ctypes.c_char_p, ctypes.POINTER(_INT), ctypes.POINTER(_INT), _VP,
                               ctypes.POINTER(_INT), _VP, ctypes.POINTER(_INT), ctypes.POINTER(_INT)]
         for name in ("mi_llt_create", "mi_llt_destroy", "mi_llt_set_stream", "mi_dpotrf", "mi_dpotrf_async",
-                     "mi_dpotrs", "mi_dposv_async", "mi_dsy_l1norm", "LAPACKE_dpotrf", "LAPACKE_dpotrs",
+                     "mi_dpotrs", "mi_dposv_async", "mi_dsy_l1norm", "mi_ssy_l1norm", "LAPACKE_dpotrf", "LAPACKE_dpotrs",
                      "mi_llt_trace", "mi_llt_trace_read", "mi_llt_trace_reset", "mi_llt_status", "mi_llt_inject_status",
                      "mi_dposv_mixed", "mi_dposv_vbatched", "mi_sposv_vbatched", "mi_llt_set_vbatched_config",
                      "mi_llt_get_vbatched_config", "mi_dpotrf_adjoint", "mi_dpotrs_adjoint", "mi_spotrf",
@@ -402,11 +403,13 @@ def posv_mixed(a: torch.Tensor, b: torch.Tensor, x: torch.Tensor | None = None, 
 
 
 def sy_l1norm(a: torch.Tensor, uplo: str = "L", handle: Handle | None = None) -> torch.Tensor:
-    """``m_l1_norm`` of LLT::compute (LLT.h:442-453) as a 0-d float64 device tensor."""
+    """``m_l1_norm`` of LLT::compute (LLT.h:442-453) of a float64 or float32 ``a``, summed in FP64,
+    as a 0-d float64 device tensor."""
     h = handle.bind_stream() if handle else default_handle()
     out = torch.empty((), dtype=torch.float64, device=a.device)
-    h.check(lib().mi_dsy_l1norm(h.ptr, _uplo(uplo), int(a.shape[0]), _VP(a.data_ptr()), _ld(a),
-                                _VP(out.data_ptr())), "mi_dsy_l1norm")
+    f, what = (lib().mi_ssy_l1norm, "mi_ssy_l1norm") if a.dtype == torch.float32 else (lib().mi_dsy_l1norm,
+                                                                                      "mi_dsy_l1norm")
+    h.check(f(h.ptr, _uplo(uplo), int(a.shape[0]), _VP(a.data_ptr()), _ld(a), _VP(out.data_ptr())), what)
     return out
 
 

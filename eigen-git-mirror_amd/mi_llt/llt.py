@@ -71,7 +71,7 @@ class LLT:
             self._l1 = sy_l1norm(self._m, self.uplo)
             info = potrf_(self._m, self.uplo)
         else:
-            self._l1 = sy_l1norm(colmajor(self._m.double()), self.uplo).float()
+            self._l1 = sy_l1norm(self._m, self.uplo).float()
             info = spotrf_(self._m, self.uplo)
         self._info = ComputationInfo.Success if info == 0 else ComputationInfo.NumericalIssue
         return self

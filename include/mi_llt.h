@@ -158,6 +158,9 @@ int mi_spotrs(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const float *
  * whose `uplo` triangle is stored at dA.  Writes one double to the device pointer d_norm. */
 int mi_dsy_l1norm(mi_llt_handle h, char uplo, int64_t n, const double *dA, int64_t lda,
                   double *d_norm);
+/* The same for float storage (summed in FP64). */
+int mi_ssy_l1norm(mi_llt_handle h, char uplo, int64_t n, const float *dA, int64_t lda,
+                  double *d_norm);
 
 /* ---- rest of the LLT surface ----------------------------------------------------------
  * mi_dpocon: reciprocal condition number estimate of A from its factor (as left by mi_dpotrf

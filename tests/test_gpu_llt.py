@@ -174,6 +174,26 @@ def test_l1_norm(dev):
     assert v == pytest.approx(oracle.l1_norm_lower(junk), rel=1e-14)
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 130, 500])
+@pytest.mark.parametrize("uplo", ["L", "U"])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_l1_norm_tiles(dev, n, uplo, dtype):
+    """Around the 64 x 64 tiles, a padded leading dimension, junk in the other triangle; the sums
+    are FP64 in both storages (a column of n terms: n eps)."""
+    say(f"[gpu] l1 norm n={n} {uplo} {dtype}")
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n)).astype(np.float32).astype(np.float64)
+    a = a + a.T
+    a[min(n - 1, n // 2), 0] = a[0, min(n - 1, n // 2)] = -9.0  # a large entry off the diagonal
+    keep = np.tril(np.ones((n, n), bool)) if uplo == "L" else np.triu(np.ones((n, n), bool))
+    buf = torch.full((n, n + 3), 1e30, dtype=dtype, device=dev).t()  # column-major, ld n + 3
+    m = buf[:n, :]
+    m.copy_(torch.from_numpy(np.where(keep, a, 1e30)).to(dev))
+    want = np.abs(a.astype(np.float32).astype(np.float64) if dtype == torch.float32 else a).sum(0).max()
+    assert float(mi_llt.sy_l1norm(m, uplo)) == pytest.approx(want, rel=(n + 1) * 2.3e-16)
+
+
+
 def test_llt_object_mirror(dev):
     say("[gpu] LLT object")
     n = 260
