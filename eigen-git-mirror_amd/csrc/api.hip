@@ -52,7 +52,8 @@ struct mi_llt_context {
     // size, so a captured graph keeps valid pointers) and the schedule parameters
     void *vb_ws = nullptr;
     size_t vb_bytes = 0;
-    int vb_wg_per_cu = 2, vb_group = 0, vb_lpt = 1;  // group 0: by precision (FP64 2, FP32 4)
+    int vb_wg_per_cu = 2, vb_group = 0, vb_lpt = 1;
+    bool vb_set = false;  // the schedule was set; otherwise workgroups per CU by precision
     int cus = 0;
     double t_flops[MI_TRACE_KINDS] = {0};
     int64_t t_calls[MI_TRACE_KINDS] = {0};
@@ -312,14 +313,9 @@ int vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n, T *const
     if (!d_B) return -8;
     if (!d_ldb) return -9;
     if (!d_info) return -10;
-    int64_t grid = (int64_t)h->cus * h->vb_wg_per_cu;
-    const int64_t need_wg = (batch + 3) / 4;  // one system per worker wave at least
-    if (grid > need_wg) grid = need_wg;
-    if (grid < 1) grid = 1;
-    const size_t order_b = round_up((size_t)batch * sizeof(int));
-    const size_t ctr_b = 256;
-    const size_t scr_b = round_up((size_t)mi::vb_scratch_elems((int)grid) * sizeof(T));
-    const size_t need = order_b + ctr_b + scr_b;
+    const int64_t most = (int64_t)h->cus * (h->vb_set ? h->vb_wg_per_cu : mi::vb_workgroups_per_cu<T>());
+    const int grid = (int)(batch < most ? batch : most);  // a workgroup holds one system at least
+    const size_t need = round_up((size_t)mi::vb_plan_bytes(batch));
     if (need > h->vb_bytes) {
         hipError_t e = hipStreamSynchronize(h->stream);
         if (e != hipSuccess) return fail_hip(h, e, "hipStreamSynchronize");
@@ -333,16 +329,31 @@ int vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n, T *const
         }
         h->vb_bytes = need;
     }
-    char *p = (char *)h->vb_ws;
-    int *order = (int *)p;
-    int *counter = (int *)(p + order_b);
-    T *scratch = (T *)(p + order_b + ctr_b);
-    const double fl_est = 0.0;
-    traced(h, h->stream, MI_TRACE_BATCH, fl_est, [&] {
-        mi::launch_vbatched<T>(batch, d_n, d_A, d_lda, d_nrhs, d_B, d_ldb, d_info, order, counter, scratch, (int)grid,
-                               h->vb_group ? h->vb_group : (sizeof(T) == 8 ? 2 : 4), h->vb_lpt, h->stream);
+    traced(h, h->stream, MI_TRACE_BATCH, 0.0, [&] {
+        mi::launch_vbatched<T>(batch, d_n, d_A, d_lda, d_nrhs, d_B, d_ldb, d_info, h->vb_ws, grid, h->vb_lpt,
+                               h->stream);
     });
     return check_launch(h, "vbatched");
+}
+
+template <typename T>
+int sy_l1norm(mi_llt_handle h, char uplo, int64_t n, const T *dA, int64_t lda, double *d_norm)
+{
+    if (!valid(h)) return MI_LLT_E_HANDLE;
+    const int up = uplo_code(uplo);
+    if (up < 0) return -2;
+    if (n < 0) return -3;
+    if (dA == nullptr && n > 0) return -4;
+    if (lda < (n > 1 ? n : 1)) return -5;
+    if (d_norm == nullptr) return -6;
+    if (n == 0) {
+        hipLaunchKernelGGL(set_double_kernel, dim3(1), dim3(1), 0, h->stream, d_norm, 0.0);
+        return check_launch(h, "l1norm");
+    }
+    int rc = reserve(h, round_up((size_t)mi::l1norm_scratch_doubles(n) * sizeof(double)));
+    if (rc) return rc;
+    mi::launch_sy_l1norm<T>(dA, lda, n, up == 1, (double *)h->ws, d_norm, h->stream);
+    return check_launch(h, "l1norm");
 }
 
 // Waits for the stream, then reads and clears the status word (0 when none is allocated yet).
@@ -921,22 +932,12 @@ int mi_dpocon(mi_llt_handle h, char uplo, int64_t n, const double *dL, int64_t l
 
 int mi_dsy_l1norm(mi_llt_handle h, char uplo, int64_t n, const double *dA, int64_t lda, double *d_norm)
 {
-    if (!valid(h)) return MI_LLT_E_HANDLE;
-    const int up = uplo_code(uplo);
-    if (up < 0) return -2;
-    if (n < 0) return -3;
-    if (dA == nullptr && n > 0) return -4;
-    if (lda < (n > 1 ? n : 1)) return -5;
-    if (d_norm == nullptr) return -6;
-    if (n == 0) {
-        hipLaunchKernelGGL(set_double_kernel, dim3(1), dim3(1), 0, h->stream, d_norm, 0.0);
-        return check_launch(h, "l1norm");
-    }
-    int rc = reserve(h, round_up((size_t)n * sizeof(double)) > h->ws_bytes ? round_up((size_t)n * sizeof(double))
-                                                                            : h->ws_bytes);
-    if (rc) return rc;
-    mi::launch_sy_l1norm(dA, lda, n, up == 1, (double *)h->ws, d_norm, h->stream);
-    return check_launch(h, "l1norm");
+    return sy_l1norm<double>(h, uplo, n, dA, lda, d_norm);
+}
+
+int mi_ssy_l1norm(mi_llt_handle h, char uplo, int64_t n, const float *dA, int64_t lda, double *d_norm)
+{
+    return sy_l1norm<float>(h, uplo, n, dA, lda, d_norm);
 }
 
 int mi_dposv_mixed(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const double *dA, int64_t lda,
@@ -1050,6 +1051,7 @@ int mi_llt_set_vbatched_config(mi_llt_handle h, int wg_per_cu, int group, int lo
     if (!valid(h)) return MI_LLT_E_HANDLE;
     if (wg_per_cu < 1 || wg_per_cu > 64) return -2;
     if (group != 0 && group != 2 && group != 4) return -3;
+    h->vb_set = true;
     h->vb_wg_per_cu = wg_per_cu;
     h->vb_group = group;
     h->vb_lpt = longest_first ? 1 : 0;

@@ -112,8 +112,10 @@ void launch_upper_to_lower(const double *A, int64_t lda, int64_t n, double *W, i
 // triangle that the backward solve reads with upper_copy).
 template <typename T>
 void launch_lower_to_upper(const T *W, int64_t ldw, int64_t n, T *A, int64_t lda, hipStream_t s);
-void launch_sy_l1norm(const double *A, int64_t lda, int64_t n, bool upper, double *colsum, double *out,
-                      hipStream_t s);
+// *out = the symmetric L1 norm; part: l1norm_scratch_doubles(n) doubles.
+int64_t l1norm_scratch_doubles(int64_t n);
+template <typename T>
+void launch_sy_l1norm(const T *A, int64_t lda, int64_t n, bool upper, double *part, double *out, hipStream_t s);
 
 // Mixed-precision solve helpers (mixed.hip).
 int64_t sym_tiles64(int64_t n);  // lower 64 x 64 tiles: size of the norm partials
@@ -130,14 +132,14 @@ void launch_residual(const double *A, int64_t lda, int64_t n, bool upper, const 
 void launch_add_in_place(double *X, int64_t ldx, const double *D, int64_t ldd, int64_t n, int64_t nrhs,
                          hipStream_t s);
 
-// Batched uneven factor + solve (vbatched.hip): plan (argument checks, longest-first order,
-// counter reset) + one persistent launch of `grid` workgroups of 4 independent waves.
-// order: batch ints; counter: 1 int; scratch: vb_scratch_elems(grid) elements.
-int64_t vb_scratch_elems(int grid);
+// Batched uneven factor + solve (vbatched.hip): plan (argument checks, queues by order) + one
+// persistent launch of `grid` workgroups (vb_workgroups_per_cu fit a CU).  plan: vb_plan_bytes(batch) bytes.
+int64_t vb_plan_bytes(int64_t batch);
+template <typename T>
+int vb_workgroups_per_cu();
 template <typename T>
 void launch_vbatched(int64_t batch, const int *d_n, T *const *d_A, const int *d_lda, const int *d_nrhs,
-                     T *const *d_B, const int *d_ldb, int *d_info, int *order, int *counter, T *scratch, int grid,
-                     int group, int lpt, hipStream_t s);
+                     T *const *d_B, const int *d_ldb, int *d_info, void *plan, int grid, int lpt, hipStream_t s);
 
 // Level-3 pieces of the BLAS route (blas3.hip).
 // L (lower, ld ldl) = the lower triangle of A, or the upper one transposed; unit: diagonal 1.

@@ -5,44 +5,42 @@
 // unblocked (Eigen/src/Cholesky/LLT.h:312-368; below 32 columns Eigen runs the unblocked
 // column loop on the whole matrix, LLT.h:345) and LLT::_solve_impl (LLT.h:483-498) per system.
 //
-// Every wave is an independent worker: it draws the next system from a ticket counter (the
-// systems sorted longest first by a one-workgroup plan kernel) and factors and solves it
-// alone, so no wave ever waits for another and the launch always drains.  Per system
-// (T = ceil(n/16) tiles of 16), left-looking by tile columns k = 0..T-1:
-//   C_kk = A_kk - sum_{j<k} L_kj L_kj^T        (MFMA, operands read back from the system)
-//   leaf: L_kk = chol(C_kk) and X_kk = L_kk^{-1} in one pass of the column loop of
-//         LLT.h:320-334 -- lanes 0..15 hold the rows of C_kk, lanes 16..31 rows of the
-//         identity, and the same column operations turn the identity rows into L_kk^{-T};
-//   L_ik = (A_ik - sum_{j<k} L_ij L_kj^T) X_kk^T, tile rows i > k in groups of G
-// then the forward and backward substitutions by tiles with the stored X_kk, all products
-// on MFMA 16x16x4 (FP64 or FP32).  A partial last tile is padded with the identity.
-// The MFMA accumulator layout (element r of lane l: row l%16, column kx(r, l/16)) is the
-// operand layout of k-step r of the next product, so C_ik feeds C_ik X_kk^T directly.
+// A system is factored by a group of W waves, W = 1, 2 or 4 by its order (n <= 64, 128, 256), in
+// block columns of 64, left-looking: a wave holds its rows' part of the block column -- up to 4
+// tile rows of 16 (dealt round-robin over the group's waves) x 4 tile columns -- in registers:
+//   accumulate: C_ic = A_ic - sum_k L_ik L_ck^T over the finished columns (the wave's rows and the
+//               block's own four tile rows are read back once per block column), MFMA
+//   then for each of the 4 tile columns c, right-looking inside the block:
+//   leaf:   L_cc = chol(C_cc), X_cc = L_cc^{-1} in one column loop (leaf_device.hpp), by the wave
+//           that owns the row; X_cc to LDS
+//   panel:  L_ic = C_ic X_cc^T for the wave's rows below, the block's own rows to LDS
+//   update: C_ic' -= L_ic L_c'c^T, c' > c.
+// The MFMA result layout (element r of lane l: row l%16, column kx(r, l/16)) is the operand layout of
+// k-step r of the next product, so C_ic feeds C_ic X_cc^T and L_ic the update from registers.
+// What used to bound this path was re-reading the system, 14 times its size (one wave per system,
+// left-looking by single tile columns: 26.6 GB a launch of 20,000 systems, 5.7 TB/s beyond L2):
+// with 64-column blocks held by the group a factor of 256 reads its finished columns about twice,
+// and a CU has 2 to 12 systems in flight instead of 8 of any size.  20,000 systems, n ~ U[8, 256]:
+// FP64 4.6 -> 3.5 ms, FP32 3.0 -> 2.2 ms; 700 systems FP64 0.60 -> 0.19 ms.  What bounds it now is
+// the chain of a system's steps (about 6.5k cycles per 16 columns with two workgroups on a CU: leaf,
+// two barriers, panel, update; then 3.5k per step of each substitution), not memory: one workgroup
+// per CU takes 5.7 ms.
+// The substitutions run over the same blocks: the tiles of a block are dealt over the waves, each
+// sums the finished part on its own, and the block's 4 steps pass through LDS.  A partial last tile
+// is padded with the identity.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "leaf_device.hpp"
 
 namespace mi {
 
 constexpr int kVbMaxN = 256;
 constexpr int kVbMaxT = kVbMaxN / 16;
-constexpr int kVbWaves = 4;  // waves (workers) per workgroup
-
-__device__ __forceinline__ double vb_readlane(double x, int lane)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, x);
-    const int lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-__device__ __forceinline__ float vb_readlane(float x, int lane)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
-}
+constexpr int kVbPlan = 1024;  // systems per workgroup of the plan
 
 // Global-memory views of a system's pointers.  A pointer rebuilt from readfirstlane'd integers
 // is a generic one, and generic (flat) loads count in both the vector-memory and the LDS
-// counters, which the compiler can only wait on as a whole: with flat loads it waited for the
-// prefetched k-step together with the current one.  Global loads are counted in order.
+// counters, which the compiler can only wait on as a whole.  Global loads are counted in order.
 template <typename T>
 using gptr = __attribute__((address_space(1))) T *;
 template <typename T>
@@ -50,441 +48,692 @@ __device__ __forceinline__ gptr<T> to_global(T *p)
 {
     return (gptr<T>)p;
 }
-// Load at a byte offset from a wave-uniform base (scalar base + 32-bit vector offset form).
 template <typename T>
 __device__ __forceinline__ T load_at(gptr<const T> base, uint32_t off)
 {
     return *(gptr<const T>)((__attribute__((address_space(1))) const char *)base + off);
 }
+// Element at a byte offset from a wave-uniform base (scalar base + 32-bit vector offset form).
+template <typename T>
+__device__ __forceinline__ gptr<T> elem_at(gptr<T> base, uint32_t off)
+{
+    return (gptr<T>)((__attribute__((address_space(1))) char *)base + off);
+}
 
+// The lane layout of a 16 x 16 tile: element r of lane (l%16, g = l/16) is column kx(r, g), the k
+// index of operand k-step r (FP32 permutes k: any common order gives the same products).
+// LS: padded column of a leaf (16-byte aligned).
 template <typename T>
 struct VbArith;
-// FP64: v_mfma_f64_16x16x4f64; k-step s, lane group g supplies k = 4s + g
 template <>
-struct VbArith<double> {
+struct VbArith<double> {  // v_mfma_f64_16x16x4f64
     using acc_t = dvec4;
+    static constexpr int LS = 18;
     __device__ static acc_t mma(double q, double p, acc_t c) { return mfma_f64(q, p, c); }
     __device__ static int kx(int s, int g) { return 4 * s + g; }
     __device__ static constexpr int step(int s) { return 4 * s; }  // kx(s, g) - kx(0, g)
-    __device__ static double rsqrt(double x)
-    {
-        const double r = __builtin_amdgcn_rsq(x);
-        return r * (1.5 - 0.5 * x * r * r);
-    }
 };
-// FP32: v_mfma_f32_16x16x4f32, whose result element r of lane l is column 4(l/16) + r; the
-// k index of the operands is permuted the same way (any common order gives the same sums)
 template <>
-struct VbArith<float> {
+struct VbArith<float> {  // v_mfma_f32_16x16x4f32
     using acc_t = fvec4;
+    static constexpr int LS = 20;
     __device__ static acc_t mma(float q, float p, acc_t c) { return mfma_f32(q, p, c); }
     __device__ static int kx(int s, int g) { return 4 * g + s; }
-    __device__ static constexpr int step(int s) { return s; }  // kx(s, g) - kx(0, g)
-    __device__ static float rsqrt(float x)
-    {
-        const float r = __builtin_amdgcn_rsqf(x);
-        return r * (1.5f - 0.5f * x * r * r);
-    }
+    __device__ static constexpr int step(int s) { return s; }
 };
 
-// Memory ordering between the lanes of one wave for data it stored and reads back: the
-// wave's global stores complete (s_waitcnt 0) before any later load is issued.
-__device__ __forceinline__ void vb_fence()
+// Workgroups per CU: FP64 holds 4 x 4 tiles in 128 registers a lane and two workgroups; FP32 fits
+// three, which measured 2.17 ms against 2.70 with two (20,000 systems).  FP64 blocks of two tile
+// columns with three workgroups measured 3.7 ms against 3.5.
+template <typename T>
+constexpr int kVbPerCu = sizeof(T) == 8 ? 2 : 3;
+
+// One system, in the order of the queue.
+struct VbDesc {
+    uint64_t a, b;
+    int n, lda, nrhs, ldb;
+    int index, pad[3];
+};
+// Queue of mode c (0: groups of four waves, 1: of two, 2: single waves): systems [begin[c], end[c]),
+// dealt round-robin over eight counters on lines of their own -- workgroups take from their XCD's
+// counter first.  Every draw is an atomic at the memory side: at one counter they queued up for
+// about 17 ns each, which alone took 140 us for 8,000 systems of order 16.
+struct VbQueue {
+    int begin[4], end[4];
+    int pad[24];
+    int next[3][8][32];  // counter x of mode c: next[c][x][0]
+};
+
+// Largest order in tiles of a group of W waves.
+constexpr int vb_tm(int W) { return 4 * W; }
+
+// LDS of a group, per tile of its largest order: X_kk by columns (before: the leaf's rows), and the
+// block's own panel tiles, then Y_k^T, then X_k^T (lane order).
+template <typename T>
+constexpr int vb_lds_tile = 16 * VbArith<T>::LS + 256;
+
+// Progress of a group of two waves; counts on over the systems, never reset.
+struct VbSync {
+    uint32_t bar[2];
+    int fail, ticket[2], pad[3];
+};
+
+// Orders the LDS accesses of this wave's lanes (a wave's LDS operations execute in order).
+__device__ __forceinline__ void lds_order()
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Factor + solve one system with one wave.  Ls, Xs: 256 elements of LDS each (this wave's);
-// Xg: kVbMaxT * 256 elements of global scratch (this wave's).  Returns LAPACK info.
-//
-// Loads of a k-step s of column block j use a wave-uniform base (A + (16j + step(s)) * lda)
-// and a per-lane 32-bit byte offset of (row, lane group's column), the scalar-base form of
-// the global loads.  Every left-looking loop over j is software-pipelined: the loads of step
-// j+1 go out before the MFMAs of step j (two register buffers used alternately by name, so
-// no buffer is indexed at run time).
-template <typename T, int G>
-__device__ int vb_system(int n, T *A_, int64_t lda, int nrhs, T *B_, int64_t ldb, T *Ls, T *Xs, T *Xg_)
-{
+// A group of W waves (1, 2 or 4; a run-time scalar: one copy of the code serves all modes, and the
+// kernel must stay small -- unrolled per mode and column it took 200 KB, three times the instruction
+// cache, and ran at half the speed).
+template <typename T>
+struct VbGroup {
     using M = VbArith<T>;
     using acc_t = typename M::acc_t;
-    const gptr<T> A = to_global(A_), B = to_global(B_), Xg = to_global(Xg_);
-    const int l = lane_id(), li = l & 15, g = l >> 4;
-    const int nt = (n + 15) >> 4;
-    const T zero = (T)0, one = (T)1;
-    const int kx0 = M::kx(0, g);  // kx(s, g) = kx0 + M::step(s)
-    auto at = [](gptr<const T> base, uint32_t off) -> T { return load_at<T>(base, off); };
-    auto lane_off = [&](int row, int64_t ld) -> uint32_t { return (uint32_t)((row + (int64_t)kx0 * ld) * (int64_t)sizeof(T)); };
+    static constexpr int LS = M::LS;
 
-    for (int k = 0; k < nt; ++k) {
-        const int k0 = 16 * k;
-        const int rk = k0 + li < n ? k0 + li : n - 1;
-        const uint32_t offq = lane_off(rk, lda);
-        // ---- C_kk = A_kk - sum_{j<k} L_kj L_kj^T -> Ls (identity beyond n)
-        {
-            acc_t acc = {zero, zero, zero, zero};
-            const bool kin = k0 + li < n;
-            T qa[4], qb[4];
-#define VB_LOADD(q_, j_)                                                                           \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s) q_[s] = at(A + (int64_t)(16 * (j_) + M::step(s)) * lda, offq); \
-    } while (0)
-#define VB_MMAD(q_)                                                                                \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s) acc = M::mma(kin ? q_[s] : zero, kin ? q_[s] : zero, acc); \
-    } while (0)
-            if (k > 0) {
-                VB_LOADD(qa, 0);
-                for (int j = 0; j < k; j += 2) {
-                    if (j + 1 < k) VB_LOADD(qb, j + 1);
-                    VB_MMAD(qa);
-                    if (j + 1 >= k) break;
-                    if (j + 2 < k) VB_LOADD(qa, j + 2);
-                    VB_MMAD(qb);
-                }
-            }
-#undef VB_LOADD
-#undef VB_MMAD
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = li, col = M::kx(r, g);
-                const int gi = k0 + row, gj = k0 + col;
-                const bool in = gi < n && gj < n;
-                const T a = A[(in ? gi : 0) + (int64_t)(in ? gj : 0) * lda];
-                Ls[row + 16 * col] = in ? (T)(a - acc[r]) : (row == col ? one : zero);
-            }
+    T *X, *Y;  // LDS: X_kk at X + 16 LS k, tiles at Y + 256 k
+    VbSync *sy;
+    int W, w;  // waves of the group, this wave
+    uint32_t bars;
+    int parity;
+
+    // Barrier of the group for its LDS data (global stores may stay in flight).  Two waves of a
+    // workgroup meet through two words of LDS: each counts its barriers there and waits for the
+    // other's count, which the other -- resident, being of the same workgroup -- reaches without
+    // waiting for anything but earlier barriers, so the wait ends.
+    __device__ __forceinline__ void barrier()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        if (W == 4) {
+            __builtin_amdgcn_s_barrier();
+        } else if (W == 2) {
+            ++bars;
+            __hip_atomic_store(&sy->bar[w], bars, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            while ((int)(__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(&sy->bar[w ^ 1], __ATOMIC_RELAXED,
+                                                                               __HIP_MEMORY_SCOPE_WORKGROUP)) -
+                         (int)bars) < 0)
+                __builtin_amdgcn_s_sleep(0);
         }
-        // ---- leaf: lanes 0..15 rows of C_kk, lanes 16..31 identity rows; the column operations
-        // run on every lane without lane predicates (entries above a leaf lane's diagonal change
-        // but are never broadcast nor stored), column j+1 -- the next pivot -- first
-        {
-            T v[16];
-#pragma unroll
-            for (int c = 0; c < 16; ++c) v[c] = l < 16 ? Ls[li + 16 * c] : ((l < 32 && c == l - 16) ? one : zero);
-            int fail = -1;
-            T x = vb_readlane(v[0], 0);
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                if (fail < 0 && x <= zero) fail = j;  // LLT.h:327-330; a NaN pivot passes
-                v[j] *= M::rsqrt(x);
-                if (j + 1 < 16) {
-                    v[j + 1] -= v[j] * vb_readlane(v[j], j + 1);
-                    x = vb_readlane(v[j + 1], j + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-#pragma unroll
-                for (int c = j + 2; c < 16; ++c) v[c] -= v[j] * vb_readlane(v[j], c);
-            }
-            if (fail >= 0) return k0 + fail + 1;
-            // L_kk to the system (lower part), X_kk = L_kk^{-1} to Xs / Xg (column-major)
-            if (l < 16 && k0 + l < n) {
-#pragma unroll
-                for (int c = 0; c < 16; ++c)
-                    if (c <= l) A[(k0 + l) + (int64_t)(k0 + c) * lda] = v[c];
-            }
-            if (l >= 16 && l < 32) {
-#pragma unroll
-                for (int c = 0; c < 16; ++c) {
-                    Xs[c + 16 * (l - 16)] = v[c];  // lane 16+i holds row i of L^{-T} = column i of X
-                    Xg[k * 256 + c + 16 * (l - 16)] = v[c];
-                }
-            }
-        }
-        // ---- panel: L_ik = (A_ik - sum_{j<k} L_ij L_kj^T) X_kk^T, i > k, G tile rows at a time
-        T xq[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xq[s] = Xs[li + 16 * M::kx(s, g)];
-        for (int i0 = k + 1; i0 < nt; i0 += G) {
-            uint32_t offp[G];
-            bool pin[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                const int row = 16 * (i0 + u) + li;
-                pin[u] = row < n;
-                offp[u] = lane_off(row < n ? row : n - 1, lda);
-            }
-            acc_t pa[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) pa[u] = acc_t{zero, zero, zero, zero};
-            T qa[4], qb[4], xa[G][4], xb[G][4];
-#define VB_LOAD(q_, x_, j_)                                                                        \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s)                                              \
-        {                                                                                          \
-            const gptr<const T> base_ = A + (int64_t)(16 * (j_) + M::step(s)) * lda;               \
-            q_[s] = at(base_, offq);                                                               \
-            _Pragma("unroll") for (int u = 0; u < G; ++u) x_[u][s] = at(base_, offp[u]);            \
-        }                                                                                          \
-    } while (0)
-#define VB_MMA(q_, x_)                                                                             \
-    do {                                                                                           \
-        _Pragma("unroll") for (int u = 0; u < G; ++u)                                              \
-        {                                                                                          \
-            _Pragma("unroll") for (int s = 0; s < 4; ++s) pa[u] = M::mma(q_[s], pin[u] ? x_[u][s] : zero, pa[u]); \
-        }                                                                                          \
-    } while (0)
-            if (k > 0) {
-                VB_LOAD(qa, xa, 0);
-                for (int j = 0; j < k; j += 2) {
-                    if (j + 1 < k) VB_LOAD(qb, xb, j + 1);
-                    VB_MMA(qa, xa);
-                    if (j + 1 >= k) break;
-                    if (j + 2 < k) VB_LOAD(qa, xa, j + 2);
-                    VB_MMA(qb, xb);
-                }
-            }
-#undef VB_LOAD
-#undef VB_MMA
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                if (i0 + u < nt) {
-                    const int row = 16 * (i0 + u) + li;
-                    const int rc = row < n ? row : n - 1;
-                    T c[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const T a = A[rc + (int64_t)(k0 + M::kx(r, g)) * lda];
-                        c[r] = row < n ? (T)(a - pa[u][r]) : zero;
-                    }
-                    acc_t o = {zero, zero, zero, zero};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) o = M::mma(xq[s], c[s], o);
-                    if (row < n) {
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) A[row + (int64_t)(k0 + M::kx(r, g)) * lda] = o[r];
-                    }
-                }
-            }
-        }
-        vb_fence();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
+    // The same after which the waves' global stores can be read by all of them.
+    __device__ __forceinline__ void barrier_global()
+    {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     }
 
-    // ---- solve, 16 right-hand sides at a time; products on the transposed blocks
-    // (C[c][i] = sum_m P[c][m] Q[i][m] with P from B, Q from L or X)
-    for (int c0 = 0; c0 < nrhs; c0 += 16) {
+    // Runs a mode's queue.  Every value that steers the loop is wave-uniform.
+    __device__ __forceinline__ void run(const VbDesc *__restrict__ desc, VbQueue *queue, int mode, int *__restrict__ d_info)
+    {
+        const int l = lane_id();
+        auto sc = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+        const int begin = sc(queue->begin[mode]), end = sc(queue->end[mode]);
+        int *next = &queue->next[mode][0][0];
+        int x = (int)(blockIdx.x & 7);  // the counter drawn from
+        const bool draws = w == 0;
+        // a ticket of counter x (valid in lane 0), and the system it stands for: when it is past the
+        // end, another counter's, as long as one has systems left (counters only grow: it ends)
+        auto draw = [&]() -> int { return atomicAdd(next + 32 * x, l == 0 ? 1 : 0); };
+        auto settle = [&](int ticket) -> int {
+            for (;;) {
+                const int i = begin + x + 8 * sc(ticket);
+                if (i < end) return i;
+                const int v = __hip_atomic_load(next + 32 * (l & 7), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t left = (uint32_t)__ballot(begin + (l & 7) + 8 * v < end) & 0xffu;
+                if (!left) return end;
+                const uint32_t turned = ((left >> x) | (left << (8 - x))) & 0xffu;  // from x on
+                x = (x + __builtin_ctz(turned)) & 7;
+                ticket = draw();
+            }
+        };
+        // first pass: no system yet, only the ticket; then each pass takes one system: the loop ends
+        int t = begin - 1;
+        VbDesc d = desc[0];
+        for (;;) {
+            auto sc64 = [&](uint64_t v) {
+                return ((uint64_t)(uint32_t)sc((int)(v >> 32)) << 32) | (uint32_t)sc((int)(uint32_t)v);
+            };
+            const bool have = t >= begin;
+            const int n = have ? sc(d.n) : 0, lda = sc(d.lda), nrhs = sc(d.nrhs), ldb = sc(d.ldb), idx = sc(d.index);
+            const gptr<T> A = to_global((T *)(uintptr_t)sc64(d.a)), B = to_global((T *)(uintptr_t)sc64(d.b));
+            // the next ticket is drawn now, its descriptor read before the substitutions
+            int tn = 0;
+            if (draws) tn = draw();
+            const int info = factor(n, A, lda);
+            if (draws) sy->ticket[parity] = settle(tn);
+            barrier_global();  // L to every wave
+            tn = sc(sy->ticket[parity]);
+            d = desc[tn < end ? tn : 0];
+            if (info == 0 && n > 0)
+                for (int c0 = 0; c0 < nrhs; c0 += 16) solve(n, A, lda, nrhs, B, ldb, c0);
+            if (draws && have) d_info[idx] = info;
+            barrier();  // every wave is done with this system's LDS
+            if (tn >= end) return;
+            parity ^= 1;
+            t = tn;
+        }
+    }
+
+    // C[r][c] = sum_k L[row_r, k] L[4J + c, k]^T over the k tiles [0, 4J), r < NR.
+    template <int NR>
+    __device__ __forceinline__ void accumulate(acc_t (&C)[4][4], gptr<const T> A, int64_t lda, int J,
+                                               const uint32_t (&offp)[4], const uint32_t (&offq)[4])
+    {
+        constexpr int U = 4;  // k-steps in flight (16 J of them)
+        T p[U][NR], q[U][4];
+        const int steps = 16 * J;
+        auto load = [&](int u, int s) {
+            s = s < steps ? s : steps - 1;
+            const gptr<const T> base = A + (int64_t)(16 * (s >> 2) + M::step(1) * (s & 3)) * lda;
+#pragma unroll
+            for (int r = 0; r < NR; ++r) p[u][r] = load_at<T>(base, offp[r]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) q[u][c] = load_at<T>(base, offq[c]);
+        };
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u) load(u, u);
+        for (int s0 = 0; s0 < steps; s0 += U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                load((u + U - 1) % U, s0 + u + U - 1);
+#pragma unroll
+                for (int r = 0; r < NR; ++r)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) C[r][c] = M::mma(q[u][c], p[u][r], C[r][c]);
+                __builtin_amdgcn_sched_barrier(0);  // keeps the wait counts exact
+            }
+        }
+    }
+
+    // LAPACK info (uniform over the group).
+    __device__ __forceinline__ int factor(const int n, const gptr<T> A, const int64_t lda)
+    {
+        const int l = lane_id(), li = l & 15, g = l >> 4;
+        const int nt = (n + 15) >> 4;
+        const T zero = (T)0, one = (T)1;
+        const int kx0 = M::kx(0, g);
+        auto lane_off = [&](int r) -> uint32_t { return (uint32_t)((r + (int64_t)kx0 * lda) * (int64_t)sizeof(T)); };
+        for (int J = 0; 4 * J < nt; ++J) {
+            const int nb = nt - 4 * J < 4 ? nt - 4 * J : 4;  // tile columns of the block
+            // slot r: tile row 4J + q, q = r W + w; ns slots in use
+            const int left = nt - 4 * J - w, ns = left <= 0 ? 0 : left <= W ? 1 : left <= 2 * W ? 2 : left <= 3 * W ? 3 : 4;
+            acc_t C[4][4];
+            uint32_t offp[4], offq[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * (4 * J + r * W + w) + li, j = 16 * (4 * J + r) + li;
+                offp[r] = lane_off(i < n ? i : n - 1);
+                offq[r] = lane_off(j < n ? j : n - 1);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) C[r][c] = acc_t{zero, zero, zero, zero};
+            }
+            if (J > 0) {
+                if (ns > 2)
+                    accumulate<4>(C, A, lda, J, offp, offq);
+                else if (ns == 2)
+                    accumulate<2>(C, A, lda, J, offp, offq);
+                else if (ns == 1)
+                    accumulate<1>(C, A, lda, J, offp, offq);
+            }
+            // A minus the sum: the tiles at and left of the diagonal (the strictly upper part of a
+            // diagonal tile is read but never used: every lane stops at its own diagonal entry).  The
+            // sum is formed by itself first: in FP32 it keeps its own rounding, not A's.
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int col = 16 * (4 * J + c);
+                if (col + 16 <= n) {
+                    T a[4][4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const gptr<T> base = A + (int64_t)(col + M::step(e)) * lda;
+                        // rows above the block's diagonal and empty slots: a row that is read anyway
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            a[r][e] = *elem_at(base, r < ns && r * W + w >= c ? offp[r] : offp[0]);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) C[r][c][e] = a[r][e] - C[r][c][e];
+                } else if (c < nb) {  // the last, partial tile column: columns past n - 1 read n - 1's
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (r < ns && r * W + w == c) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int i = col + li, cc = col + M::kx(e, g);
+                                C[r][c][e] = A[(i < n ? i : n - 1) + (int64_t)(cc < n ? cc : n - 1) * lda] - C[r][c][e];
+                            }
+                        }
+                }
+            }
+            // rows past n: zero, the identity on the diagonal
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int q = r * W + w, i = 16 * (4 * J + q) + li;
+                if (r < ns && 16 * (4 * J + q) + 16 > n) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int col = 16 * (4 * J + c) + M::kx(e, g);
+                            C[r][c][e] = i < n && col < n ? C[r][c][e] : (i == col ? one : zero);
+                        }
+                }
+            }
+            // this wave's diagonal tile of the block column at hand, in C[r][0]: to LDS for the leaf
+            auto give_leaf = [&](int c) {
+                T *xs = X + 16 * LS * (4 * J + c);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (r * W + w == c) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) xs[LS * li + M::kx(e, g)] = C[r][0][e];
+                    }
+            };
+            give_leaf(0);
+            // the column at hand is always C[.][0]; the others move up after each
+#pragma unroll 1
+            for (int c = 0; c < nb; ++c) {
+                const int k = 4 * J + c, k0 = 16 * k;
+                T *xs = X + 16 * LS * k;
+                // ---- leaf
+                T u[16];
+                if (w == (c & (W - 1))) {
+                    lds_order();
+                    // (opaque: the identity's rows, hoisted out of the loops, would fill the registers)
+                    int own = li;
+                    asm volatile("" : "+v"(own));
+                    T v[16];
+#pragma unroll
+                    for (int m = 0; m < 16; ++m) u[m] = xs[LS * li + m];
+#pragma unroll
+                    for (int m = 0; m < 16; ++m) v[m] = m == own ? one : zero;
+                    const int f = leaf_factor(u, v);
+                    lds_order();
+                    sy->fail = f >= 0 ? k0 + f + 1 : 0;
+                    if (l < 16) {
+#pragma unroll
+                        for (int m = 0; m < 16; ++m) xs[LS * li + m] = v[m];
+                    }
+                }
+                barrier();
+                {
+                    const int f = __builtin_amdgcn_readfirstlane(sy->fail);
+                    if (f != 0) return f;
+                }
+                if (w == (c & (W - 1)) && l < 16 && k0 + l < n) {  // L_kk
+                    gptr<T> p = A + (k0 + l) + (int64_t)k0 * lda;
+#pragma unroll
+                    for (int m = 0; m < 16; ++m, p += lda)
+                        if (m <= l) *p = u[m];
+                }
+                // ---- panel
+                T xq[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) xq[e] = xs[LS * M::kx(e, g) + li];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int q = r * W + w;
+                    if (r < ns && q > c) {
+                        acc_t o = {zero, zero, zero, zero};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o = M::mma(xq[e], C[r][0][e], o);
+                        C[r][0] = o;
+                        if (q < 4) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) Y[256 * q + 64 * e + l] = o[e];
+                        }
+                        const int i = 16 * (4 * J + q) + li;
+                        if (i < n) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) *elem_at(A + (int64_t)(k0 + M::step(e)) * lda, offp[r]) = o[e];
+                        }
+                    }
+                }
+                if (c + 1 == nb) break;
+                barrier();
+                // ---- update, and the columns move up
+                T np[4][4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) np[r][e] = -C[r][0][e];
+#pragma unroll
+                for (int h = 1; h < 4; ++h) {  // tile column c + h
+                    T pq[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) pq[e] = Y[256 * ((c + h) & 3) + 64 * e + l];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        C[r][h - 1] = C[r][h];
+                        if (r < ns && c + h < nb && r * W + w >= c + h) {
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) C[r][h - 1] = M::mma(pq[e], np[r][e], C[r][h - 1]);
+                        }
+                    }
+                    if (h == 1) give_leaf(c + 1);
+                }
+            }
+            barrier_global();  // the next block reads this one's columns (and the panel tiles are free)
+        }
+        return 0;
+    }
+
+    // z[h] += sum over the tiles j of [j0, j1) of Y_j^T times the operand tile load(q, j) of this
+    // wave's tiles h < NC, four operand tiles at a time.
+    template <int NC, class Load>
+    __device__ __forceinline__ void sum(acc_t (&z)[4], int j0, int j1, Load &&load)
+    {
+        constexpr int U = 4 / NC;
+        const int l = lane_id();
+        T q[U][NC][4];
+        if (j0 >= j1) return;
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u) load(q[u], j0 + u < j1 ? j0 + u : j1 - 1);
+        for (int j = j0; j < j1; j += U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                load(q[(u + U - 1) % U], j + u + U - 1 < j1 ? j + u + U - 1 : j1 - 1);
+                const bool in = j + u < j1;  // past the end: times zero
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const T y = Y[256 * (in ? j + u : j0) + 64 * e + l], p = in ? y : (T)0;
+#pragma unroll
+                    for (int h = 0; h < NC; ++h) z[h] = M::mma(q[u][h][e], p, z[h]);
+                }
+            }
+        }
+    }
+
+    // B[:, c0..c0+15] <- A^{-1} B with the factor in A and the X_kk in LDS, as transposed tiles (rows:
+    // right-hand sides); a block's tile column c belongs to wave c % W as its tile h = c / W.
+    __device__ __forceinline__ void solve(const int n, const gptr<T> A, const int64_t lda, const int nrhs,
+                                          const gptr<T> B, const int64_t ldb, const int c0)
+    {
+        const int nbk = (((n + 15) >> 4) + 3) >> 2;
+#pragma unroll 1
+        for (int J = 0; J < nbk; ++J) solve_block<false>(n, A, lda, nrhs, B, ldb, c0, J);
+#pragma unroll 1
+        for (int J = nbk - 1; J >= 0; --J) solve_block<true>(n, A, lda, nrhs, B, ldb, c0, J);
+        barrier();  // the next right-hand sides overwrite Y
+    }
+
+    // Forward:  Y_c^T = (B_c^T - sum_{j<c} Y_j^T L_cj^T) X_cc^T.
+    // Backward: X_c^T = (Y_c^T - sum_{i>c} X_i^T L_ic) X_cc.
+    template <bool BACK>
+    __device__ __forceinline__ void solve_block(const int n, const gptr<T> A, const int64_t lda, const int nrhs,
+                                                const gptr<T> B, const int64_t ldb, const int c0, const int J)
+    {
+        const int l = lane_id(), li = l & 15, g = l >> 4;
+        const int nt = (n + 15) >> 4, nb = nt - 4 * J < 4 ? nt - 4 * J : 4;
+        const T zero = (T)0;
         const int col = c0 + li;
         const bool cin = col < nrhs;
         const int64_t bcol = (int64_t)(cin ? col : c0) * ldb;
-        const gptr<const T> Bc = B + bcol;
-        // forward: Y_k^T = (B_k^T - sum_{j<k} Y_j^T L_kj^T) X_kk^T
-        for (int k = 0; k < nt; ++k) {
-            const int k0 = 16 * k;
-            const int rk = k0 + li < n ? k0 + li : n - 1;
-            const uint32_t offq = lane_off(rk, lda);
-            const uint32_t offb = (uint32_t)(kx0 * (int64_t)sizeof(T));
-            acc_t acc = {zero, zero, zero, zero};
-            T pa_[4], qa_[4], pb_[4], qb_[4];
-#define VB_LOADF(p_, q_, j_)                                                                       \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s)                                              \
-        {                                                                                          \
-            p_[s] = at(Bc + 16 * (j_) + M::step(s), offb);                                         \
-            q_[s] = at(A + (int64_t)(16 * (j_) + M::step(s)) * lda, offq);                         \
-        }                                                                                          \
-    } while (0)
-#define VB_MMAF(p_, q_)                                                                            \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s) acc = M::mma(k0 + li < n ? q_[s] : zero, cin ? p_[s] : zero, acc); \
-    } while (0)
-            if (k > 0) {
-                VB_LOADF(pa_, qa_, 0);
-                for (int j = 0; j < k; j += 2) {
-                    if (j + 1 < k) VB_LOADF(pb_, qb_, j + 1);
-                    VB_MMAF(pa_, qa_);
-                    if (j + 1 >= k) break;
-                    if (j + 2 < k) VB_LOADF(pa_, qa_, j + 2);
-                    VB_MMAF(pb_, qb_);
-                }
-            }
-#undef VB_LOADF
-#undef VB_MMAF
-            T c[4], xq2[4];
+        auto clamp = [&](int i) { return i < n ? i : n - 1; };
+        // operand of tile j for this wave's tile h (column 4J + c, c = h W + w): L_cj[li][k] (forward),
+        // L_jc[k][li].  Only a backward j can be a partial tile (its rows past n read row n - 1).
+        uint32_t off[4];
+        const bool near = lda <= (1 << 20);  // 256 columns within 32-bit offsets
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = k0 + M::kx(r, g);
-                const T bv = B[(row < n ? row : n - 1) + bcol];
-                c[r] = (row < n && cin) ? (T)(bv - acc[r]) : zero;
-                xq2[r] = Xg[k * 256 + li + 16 * M::kx(r, g)];
-            }
-            acc_t y = {zero, zero, zero, zero};
-#pragma unroll
-            for (int s = 0; s < 4; ++s) y = M::mma(xq2[s], c[s], y);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = k0 + M::kx(r, g);
-                if (row < n && cin) B[row + bcol] = y[r];
-            }
-            vb_fence();
+        for (int h = 0; h < 4; ++h) {
+            const int64_t own = clamp(16 * (4 * J + h * W + w) + li), k = M::kx(0, g);
+            off[h] = (uint32_t)((BACK ? k + own * lda : own + k * lda) * (int64_t)sizeof(T));
         }
-        // backward: X_k^T = (Y_k^T - sum_{j>k} X_j^T L_jk) X_kk
-        for (int k = nt - 1; k >= 0; --k) {
-            const int k0 = 16 * k;
-            // column k0 + li of L: below n whenever the loop runs (k < nt - 1); clamped anyway
-            const int64_t colkc = (int64_t)(k0 + li < n ? k0 + li : n - 1) * lda;
-            acc_t acc = {zero, zero, zero, zero};
-            T pa_[4], qa_[4], pb_[4], qb_[4];
-            bool oka[4], okb[4];
-#define VB_LOADB(p_, q_, ok_, j_)                                                                  \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s)                                              \
-        {                                                                                          \
-            const int m = 16 * (j_) + M::kx(s, g);                                                 \
-            ok_[s] = m < n;                                                                        \
-            const int mc = ok_[s] ? m : n - 1;                                                     \
-            p_[s] = B[mc + bcol];                                                                  \
-            q_[s] = A[mc + colkc];                                                                 \
-        }                                                                                          \
-    } while (0)
-#define VB_MMAB(p_, q_, ok_)                                                                       \
-    do {                                                                                           \
-        _Pragma("unroll") for (int s = 0; s < 4; ++s) acc = M::mma(ok_[s] ? q_[s] : zero, (ok_[s] && cin) ? p_[s] : zero, acc); \
-    } while (0)
-            if (k + 1 < nt) {
-                VB_LOADB(pa_, qa_, oka, k + 1);
-                for (int j = k + 1; j < nt; j += 2) {
-                    if (j + 1 < nt) VB_LOADB(pb_, qb_, okb, j + 1);
-                    VB_MMAB(pa_, qa_, oka);
-                    if (j + 1 >= nt) break;
-                    if (j + 2 < nt) VB_LOADB(pa_, qa_, oka, j + 2);
-                    VB_MMAB(pb_, qb_, okb);
+        auto operand = [&](T(&q)[4], int h, int j) {
+            if (near && (!BACK || 16 * j + 16 <= n)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    q[e] = load_at<T>(A + (BACK ? (int64_t)(16 * j + M::step(e)) : (int64_t)(16 * j + M::step(e)) * lda), off[h]);
+            } else {
+                const int own = clamp(16 * (4 * J + h * W + w) + li);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int k = clamp(16 * j + M::kx(e, g));
+                    q[e] = A[BACK ? k + (int64_t)own * lda : own + (int64_t)k * lda];
                 }
             }
-#undef VB_LOADB
-#undef VB_MMAB
-            T c[4], xq2[4];
+        };
+        acc_t z[4];  // the sums, by themselves (see factor)
+        T bv[4][4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = k0 + M::kx(r, g);
-                const T bv = B[(row < n ? row : n - 1) + bcol];
-                c[r] = (row < n && cin) ? (T)(bv - acc[r]) : zero;
-                xq2[r] = Xg[k * 256 + M::kx(r, g) + 16 * li];
+        for (int h = 0; h < 4; ++h) {
+            z[h] = acc_t{zero, zero, zero, zero};
+            const int k = 4 * J + h * W + w;
+            if (h * W + w < nb) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 16 * k + M::kx(e, g);
+                    if (BACK) {
+                        bv[h][e] = Y[256 * k + 64 * e + l];
+                    } else {
+                        const T v = B[clamp(i) + bcol];
+                        bv[h][e] = i < n && cin ? v : zero;
+                    }
+                }
             }
-            acc_t y = {zero, zero, zero, zero};
+        }
+        const int j0 = BACK ? 4 * J + 4 : 0, j1 = BACK ? nt : 4 * J;
+        if (W == 4)
+            sum<1>(z, j0, j1, [&](T(&q)[1][4], int j) { operand(q[0], 0, j); });
+        else if (W == 2)
+            sum<2>(z, j0, j1, [&](T(&q)[2][4], int j) {
+                operand(q[0], 0, j);
+                operand(q[1], 1, j);
+            });
+        // (a single wave's systems are one block: nothing to sum)
+        T in[4][4];  // the operand tiles for the block's column at hand, read one column ahead
+        auto needs = [&](int h, int c) -> bool { return h * W + w < nb && (BACK ? h * W + w < c : h * W + w > c); };
+        auto ahead = [&](int c) {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) y = M::mma(xq2[s], c[s], y);
+            for (int h = 0; h < 4; ++h)
+                if (needs(h, c)) operand(in[h], h, 4 * J + c);
+        };
+        ahead(BACK ? nb - 1 : 0);
+#pragma unroll 1
+        for (int s = 0; s < nb; ++s) {
+            const int c = BACK ? nb - 1 - s : s, k = 4 * J + c;
+            if (w == (c & (W - 1))) {
+                acc_t o = {zero, zero, zero, zero}, zi = o;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = k0 + M::kx(r, g);
-                if (row < n && cin) B[row + bcol] = y[r];
+                for (int h = 0; h < 4; ++h)
+                    if (h * W + w == c) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) zi[e] = bv[h][e] - z[h][e];
+                    }
+                const T *xs = X + 16 * LS * k;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // rows past n (forward): their sums come from copies of L's row n - 1
+                    const T zz = BACK || 16 * k + M::kx(e, g) < n ? zi[e] : zero;
+                    o = M::mma(xs[BACK ? LS * li + M::kx(e, g) : LS * M::kx(e, g) + li], zz, o);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 16 * k + M::kx(e, g);
+                    Y[256 * k + 64 * e + l] = !BACK || i < n ? o[e] : zero;
+                    if (BACK && i < n && cin) B[i + bcol] = o[e];
+                }
             }
-            vb_fence();
+            barrier();
+            if (s + 1 < nb) {
+                T y[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] = Y[256 * k + 64 * e + l];
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    if (needs(h, c)) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) z[h] = M::mma(in[h][e], y[e], z[h]);
+                    }
+                ahead(BACK ? c - 1 : c + 1);
+            }
         }
     }
-    return 0;
+};
+
+template <typename T>
+__global__ __launch_bounds__(256, kVbPerCu<T>) void vb_persistent_kernel(const VbDesc *__restrict__ desc, VbQueue *queue,
+                                                               int *__restrict__ d_info)
+{
+    // one group of four waves, then two of two, then four single waves; a group's LDS grows with its
+    // largest order, so wave w's part starts at its first wave's four tiles in every mode
+    static_assert(16 * vb_lds_tile<T> * sizeof(T) + 7 * sizeof(VbSync) <= 160 * 1024 / kVbPerCu<T>, "workgroups per CU");
+    __shared__ __align__(16) T lds[16 * vb_lds_tile<T>];
+    __shared__ VbSync sync[7];
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int i = threadIdx.x; i < (int)(sizeof(sync) / 4); i += 256) ((uint32_t *)sync)[i] = 0u;
+    __syncthreads();
+#pragma unroll 1
+    for (int mode = 0; mode < 3; ++mode) {
+        VbGroup<T> q;
+        q.W = 4 >> mode;
+        q.w = w & (q.W - 1);
+        q.sy = &sync[mode == 0 ? 0 : mode == 1 ? 1 + (w >> 1) : 3 + w];
+        const int first = w - q.w;  // the group's first wave
+        q.X = lds + 4 * first * vb_lds_tile<T>;
+        q.Y = q.X + 4 * q.W * 16 * VbArith<T>::LS;
+        q.bars = 0;
+        q.parity = 0;
+        q.run(desc, queue, mode, d_info);
+    }
 }
 
-// Plan: check every system's arguments, sort the systems longest first (counting sort by
-// tile count; LPT order keeps the tail of the launch short) or keep the given order, and
-// reset the work counter.  One workgroup.
-__global__ __launch_bounds__(1024) void vb_plan_kernel(int64_t batch, const int *__restrict__ d_n,
-                                                       const int *__restrict__ d_lda, const int *__restrict__ d_nrhs,
-                                                       const int *__restrict__ d_ldb, int *__restrict__ d_info,
-                                                       int *__restrict__ order, int lpt, int *counter)
+// Plan: every system's arguments checked (its info set), the valid ones sorted into the queues,
+// longest first within a queue (lpt: the tail of the launch stays short) or in the given order.
+// Two launches of one workgroup per kVbPlan systems: each counts its systems per bucket (tile
+// count, longest first; lpt = 0: per mode), then each places its own behind the earlier workgroups'.
+constexpr int kVbBuckets = kVbMaxT + 1;
+__device__ __forceinline__ int vb_check(int n, int lda, int nr, int ldb)
 {
-    __shared__ int hist[kVbMaxT + 2], start[kVbMaxT + 2];
+    if (n < 0 || n > kVbMaxN) return -1;
+    if (lda < (n > 1 ? n : 1)) return -2;
+    if (nr < 0) return -3;
+    if (nr > 0 && ldb < (n > 1 ? n : 1)) return -4;
+    return 0;
+}
+// Mode of a system of nt tiles: 0: four waves, 1: two, 2: one.
+__host__ __device__ constexpr int vb_mode(int nt) { return nt <= vb_tm(1) ? 2 : nt <= vb_tm(2) ? 1 : 0; }
+__device__ __forceinline__ int vb_bucket(int n, int lpt)
+{
+    const int nt = (n + 15) / 16;
+    return kVbMaxT - (lpt ? nt : vb_tm(4 >> vb_mode(nt)));  // not lpt: the bucket of the mode's largest order
+}
+
+__global__ __launch_bounds__(kVbPlan) void vb_count_kernel(int64_t batch, const int *__restrict__ d_n,
+                                                           const int *__restrict__ d_lda, const int *__restrict__ d_nrhs,
+                                                           const int *__restrict__ d_ldb, int *__restrict__ d_info,
+                                                           int *__restrict__ hist, int lpt)
+{
+    __shared__ int cnt[kVbBuckets];
     const int tid = threadIdx.x;
-    if (tid < kVbMaxT + 2) hist[tid] = 0;
+    if (tid < kVbBuckets) cnt[tid] = 0;
     __syncthreads();
-    for (int64_t i = tid; i < batch; i += blockDim.x) {
-        const int n = d_n[i], lda = d_lda[i], nr = d_nrhs[i], ldb = d_ldb[i];
-        int bad = 0;
-        if (n < 0 || n > kVbMaxN) bad = -1;
-        else if (lda < (n > 1 ? n : 1)) bad = -2;
-        else if (nr < 0) bad = -3;
-        else if (nr > 0 && ldb < (n > 1 ? n : 1)) bad = -4;
+    const int64_t i = (int64_t)blockIdx.x * kVbPlan + tid;
+    if (i < batch) {
+        const int n = d_n[i];
+        const int bad = vb_check(n, d_lda[i], d_nrhs[i], d_ldb[i]);
         d_info[i] = bad;
-        const int b = bad ? kVbMaxT + 1 : (n + 15) / 16;  // bucket; invalid systems last
-        atomicAdd(&hist[b], 1);
+        if (!bad) atomicAdd(&cnt[vb_bucket(n, lpt)], 1);
+    }
+    __syncthreads();
+    if (tid < kVbBuckets) hist[(int64_t)blockIdx.x * kVbBuckets + tid] = cnt[tid];
+}
+
+template <typename T>
+__global__ __launch_bounds__(kVbPlan) void vb_place_kernel(int64_t batch, const int *__restrict__ d_n,
+                                                           T *const *__restrict__ d_A, const int *__restrict__ d_lda,
+                                                           const int *__restrict__ d_nrhs, T *const *__restrict__ d_B,
+                                                           const int *__restrict__ d_ldb, const int *__restrict__ hist,
+                                                           VbDesc *__restrict__ desc, VbQueue *__restrict__ queue,
+                                                           int lpt)
+{
+    __shared__ int total[kVbBuckets], before[kVbBuckets], start[kVbBuckets + 1];
+    const int tid = threadIdx.x;
+    if (tid < kVbBuckets) total[tid] = before[tid] = 0;
+    __syncthreads();
+    for (int e = tid; e < (int)gridDim.x * kVbBuckets; e += kVbPlan) {
+        const int wg = e / kVbBuckets, b = e % kVbBuckets, v = hist[e];
+        if (v) {
+            atomicAdd(&total[b], v);
+            if (wg < (int)blockIdx.x) atomicAdd(&before[b], v);
+        }
     }
     __syncthreads();
     if (tid == 0) {
         int s = 0;
-        for (int b = kVbMaxT; b >= 0; --b) {  // longest first
+        for (int b = 0; b < kVbBuckets; ++b) {
             start[b] = s;
-            s += hist[b];
+            s += total[b];
         }
-        start[kVbMaxT + 1] = s;
-        *counter = 0;
+        start[kVbBuckets] = s;
     }
     __syncthreads();
-    for (int64_t i = tid; i < batch; i += blockDim.x) {
-        if (!lpt) {
-            order[i] = (int)i;
-            continue;
+    if (blockIdx.x == 0) {
+        if (tid < 3) {  // buckets from the mode's largest order on
+            queue->begin[tid] = start[kVbMaxT - vb_tm(4 >> tid)];
+            queue->end[tid] = start[tid < 2 ? kVbMaxT - vb_tm(2 >> tid) : kVbBuckets];
         }
-        const int n = d_n[i];
-        const int b = d_info[i] ? kVbMaxT + 1 : (n + 15) / 16;
-        order[atomicAdd(&start[b], 1)] = (int)i;
+        if (tid < 3 * 8) queue->next[tid / 8][tid % 8][0] = 0;
     }
+    if (tid < kVbBuckets) before[tid] += start[tid];
+    __syncthreads();
+    const int64_t i = (int64_t)blockIdx.x * kVbPlan + tid;
+    if (i >= batch) return;
+    VbDesc d;
+    d.n = d_n[i];
+    d.lda = d_lda[i];
+    d.nrhs = d_nrhs[i];
+    d.ldb = d_ldb[i];
+    if (vb_check(d.n, d.lda, d.nrhs, d.ldb)) return;
+    d.a = (uint64_t)(uintptr_t)d_A[i];
+    d.b = (uint64_t)(uintptr_t)d_B[i];
+    d.index = (int)i;
+    d.pad[0] = d.pad[1] = d.pad[2] = 0;
+    desc[atomicAdd(&before[vb_bucket(d.n, lpt)], 1)] = d;
 }
 
-template <typename T, int G>
-__global__ __launch_bounds__(64 * kVbWaves, 2) void vb_persistent_kernel(int64_t batch, const int *__restrict__ d_n,
-                                                                      T *const *__restrict__ d_A,
-                                                                      const int *__restrict__ d_lda,
-                                                                      const int *__restrict__ d_nrhs,
-                                                                      T *const *__restrict__ d_B,
-                                                                      const int *__restrict__ d_ldb, int *d_info,
-                                                                      const int *__restrict__ order, int *counter,
-                                                                      T *__restrict__ scratch)
+constexpr int64_t kVbQueueBytes = ((int64_t)sizeof(VbQueue) + 255) / 256 * 256;
+// Bytes of the plan: the queues, the workgroups' counts and the systems in queue order.
+int64_t vb_plan_bytes(int64_t batch)
 {
-    __shared__ T lds[kVbWaves][2][256];
-    const int w = threadIdx.x >> 6, l = lane_id();
-    const int worker = blockIdx.x * kVbWaves + w;
-    T *Xg = scratch + (size_t)worker * kVbMaxT * 256;
-    // The loop has no lane-dependent branch: every value that steers it is wave-uniform
-    // (scalar).  The ticket is drawn by all lanes adding (lane == 0) -- one atomic add of 1
-    // after the wave reduction -- and read from lane 0; the per-system parameters go through
-    // readfirstlane; the info store is done by every lane (same address, same value).  (A
-    // branch on `lane == 0` both at the top and at the bottom of the body lets the compiler
-    // merge the two across the back edge and split the loop so that lanes leave it one at a
-    // time, with the others re-reading a ticket they never drew: that never terminates.)
-    // Each pass draws one ticket and tickets only grow, so no worker needs more than batch + 1
-    // passes; the bound keeps the loop finite whatever the counter holds.
-    for (int64_t pass = 0; pass <= batch; ++pass) {
-        int t = atomicAdd(counter, l == 0 ? 1 : 0);
-        t = __builtin_amdgcn_readlane(t, 0);
-        if (t >= batch) break;
-        const int i = __builtin_amdgcn_readfirstlane(order[t]);
-        const int pre = __builtin_amdgcn_readfirstlane(d_info[i]);  // argument error set by the plan
-        if (pre == 0) {
-            const int n = __builtin_amdgcn_readfirstlane(d_n[i]);
-            const int lda = __builtin_amdgcn_readfirstlane(d_lda[i]);
-            const int nr = __builtin_amdgcn_readfirstlane(d_nrhs[i]);
-            const int ldb = __builtin_amdgcn_readfirstlane(d_ldb[i]);
-            const uint64_t pa = (uint64_t)(uintptr_t)d_A[i], pb = (uint64_t)(uintptr_t)d_B[i];
-            T *A = (T *)(uintptr_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(pa >> 32)) << 32) |
-                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pa));
-            T *B = (T *)(uintptr_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(pb >> 32)) << 32) |
-                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pb));
-            const int info = vb_system<T, G>(n, A, lda, nr, B, ldb, lds[w][0], lds[w][1], Xg);
-            d_info[i] = info;
-        }
-    }
+    const int64_t wgs = (batch + kVbPlan - 1) / kVbPlan;
+    return kVbQueueBytes + (wgs * kVbBuckets * 4 + 255) / 256 * 256 + batch * (int64_t)sizeof(VbDesc);
 }
-
-int64_t vb_scratch_elems(int grid) { return (int64_t)grid * kVbWaves * kVbMaxT * 256; }
 
 template <typename T>
 void launch_vbatched(int64_t batch, const int *d_n, T *const *d_A, const int *d_lda, const int *d_nrhs,
-                     T *const *d_B, const int *d_ldb, int *d_info, int *order, int *counter, T *scratch, int grid,
-                     int group, int lpt, hipStream_t s)
+                     T *const *d_B, const int *d_ldb, int *d_info, void *plan, int grid, int lpt, hipStream_t s)
 {
-    hipLaunchKernelGGL(vb_plan_kernel, dim3(1), dim3(1024), 0, s, batch, d_n, d_lda, d_nrhs, d_ldb, d_info, order,
-                       lpt, counter);
-    if (group == 2)
-        hipLaunchKernelGGL((vb_persistent_kernel<T, 2>), dim3(grid), dim3(64 * kVbWaves), 0, s, batch, d_n, d_A,
-                           d_lda, d_nrhs, d_B, d_ldb, d_info, order, counter, scratch);
-    else
-        hipLaunchKernelGGL((vb_persistent_kernel<T, 4>), dim3(grid), dim3(64 * kVbWaves), 0, s, batch, d_n, d_A,
-                           d_lda, d_nrhs, d_B, d_ldb, d_info, order, counter, scratch);
+    const unsigned wgs = (unsigned)((batch + kVbPlan - 1) / kVbPlan);
+    VbQueue *queue = (VbQueue *)plan;
+    int *hist = (int *)((char *)plan + kVbQueueBytes);
+    VbDesc *desc = (VbDesc *)((char *)plan + kVbQueueBytes + ((int64_t)wgs * kVbBuckets * 4 + 255) / 256 * 256);
+    hipLaunchKernelGGL(vb_count_kernel, dim3(wgs), dim3(kVbPlan), 0, s, batch, d_n, d_lda, d_nrhs, d_ldb, d_info,
+                       hist, lpt);
+    hipLaunchKernelGGL(vb_place_kernel<T>, dim3(wgs), dim3(kVbPlan), 0, s, batch, d_n, d_A, d_lda, d_nrhs, d_B, d_ldb,
+                       hist, desc, queue, lpt);
+    hipLaunchKernelGGL(vb_persistent_kernel<T>, dim3(grid), dim3(256), 0, s, desc, queue, d_info);
 }
 
+template <typename T>
+int vb_workgroups_per_cu()
+{
+    return kVbPerCu<T>;
+}
+template int vb_workgroups_per_cu<double>();
+template int vb_workgroups_per_cu<float>();
+
 template void launch_vbatched<double>(int64_t, const int *, double *const *, const int *, const int *,
-                                      double *const *, const int *, int *, int *, int *, double *, int, int, int,
-                                      hipStream_t);
+                                      double *const *, const int *, int *, void *, int, int, hipStream_t);
 template void launch_vbatched<float>(int64_t, const int *, float *const *, const int *, const int *, float *const *,
-                                     const int *, int *, int *, int *, float *, int, int, int, hipStream_t);
+                                     const int *, int *, void *, int, int, hipStream_t);
 
 }  // namespace mi

@@ -9,8 +9,8 @@ lda = n_i, B_i n_i x nrhs_i with ldb = n_i) plus the device arrays the C ABI tak
 launch allocates nothing once the handle's batched workspace is large enough, so repeated
 calls can be captured in a CUDA/HIP graph (``torch.cuda.graph``).
 
-:func:`autotune` times the schedule parameters of the launch (workgroups of 4 worker waves
-per CU, tile rows per register block, longest-first order) on the caller's batch and keeps
+:func:`autotune` times the schedule parameters of the launch (workgroups of 4 waves per CU,
+longest-first order; the register-block size is accepted and has no effect) on the caller's batch and keeps
 the fastest on the handle; results are cached per batch signature in a JSON file.
 """
 from __future__ import annotations

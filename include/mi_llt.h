@@ -216,8 +216,8 @@ int mi_dposv_mixed(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const do
 /* ---- batched, uneven sizes ------------------------------------------------------------
  * Counterpart: a loop of LLT<MatrixXd>(A_i).solve(B_i) (LLT.h:104-110, 430-460, 483-498) over
  * independent systems.  Factors each A_i (n_i x n_i, lower triangle, in place) and overwrites
- * B_i (n_i x nrhs_i) with A_i^{-1} B_i, for i < batch, in one persistent launch (plus a
- * one-workgroup plan launch); nothing is allocated when the handle's batched workspace is
+ * B_i (n_i x nrhs_i) with A_i^{-1} B_i, for i < batch, in one persistent launch (plus
+ * two small plan launches); nothing is allocated when the handle's batched workspace is
  * already large enough, so repeated calls can be captured in a HIP graph.  All arrays are
  * device arrays of `batch` entries.  0 <= n_i <= 256; uplo 'L' only (MI_LLT_E_UNSUPPORTED
  * for 'U').  d_info[i]: 0, k+1 for a failing pivot at column k (B_i unchanged), or -1 n_i out
@@ -228,10 +228,10 @@ int mi_dposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n,
 int mi_sposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n, float *const *d_A,
                       const int *d_lda, const int *d_nrhs, float *const *d_B, const int *d_ldb, int *d_info);
 /* Schedule of the batched launch (no reference counterpart; set by the autotuner in
- * mi_llt.batched): workgroups of 4 worker waves per CU (1..64), tile rows per register block
- * of the panel update (2 or 4; 0, the default: 2 for FP64 and 4 for FP32, the largest each
- * precision holds in registers without spilling), and longest-first ordering (1) or the given
- * order (0). */
+ * mi_llt.batched): workgroups of 4 waves launched per CU (1..64; until it is set, as many as fit
+ * a CU: 2 for FP64, 3 for FP32), a register-block size (0, 2 or 4; accepted and kept, the kernel's
+ * blocks are fixed per precision), and longest-first ordering within the size classes (1) or the
+ * given order (0). */
 int mi_llt_set_vbatched_config(mi_llt_handle h, int wg_per_cu, int group, int longest_first);
 int mi_llt_get_vbatched_config(mi_llt_handle h, int *wg_per_cu, int *group, int *longest_first);
 

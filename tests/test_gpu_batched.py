@@ -180,3 +180,49 @@ def test_vbatched_full_workload_backward_error(dev):
             worst_s = max(worst_s, be)
     assert worst_f <= 1e-14, worst_f
     assert worst_s <= 1e-14, worst_s
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_vbatched_group_edges(dev, dtype):
+    """Orders around the group sizes (64, 128 and 256: one, two and four waves) and the 64-column
+    blocks, leading dimensions larger than the order, 1, 16 and 17 right-hand sides, systems that
+    fail in their last column in between; the bounds are those of the tests above."""
+    ns = [48, 49, 63, 64, 65, 80, 112, 127, 128, 129, 144, 177, 192, 193, 240, 241, 255, 256] * 2
+    pads = [(5 * i) % 4 for i in range(len(ns))]
+    rs = [(1, 16, 17, 0, 3)[i % 5] for i in range(len(ns))]
+    big = batched.VBatch([n + p for n, p in zip(ns, pads)], rs, dtype=dtype, device=dev)
+    big.d_n.copy_(torch.tensor(ns, dtype=torch.int32))
+    rng = np.random.default_rng(5)
+    mats, rhss, before = [], [], []
+    for i, n in enumerate(ns):
+        bad = i % 9 == 4
+        a = workloads.indefinite_at(n, n - 1, seed=60 + i) if bad else workloads.gram_spd(n, seed=60 + i)
+        a = np.array(a)
+        a[np.triu_indices(n, 1)] = 1e30  # must never be read
+        b = rng.standard_normal((n, rs[i]))
+        if dtype == torch.float32:
+            a, b = a.astype(np.float32).astype(np.float64), b.astype(np.float32).astype(np.float64)
+        big.A(i)[:n, :n].copy_(torch.from_numpy(a))
+        if rs[i]:
+            big.B(i)[:n].copy_(torch.from_numpy(b))
+        mats.append(a)
+        rhss.append(b)
+        before.append(big.B(i).clone())
+    info = batched.posv_vbatched_(big, mi_llt.Handle()).cpu().tolist()
+    f32 = dtype == torch.float32
+    for i, n in enumerate(ns):
+        if i % 9 == 4:
+            assert info[i] == n, (i, n, info[i])
+            assert torch.equal(big.B(i), before[i])
+            continue
+        assert info[i] == 0, (i, n, info[i])
+        a, b = mats[i], rhss[i]
+        asym = np.tril(a) + np.tril(a, -1).T
+        l = big.A(i)[:n, :n].cpu().double().numpy()
+        assert np.all(np.triu(l, 1) == np.triu(a, 1).astype(l.dtype)) or f32, f"system {i}: upper triangle modified"
+        lo = np.tril(oracle.llt_blocked(np.asfortranarray(asym))[0])
+        assert np.linalg.norm(np.tril(l) - lo) <= (2e-5 * n / 16 if f32 else 1e-12) * np.linalg.norm(lo)
+        if rs[i]:
+            x = big.B(i)[:n].cpu().double().numpy()
+            res = np.linalg.norm(asym @ x - b, axis=0) / (np.linalg.norm(asym) * np.linalg.norm(x, axis=0))
+            assert res.max() <= (2e-6 * n / 16 if f32 else 1e-14), (i, n, rs[i], res.max())
