@@ -4,6 +4,7 @@
 #pragma once
 #include "common.hpp"
 #include "kernels.hpp"
+#include "leaf_device.hpp"
 #include "mfma_tile.hpp"
 
 namespace mi {
@@ -34,60 +35,35 @@ __device__ __forceinline__ double readlane_d(double x, int lane)
     return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// Panel p (columns c0..c0+15 of the 128 x 128 block in S, tiled: sl), waves 0..2 (wave 3 is
-// meanwhile busy with the previous panel's deferred update, see potrf_in_lds).  Each of the
-// three waves holds the 16 x 16 leaf in lanes 0..15 (row c0+l) and runs the column loop of
-// LLT.h:320-334 on it (pivot test, sqrt, scale, rank-1 update) redundantly, so its lane
-// broadcasts (readlane) need no barrier.  Lanes 16..63 hold the rows c0+16+48w+(l-16) below
-// the leaf (up to 112 rows over the three waves) and receive the same column operations, which
-// is the panel solve A_ip L_pp^{-T}; lanes 48..63 of wave 2 (never a row below) hold the rows
-// of the 16 x 16 identity, which the same operations turn into L_pp^{-T}, i.e. column i of
-// X_pp = L_pp^{-1} in lane 48+i, written to xleaf column-major.  1/sqrt from the hardware
-// estimate and one Newton step, d = x/sqrt(x).
+// Panel p (columns c0..c0+15 of the 128 x 128 block in S, tiled: sl), waves 0 and 1 (2 and 3 are
+// meanwhile busy with the previous panel's deferred update, see potrf_in_lds).  Each row of 16
+// lanes holds the whole 16 x 16 leaf in u (leaf_device.hpp), so its broadcasts need no barrier and
+// no scalar registers; v holds one more row per lane, which takes the same column operations: the
+// up to 112 rows below the leaf (row c0+16+64w+l), for which they are the panel solve A_ip
+// L_pp^{-T}, and in the last 16 lanes of wave 1 (never a row below) the rows of the 16 x 16
+// identity, which become L_pp^{-T}, i.e. column i of X_pp = L_pp^{-1} in lane 48+i, written to xleaf
+// column-major.  (With readlane broadcasts and the leaf in lanes 0..15, three waves took a panel in
+// 4300 cycles; this form takes 2900, and two waves are left for the deferred updates.)
 //
-// The column operations run on every lane without lane predicates: at step j, v[j] *= 1/sqrt(x)
-// gives sqrt(x) on lane j (where v[j] is the pivot x) and the scaled column below it, and the
-// rank-1 update v[c] -= v[j] * L(c0+c, c0+j), c > j, leaves every lane's entries at or below
-// its diagonal exact.  Entries above the diagonal of a leaf lane l (c > l) do change, but they
-// are never broadcast (readlane reads lane c of column j < c) nor stored.  Without per-lane
-// selects the loop holds no predicate masks, so the broadcasts get scalar registers of their
-// own and column j+1 -- the next pivot -- is updated first, off the remaining updates.
-// (Broadcasting the multipliers through LDS instead -- the leaf lanes store column j, every
-// lane reads it back with uniform addresses -- measured slower: 23 vs 21.5 us per block.)
-//
-// Returns the failing panel column or -1, the same in the three waves.  The factored leaf is
-// left in v (lanes 0..15): it is written back to S only after a barrier, since the other waves
-// read the unfactored leaf from S here and may still be doing so when one wave is done.
-__device__ __forceinline__ int panel_factor3(double *S, int c0, double *__restrict__ xleaf, double (&v)[16])
+// Returns the failing panel column or -1, the same in both waves.  The factored leaf is left in u:
+// it is written back to S only after a barrier, since the other wave reads the unfactored leaf from
+// S here and may still be doing so when one wave is done.
+__device__ __forceinline__ int panel_factor2(double *S, int c0, double *__restrict__ xleaf, double (&u)[16])
 {
     const int l = lane_id(), w = threadIdx.x >> 6;
-    const bool leaf = l < 16;
-    const int rb = c0 + 16 + 48 * w + (l - 16);
-    const bool ident = w == 2 && l >= 48;
-    const bool below = !leaf && !ident && rb < 128;
-    const int r = leaf ? c0 + l : (below ? rb : c0);
+    const int rb = c0 + 16 + 64 * w + l;
+    const bool ident = w == 1 && l >= 48, below = !ident && rb < 128;
+    const int r = below ? rb : c0 + (l & 15);
+    double v[16];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) u[c] = S[sl(c0 + (l & 15), c0 + c)];
 #pragma unroll
     for (int c = 0; c < 16; ++c) v[c] = S[sl(r, c0 + c)];
     if (ident) {
 #pragma unroll
         for (int c = 0; c < 16; ++c) v[c] = (c == l - 48) ? 1.0 : 0.0;
     }
-    int fail = -1;
-    double x = readlane_d(v[0], 0);  // pivot: leaf row j lives in lane j
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        if (fail < 0 && x <= 0.0) fail = j;  // LLT.h:327-330; a NaN pivot passes
-        double rd = __builtin_amdgcn_rsq(x);
-        rd = rd * (1.5 - 0.5 * x * rd * rd);
-        v[j] *= rd;
-        if (j + 1 < 16) {  // the next pivot first: it is the loop's serial chain
-            v[j + 1] -= v[j] * readlane_d(v[j], j + 1);
-            x = readlane_d(v[j + 1], j + 1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int c = j + 2; c < 16; ++c) v[c] -= v[j] * readlane_d(v[j], c);  // L(c0+c, c0+j)
-    }
+    const int fail = leaf_factor(u, v);
     if (fail >= 0) return fail;
     if (below) {  // rows no other wave reads before the next barrier
 #pragma unroll
@@ -159,21 +135,19 @@ __device__ __forceinline__ void lds_tile_update(double *C, const double (&Pi)[4]
 // below it and their operands P_x (tile (p+1+x, p), x < T) in every wave's registers:
 //   A(p): the leaf of p goes back to S; the T tiles of column p+1 get panel p's update (the
 //         waves round-robin), barrier;
-//   B(p): waves 0..2 factor panel p+1 (panel_factor3: VALU and lane broadcasts) while wave 3
-//         applies panel p to the tiles right of column p+1 on the matrix core -- up to kCap of
-//         them, any more go to waves 0..2 after their column loop -- barrier.
+//   B(p): waves 0 and 1 factor panel p+1 (panel_factor2: VALU) while waves 2 and 3 apply panel p
+//         to the tiles right of column p+1 on the matrix core (21 tiles at most), barrier.
 // Column p+1 thus has every earlier panel's update before its factor, the tiles beyond it get
 // panel p's before phase A(p+1) touches them, and the rank-16 updates mostly run under the
 // column loop.  Returns the first failing column or -1 (uniform); writes the 8 leaf inverses
 // to Xl.  s_fail: an LDS int.
 __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, int *s_fail)
 {
-    constexpr int kCap = 12;  // deferred tiles taken by wave 3 (about one column loop's worth)
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
     double lv[16];
     __syncthreads();
-    if (w < 3) {
-        const int f = panel_factor3(S, 0, Xl, lv);
+    if (w < 2) {
+        const int f = panel_factor2(S, 0, Xl, lv);
         if (w == 0 && l == 0) *s_fail = f;
     }
     __syncthreads();
@@ -203,18 +177,18 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
             if (x < T && (x & 3) == w) lds_tile_update(S + 256 * (((tb + x) * (tb + x + 1)) / 2 + tb) + l, P[x], P[0]);
         __syncthreads();
         // ---- B(p)
-        if (w < 3) {
-            const int f = panel_factor3(S, 16 * tb, Xl + 256 * tb, lv);
+        if (w < 2) {
+            const int f = panel_factor2(S, 16 * tb, Xl + 256 * tb, lv);
             if (w == 0 && l == 0) *s_fail = f;
-        }
+        } else {
 #pragma unroll
-        for (int ti = 1; ti < 7; ++ti) {
+            for (int ti = 1; ti < 7; ++ti) {
 #pragma unroll
-            for (int tj = 1; tj <= ti; ++tj) {
-                const int t = ((ti - 1) * ti) / 2 + (tj - 1);  // enumerates the deferred tiles
-                const int owner = t < kCap ? 3 : (t - kCap) % 3;
-                if (ti < T && w == owner)
-                    lds_tile_update(S + 256 * (((tb + ti) * (tb + ti + 1)) / 2 + tb + tj) + l, P[ti], P[tj]);
+                for (int tj = 1; tj <= ti; ++tj) {
+                    const int t = ((ti - 1) * ti) / 2 + (tj - 1);  // enumerates the deferred tiles
+                    if (ti < T && w == 2 + (t & 1))
+                        lds_tile_update(S + 256 * (((tb + ti) * (tb + ti + 1)) / 2 + tb + tj) + l, P[ti], P[tj]);
+                }
             }
         }
         __syncthreads();
