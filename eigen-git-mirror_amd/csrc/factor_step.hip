@@ -263,7 +263,8 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
                         uint32_t *tickets, uint32_t ticket_base, uint32_t *flag, uint32_t epoch, int *status,
                         hipStream_t s, uint32_t *grid_out, int prec, __bf16 *Wsplit, const Batch &bt)
 {
-    const int Gp = kp >= 0 ? (int)((n - kp + 127) / 128) : 0;
+    const int64_t below = n - kp - kNB;  // rows below the panel's diagonal block
+    const int Gp = kp < 0 ? 0 : 1 + (below > 0 ? (int)((below + 64 * kRowTiles - 1) / (64 * kRowTiles)) : 0);
     int c0 = 0, nsyrk = 0, K = k >= 1 ? 256 : 128, KQ = 0, cq0 = 0, co0 = 0, nko = 0;
     int64_t slab = k >= 1 ? (k - 1) * kNB : 0, slabq = 0, slabo = 0;
     if constexpr (sizeof(S) == 8) {

@@ -400,16 +400,17 @@ __device__ __forceinline__ void split_store_row(__bf16 *slot, int64_t part_off, 
     }
 }
 
-// Tile engine for storage type T and trailing-update arithmetic PREC.
-template <typename T, int PREC>
+// Tile engine for storage type T and trailing-update arithmetic PREC:
+// 16 TA x 64 elements per wave.
+template <typename T, int PREC, int TA = 4>
 struct TileSel {
-    using type = WaveTile<4, 4>;
+    using type = WaveTile<TA, 4>;
 };
-template <int PREC>
-struct TileSel<float, PREC> {
+template <int PREC, int TA>
+struct TileSel<float, PREC, TA> {
     // the updates inside a panel step of the 3-part split arithmetic use FP32 MFMAs (the same
     // 24-bit accuracy; the trailing update reads the split panels instead, syrk_tile_split_lds)
-    using type = WaveTileF<4, 4, PREC == kPrecBF16x6 ? kPrecF32 : PREC>;
+    using type = WaveTileF<TA, 4, PREC == kPrecBF16x6 ? kPrecF32 : PREC>;
 };
 
 // A second FP64 wave tile, for irregular k ranges: TA x TB MFMA tiles, acc[a][b] = tile

@@ -80,27 +80,24 @@ __device__ __forceinline__ int panel_factor2(double *S, int c0, double *__restri
 // factor, or the 28 strictly lower tiles of L11 plus the 8 leaf inverses for the panel solve.
 constexpr int kSmem = 36 * 256;
 
-// A (global, ld lda, valid order bs) -> S (lower part, identity beyond bs); 32 loads in
-// flight per thread, from clamped in-bounds addresses.  T = float widens to FP64.
+// A (global, ld lda, valid order bs) -> S (lower part, identity beyond bs); a thread's 64 loads all
+// in flight, from clamped in-bounds addresses.  T = float widens to FP64.
 template <typename T>
 __device__ __forceinline__ void block_to_lds(double *S, const T *__restrict__ Ab, int64_t lda, int bs)
 {
     const int tid = threadIdx.x, r = tid & 127, ch = tid >> 7;
+    T a[64];
 #pragma unroll
-    for (int q0 = 0; q0 < 64; q0 += 32) {
-        T a[32];
+    for (int q = 0; q < 64; ++q) {
+        const int c = 2 * q + ch;
+        const bool in = r < bs && c < bs;
+        a[q] = Ab[(in ? r : 0) + (int64_t)(in ? c : 0) * lda];
+    }
 #pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int c = 2 * (q0 + q) + ch;
-            const bool in = r < bs && c < bs;
-            a[q] = Ab[(in ? r : 0) + (int64_t)(in ? c : 0) * lda];
-        }
-#pragma unroll
-        for (int q = 0; q < 32; ++q) {
-            const int c = 2 * (q0 + q) + ch;
-            const bool in = r < bs && c < bs;
-            if (r >= c) S[sl(r, c)] = in ? (double)a[q] : (r == c ? 1.0 : 0.0);
-        }
+    for (int q = 0; q < 64; ++q) {
+        const int c = 2 * q + ch;
+        const bool in = r < bs && c < bs;
+        if (r >= c) S[sl(r, c)] = in ? (double)a[q] : (r == c ? 1.0 : 0.0);
     }
 }
 
@@ -140,8 +137,10 @@ __device__ __forceinline__ void lds_tile_update(double *C, const double (&Pi)[4]
 // Column p+1 thus has every earlier panel's update before its factor, the tiles beyond it get
 // panel p's before phase A(p+1) touches them, and the rank-16 updates mostly run under the
 // column loop.  Returns the first failing column or -1 (uniform); writes the 8 leaf inverses
-// to Xl.  s_fail: an LDS int.
-__device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, int *s_fail)
+// to Xl and the strictly lower tiles to the panel image W (sls order), each panel's from the operands
+// in the registers of phase A, so that only the stores' end is left to wait for when the block is done.
+// s_fail: an LDS int.
+__device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, int *s_fail, double *__restrict__ W)
 {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
     double lv[16];
@@ -172,6 +171,14 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
                 for (int s = 0; s < 4; ++s) P[x][s] = src[64 * s];
             }
         }
+        // the panel's tiles to the image
+#pragma unroll
+        for (int x = 0; x < 7; ++x)
+            if (x < T && (x & 3) == w) {
+                double *dst = W + 256 * (((tb + x) * (tb + x - 1)) / 2 + p) + l;
+#pragma unroll
+                for (int s = 0; s < 4; ++s) dst[64 * s] = P[x][s];
+            }
 #pragma unroll
         for (int x = 0; x < 7; ++x)
             if (x < T && (x & 3) == w) lds_tile_update(S + 256 * (((tb + x) * (tb + x + 1)) / 2 + tb) + l, P[x], P[0]);
@@ -203,8 +210,16 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
     return -1;
 }
 
-// The panel solve works on a wave's 32 rows x 128 columns in the FP64 MFMA result layout:
-// X[t][p][r] is row 16t + lane%16, column 16p + 4r + lane/16 (t = 0..1 row tiles, p = 0..7
+// Row tiles of 16 per wave in the panel solve: a row role is 64 kRowTiles rows.  With one, the solve
+// on the chain from panel to panel (its 144 MFMAs per row tile) and the rows' update are half as long
+// as with two, and there are twice as many roles, each staging the 72 KiB panel image.  Half as long
+// wins at every size: with the image stored as the block is factored (potrf_in_lds) and the deeper
+// operand prefetch of the diagonal update, the FP64 factor and solve took 1437 us against 1532 at
+// n = 3001 and 6282 against 6369 at n = 8192, the FP32 one 2072 against 2315 at n = 4001.
+constexpr int kRowTiles = 1;
+
+// The panel solve works on a wave's 16 RT rows x 128 columns in the FP64 MFMA result layout:
+// X[t][p][r] is row 16t + lane%16, column 16p + 4r + lane/16 (t < RT row tiles, p = 0..7
 // column strips).  It needs, in LDS, the 28 strictly lower tiles of L (Ls, sls order) and the
 // 8 leaf inverses (Xs, 256 doubles each, column-major): the panel image of kernels.hpp.
 //
@@ -212,7 +227,8 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
 //   X_p <- (X_p - sum_{q<p} X_q L_pq^T) X_pp^T,   X_pp = L_pp^{-1}
 // with the accumulator of a solved strip used directly as the operand of the next ones (its
 // layout is that of an MFMA P operand with k = 4s + lane/16).
-__device__ __forceinline__ void trsm_in_registers(const double *smem, dvec4 (&X)[2][8])
+template <int RT>
+__device__ __forceinline__ void trsm_in_registers(const double *smem, dvec4 (&X)[RT][8])
 {
     const int l = lane_id();
     const double *Ls = smem;
@@ -225,18 +241,20 @@ __device__ __forceinline__ void trsm_in_registers(const double *smem, dvec4 (&X)
             for (int s = 0; s < 4; ++s) {
                 const double lv = Ls[256 * ((p * (p - 1)) / 2 + q) + l + 64 * s];  // L[16p + l%16][16q + 4s + l/16]
 #pragma unroll
-                for (int t = 0; t < 2; ++t) X[t][p] = mfma_f64(-lv, X[t][q][s], X[t][p]);
+                for (int t = 0; t < RT; ++t) X[t][p] = mfma_f64(-lv, X[t][q][s], X[t][p]);
             }
         }
-        dvec4 z[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+        dvec4 z[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) z[t] = dvec4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const double xv = Xs[256 * p + l + 64 * s];  // X_pp[l%16][4s + l/16]
 #pragma unroll
-            for (int t = 0; t < 2; ++t) z[t] = mfma_f64(xv, X[t][p][s], z[t]);
+            for (int t = 0; t < RT; ++t) z[t] = mfma_f64(xv, X[t][p][s], z[t]);
         }
-        X[0][p] = z[0];
-        X[1][p] = z[1];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) X[t][p] = z[t];
     }
 }
 
@@ -266,8 +284,8 @@ __device__ __forceinline__ void stage_panel_image(double *smem, const double *__
     for (int i = 0; i < (int)(kPanelDoubles / 2 / 256); ++i) dst[threadIdx.x + 256 * i] = src[threadIdx.x + 256 * i];
 }
 
-// Rows 0..127 of P (valid m) <- P * L^{-T} with L and its 8 leaf inverses Xl (read from
-// global into the LDS panel image).  Each wave owns 32 rows.  T = float: P and L are read as
+// Rows 0..64 kRowTiles - 1 of P (valid m) <- P * L^{-T} with L and its 8 leaf inverses Xl (read from
+// global into the LDS panel image).  Each wave owns 16 kRowTiles rows.  T = float: P and L are read as
 // FP32 and widened, the arithmetic is FP64, the result is rounded back to FP32.  If IMAGE is given, the panel image is copied from there instead of built from
 // L and Xl.  If SPLIT (a split-panel slot) is given (T = float), the rounded rows are also
 // written split into split_parts BF16 parts (2 or 3), row i as row split_row0 + i of the slot
@@ -280,10 +298,10 @@ __device__ __forceinline__ void trsm_rows(double *smem, T *__restrict__ P, int64
                                           int64_t split_lo = 0, int64_t split_row0 = 0, int split_parts = 2)
 {
     const int l = lane_id(), w = threadIdx.x >> 6;
-    const int row0 = 32 * w;
-    dvec4 X[2][8];
+    const int row0 = 16 * kRowTiles * w;
+    dvec4 X[kRowTiles][8];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < kRowTiles; ++t) {
         const int i = row0 + 16 * t + (l & 15);
 #pragma unroll
         for (int p = 0; p < 8; ++p)
@@ -301,7 +319,7 @@ __device__ __forceinline__ void trsm_rows(double *smem, T *__restrict__ P, int64
     __syncthreads();
     trsm_in_registers(smem, X);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < kRowTiles; ++t) {
         const int i = row0 + 16 * t + (l & 15);
         if (i < m) {
 #pragma unroll
@@ -334,7 +352,7 @@ __device__ __forceinline__ void diag_update_f64(double *S, const double *__restr
                                                 const double *__restrict__ P0, int64_t lda, int bs)
 {
     constexpr uint32_t kActive = ((1u << (W + 1)) - 1u) | (((1u << (8 - W)) - 1u) << 8);
-    WaveTile<2, 8, 2, true, kActive> t;
+    WaveTile<2, 8, 5, true, kActive> t;  // 72 accumulator registers: room for five k-steps in flight
     const int rows[2] = {16 * W, 16 * (7 - W)};
     t.zero();
     t.load_acc(Akk, lda, rows, 0, bs, bs);
@@ -400,16 +418,6 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
     }
 }
 
-// The diagonal block's strictly lower tiles in S (sl order) -> the panel image W (sls order).
-__device__ __forceinline__ void publish_lower_tiles(const double *S, double *__restrict__ W)
-{
-#pragma unroll
-    for (int q = 0; q < 28; ++q) {
-        const int ti = 1 + (q >= 1) + (q >= 3) + (q >= 6) + (q >= 10) + (q >= 15) + (q >= 21);
-        W[256 * q + threadIdx.x] = S[256 * (q + ti) + threadIdx.x];  // sl tile index = sls index + ti
-    }
-}
-
 // Waits (thread 0) until *flag >= epoch, then every wave acquires: each invalidates its own
 // view of the caches, so that the loads it issues next see what the flag's release published.
 // Returns false (uniformly) on a timeout, recorded as MI_PANEL_TIMEOUT.
@@ -438,8 +446,8 @@ __device__ __forceinline__ bool wait_panel_flag(int *s_ok, const uint32_t *flag,
 //   role 0   : C = A_kk - P_0 P_0^T straight into LDS, Cholesky in LDS, the panel image
 //              (L11's strictly lower tiles and the leaf inverses) to the workspace, publish
 //              `flag` = epoch (release), then L11 into A;
-//   role g>0 : rows k0+128g..+127: C = A_gk - P_g P_0^T, wait for the flag, then rows <-
-//              rows * L11^{-T} with the published image, stored once.
+//   role g>0 : the g-th 64 kRowTiles rows below the block: C = A_gk - P_g P_0^T, wait for the flag,
+//              then rows <- rows * L11^{-T} with the published image, stored once.
 // The diagonal role publishes even on a failing pivot, so that no waiter is left behind;
 // waiters then see `info` and stop.  (LLT.h:350-366: the update of block column k by all
 // earlier panels precedes its unblocked factor and the right-side solve.)
@@ -455,10 +463,10 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
 {
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t R0 = k0 + 128 * (int64_t)g;
-    const int rows = (int)((n - R0) < 128 ? (n - R0) : 128);
+    const int64_t R0 = g == 0 ? k0 : k0 + 128 + 64 * kRowTiles * (int64_t)(g - 1);
+    const int rows = (int)((n - R0) < 64 * kRowTiles ? (n - R0) : 64 * kRowTiles);
     const int bs = (int)((n - k0) < 128 ? (n - k0) : 128);
-    T *Ck = A + R0 + k0 * lda;  // this role's 128 rows of block column k0
+    T *Ck = A + R0 + k0 * lda;  // this role's rows of block column k0
     double *Wp = Wleaf + (size_t)(k0 / 128) * kPanelDoubles;  // the panel image
     double *Xl = Wp + kLeafOffset;
 
@@ -478,12 +486,8 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
         } else {
             block_to_lds(smem, Ck, lda, bs);
         }
-        const int f = potrf_in_lds(smem, Xl, s_ok);  // begins with a barrier
-        if (f >= 0) {
-            if (tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
-        } else {
-            publish_lower_tiles(smem, Wp);
-        }
+        const int f = potrf_in_lds(smem, Xl, s_ok, Wp);  // begins with a barrier
+        if (f >= 0 && tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
         global_barrier();  // every wave's stores of the image have reached L2
         if (tid == 0) publish_flag(flag, epoch);
         if (f < 0) lds_to_block(smem, Ck, lda, bs);  // read by later launches only
@@ -491,8 +495,10 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
     }
 
     if constexpr (sizeof(T) == 8) {
-        WaveTile<2, 8, 2, true, 0xffffffffu, true> t;  // P_0 has all 128 rows (k0 + 128 < n)
-        const int r2[2] = {32 * w, 32 * w + 16};
+        WaveTile<kRowTiles, 8, 3, true, 0xffffffffu, true> t;  // P_0 has all 128 rows (k0 + 128 < n)
+        int r2[kRowTiles];
+#pragma unroll
+        for (int a = 0; a < kRowTiles; ++a) r2[a] = 16 * (kRowTiles * w + a);
         t.zero();
         t.load_acc(Ck, lda, r2, 0, rows, 128);
         if (k0 > 0) {  // C -= P_g P_0^T, P = previous panel (columns k0-128..k0-1): rows R0.. and k0..
@@ -505,7 +511,7 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
         trsm_in_registers(smem, t.acc);
         const int l = lane_id();
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
+        for (int a = 0; a < kRowTiles; ++a) {
             const int i = r2[a] + (l & 15);
             if (i < rows) {
 #pragma unroll
@@ -517,12 +523,13 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
     } else {
         if (k0 > 0) {
             const int wr = w >> 1, wc = w & 1;
-            using Tile = typename TileSel<T, PREC>::type;
+            constexpr int H = 32 * kRowTiles;  // rows of a wave tile
+            using Tile = typename TileSel<T, PREC, H / 16>::type;
             Tile t;
             t.zero();
-            t.setup(A + R0 + (k0 - 128) * lda, lda, wr * 64, rows, A + k0 + (k0 - 128) * lda, lda, wc * 64, bs, 128);
+            t.setup(A + R0 + (k0 - 128) * lda, lda, wr * H, rows, A + k0 + (k0 - 128) * lda, lda, wc * 64, bs, 128);
             t.template run_fixed<128 / Tile::KS>();
-            t.template store<false, false>(Ck, lda, wr * 64, wc * 64, rows, 128);
+            t.template store<false, false>(Ck, lda, wr * H, wc * 64, rows, 128);
         }
         global_barrier();  // this role's updated rows are in L2 before other waves read them back
         if (!wait_panel_flag(s_ok, flag, epoch, status) || factor_failed(info)) return;

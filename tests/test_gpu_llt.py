@@ -54,6 +54,26 @@ def test_factor_matches_oracle(dev, n):
     assert oracle.factor_berr(a, np.tril(m)) <= TOL_BERR
 
 
+@pytest.mark.parametrize("n", [191, 192, 193, 320, 321, 449])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_row_role_edges(dev, n, pad):
+    """Around the 64-row roles below a diagonal block, with an odd leading dimension too.  FP64
+    against the oracle; FP32 by |A - L L^T| <= (n + 2) u (|L| |L^T|) <= 2 (n + 2) u max a_ii."""
+    say(f"[gpu] row roles n={n} pad={pad}")
+    a = workloads.gram_spd(n, seed=n)
+    for dtype, factor in ((torch.float64, mi_llt.potrf_), (torch.float32, mi_llt.spotrf_)):
+        m = torch.full((n, n + pad), 7.0, dtype=dtype, device=dev).t()[:n, :]
+        m.copy_(torch.from_numpy(a).to(dev))
+        assert factor(m) == 0
+        lo = np.tril(m.cpu().numpy().astype(np.float64))
+        if dtype == torch.float64:
+            assert oracle.factor_berr(a, lo) <= TOL_BERR
+        else:
+            a32 = a.astype(np.float32).astype(np.float64)
+            assert np.abs(a32 - lo @ lo.T).max() <= 2 * (n + 2) * 2.0 ** -24 * a32.diagonal().max()
+    assert_status_ok()
+
+
 @pytest.mark.parametrize("tag", ["kat3"] + [f"spd{n}" for n in (1, 2, 3, 7, 8, 16, 31, 32, 33, 64, 100, 127,
                                                                 128, 129, 200)])
 def test_factor_solve_matches_eigen_golden(dev, tag):
