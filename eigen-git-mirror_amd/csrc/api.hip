@@ -194,7 +194,7 @@ int factor_lower(mi_llt_handle h, T *A, int64_t lda, int64_t n, double *wleaf, i
     return 0;
 }
 
-// Diagonal-block inverses of a factor (needs its leaf inverses), for solve_only.
+// Diagonal-block inverses of a factor (wleaf: its panel images, or null), for solve_only.
 template <typename T>
 void block_inverses(mi_llt_handle h, const T *L, int64_t ldl, int64_t n, const double *wleaf, double *winv,
                     const int *d_info, bool couplings = true)
@@ -585,8 +585,7 @@ int mi_dpotrs(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const double 
         L = lay.tri;
         ldl = n;
     }
-    mi::launch_leaf_inverses<double>(L, ldl, n, lay.wleaf, s);
-    rc = solve_lower(h, L, ldl, n, dB, ldb, nrhs, lay.wleaf, lay.winv, nullptr);
+    rc = solve_lower(h, L, ldl, n, dB, ldb, nrhs, nullptr, lay.winv, nullptr);
     if (rc) return rc;
     return check_launch(h, "solve");
 }
@@ -677,18 +676,17 @@ int mi_spotrs(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const float *
     if (dB == nullptr && n > 0 && nrhs > 0) return -7;
     if (ldb < (n > 1 ? n : 1)) return -8;
     if (n == 0 || nrhs == 0) return 0;
-    // [ Wleaf | Winv | lower copy (n * n floats, uplo 'U') | B in FP64 (n * nrhs) ]
+    // [ Winv | lower copy (n * n floats, uplo 'U') | B in FP64 (n * nrhs) ]
     const int64_t nblk = (n + mi::kNB - 1) / mi::kNB;
-    const size_t leaf = round_up((size_t)nblk * mi::kPanelDoubles * sizeof(double));
     const size_t inv = round_up((size_t)nblk * mi::kInvDoubles * sizeof(double));
     const size_t tri = up == 1 ? round_up((size_t)n * n * sizeof(float)) : 0;
     const size_t bw = round_up((size_t)n * nrhs * sizeof(double));
-    int rc = reserve(h, leaf + inv + tri + bw);
+    int rc = reserve(h, inv + tri + bw);
     if (rc) return rc;
     char *p = (char *)h->ws;
-    double *wleaf = (double *)p, *winv = (double *)(p + leaf);
-    float *Lc = (float *)(p + leaf + inv);
-    double *Bd = (double *)(p + leaf + inv + tri);
+    double *winv = (double *)p;
+    float *Lc = (float *)(p + inv);
+    double *Bd = (double *)(p + inv + tri);
     hipStream_t s = h->stream;
     const float *L = dA;
     int64_t ldl = lda;
@@ -698,8 +696,7 @@ int mi_spotrs(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const float *
         ldl = n;
     }
     mi::launch_convert<float, double>(dB, ldb, n, nrhs, Bd, n, s);
-    mi::launch_leaf_inverses<float>(L, ldl, n, wleaf, s);
-    rc = solve_lower<float>(h, L, ldl, n, Bd, n, nrhs, wleaf, winv, nullptr);
+    rc = solve_lower<float>(h, L, ldl, n, Bd, n, nrhs, nullptr, winv, nullptr);
     if (rc) return rc;
     mi::launch_convert<double, float>(Bd, n, n, nrhs, dB, ldb, s);
     return check_launch(h, "spotrs");
@@ -738,15 +735,14 @@ int mi_dtrsm(mi_llt_handle h, char side, char uplo, char transa, char diag, int6
     const bool stage = upper || unit;  // the solve reads a lower, non-unit triangle in place
     const int64_t nrhs = left ? n : m;
     const int64_t nblk = (k + mi::kNB - 1) / mi::kNB;
-    const size_t leaf = round_up((size_t)nblk * mi::kPanelDoubles * sizeof(double));
     const size_t inv = round_up((size_t)nblk * mi::kInvDoubles * sizeof(double));
     const size_t tri = stage ? round_up((size_t)k * k * sizeof(double)) : 0;
     const size_t ct = left ? 0 : round_up((size_t)k * nrhs * sizeof(double));
-    int rc = reserve(h, leaf + inv + tri + ct);
+    int rc = reserve(h, inv + tri + ct);
     if (rc) return rc;
     char *p = (char *)h->ws;
-    double *wleaf = (double *)p, *winv = (double *)(p + leaf);
-    double *Lw = (double *)(p + leaf + inv), *Ct = (double *)(p + leaf + inv + tri);
+    double *winv = (double *)p;
+    double *Lw = (double *)(p + inv), *Ct = (double *)(p + inv + tri);
     const double *L = dA;
     int64_t ldl = lda;
     if (stage) {
@@ -763,8 +759,7 @@ int mi_dtrsm(mi_llt_handle h, char side, char uplo, char transa, char diag, int6
         C = Ct;
         ldc = k;
     }
-    mi::launch_leaf_inverses<double>(L, ldl, k, wleaf, s);
-    block_inverses<double>(h, L, ldl, k, wleaf, winv, nullptr);
+    block_inverses<double>(h, L, ldl, k, nullptr, winv, nullptr);
     if ((rc = solve_only<double>(h, L, ldl, k, C, ldc, nrhs, winv, nullptr, forward ? 1 : 2))) return rc;
     if (!left) mi::launch_transpose_scale(Ct, k, k, m, 1.0, dB, ldb, s);  // B = C^T
     return check_launch(h, "trsm");
@@ -859,25 +854,23 @@ int mi_dpocon(mi_llt_handle h, char uplo, int64_t n, const double *dL, int64_t l
         return 0;
     }
     hipStream_t s = h->stream;
-    // [ Wleaf | Winv | lower copy for uplo 'U' | one vector ]
+    // [ Winv | lower copy for uplo 'U' | one vector ]
     const int64_t nblk = (n + mi::kNB - 1) / mi::kNB;
-    const size_t leaf = round_up((size_t)nblk * mi::kPanelDoubles * sizeof(double));
     const size_t inv = round_up((size_t)nblk * mi::kInvDoubles * sizeof(double));
     const size_t tri = up == 1 ? round_up((size_t)n * n * sizeof(double)) : 0;
-    int rc = reserve(h, leaf + inv + tri + round_up((size_t)n * sizeof(double)));
+    int rc = reserve(h, inv + tri + round_up((size_t)n * sizeof(double)));
     if (rc) return rc;
     char *p = (char *)h->ws;
-    double *wleaf = (double *)p, *winv = (double *)(p + leaf), *dv = (double *)(p + leaf + inv + tri);
+    double *winv = (double *)p, *dv = (double *)(p + inv + tri);
     const double *L = dL;
     int64_t ld = ldl;
     if (up == 1) {
-        double *Lc = (double *)(p + leaf + inv);
+        double *Lc = (double *)(p + inv);
         mi::launch_upper_to_lower(dL, ldl, n, Lc, n, s);
         L = Lc;
         ld = n;
     }
-    mi::launch_leaf_inverses<double>(L, ld, n, wleaf, s);
-    block_inverses<double>(h, L, ld, n, wleaf, winv, nullptr);
+    block_inverses<double>(h, L, ld, n, nullptr, winv, nullptr);
     std::vector<double> v((size_t)n), sgn((size_t)n), old_sgn((size_t)n);
     // v <- A^{-1} v with the factor (the same solve serves dec.solve and dec.adjoint().solve:
     // A is symmetric, LLT.h:204)
@@ -1081,23 +1074,20 @@ int mi_dpotrf_adjoint(mi_llt_handle h, char uplo, int64_t n, const double *dL, i
     if (n == 0) return 0;
     hipStream_t s = h->stream;
     const int64_t nblk = (n + mi::kNB - 1) / mi::kNB;
-    const size_t leaf = round_up((size_t)nblk * mi::kPanelDoubles * sizeof(double));
     const size_t inv = round_up((size_t)nblk * mi::kInvDoubles * sizeof(double));
     const size_t sq = round_up((size_t)n * (size_t)n * sizeof(double));
-    int rc = reserve(h, leaf + inv + 3 * sq);
+    int rc = reserve(h, inv + 3 * sq);
     if (rc) return rc;
-    double *wleaf = (double *)h->ws;
-    double *winv = (double *)((char *)h->ws + leaf);
-    double *W2 = (double *)((char *)h->ws + leaf + inv);
-    double *W3 = (double *)((char *)h->ws + leaf + inv + sq);
-    double *Wt = (double *)((char *)h->ws + leaf + inv + 2 * sq);  // tril(L)^T
+    double *winv = (double *)h->ws;
+    double *W2 = (double *)((char *)h->ws + inv);
+    double *W3 = (double *)((char *)h->ws + inv + sq);
+    double *Wt = (double *)((char *)h->ws + inv + 2 * sq);  // tril(L)^T
     const double nd = (double)n;
     mi::launch_sym_tile(4, dL, ldl, n, Wt, n, s);  // tril(L)^T
     mi::launch_sym_tile(4, dG, ldg, n, W3, n, s);  // tril(Lbar)^T, then overwritten by P
     traced(h, s, MI_TRACE_GEMM, nd * nd * nd / 3.0, [&] { mi::launch_trmm_tn_lower(Wt, n, W3, n, n, W3, n, W2, s); });
     mi::launch_sym_tile(0, W3, n, n, W2, n, s);              // M
-    mi::launch_leaf_inverses<double>(dL, ldl, n, wleaf, s);  // recomputed from L
-    block_inverses<double>(h, dL, ldl, n, wleaf, winv, nullptr, false);  // no solve here
+    block_inverses<double>(h, dL, ldl, n, nullptr, winv, nullptr, false);  // no solve here
     traced(h, s, MI_TRACE_SOLVE, nd * nd * nd,
            [&] { mi::launch_trsm_xl_multi(Wt, n, n, W2, n, n, winv, false, s); });  // Y = M L^{-1}
     mi::launch_sym_tile(1, W2, n, n, W3, n, s);                                      // Y^T = L^{-T} M
@@ -1127,17 +1117,14 @@ int mi_dpotrs_adjoint(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const
     if (n == 0 || nrhs == 0) return 0;
     hipStream_t s = h->stream;
     const int64_t nblk = (n + mi::kNB - 1) / mi::kNB;
-    const size_t leaf = round_up((size_t)nblk * mi::kPanelDoubles * sizeof(double));
     const size_t inv = round_up((size_t)nblk * mi::kInvDoubles * sizeof(double));
     const size_t vec = round_up((size_t)n * (size_t)nrhs * sizeof(double));
-    int rc = reserve(h, leaf + inv + 2 * vec);
+    int rc = reserve(h, inv + 2 * vec);
     if (rc) return rc;
-    double *wleaf = (double *)h->ws;
-    double *winv = (double *)((char *)h->ws + leaf);
-    double *U = (double *)((char *)h->ws + leaf + inv);
-    double *V = (double *)((char *)h->ws + leaf + inv + vec);
-    mi::launch_leaf_inverses<double>(dL, ldl, n, wleaf, s);
-    block_inverses<double>(h, dL, ldl, n, wleaf, winv, nullptr);
+    double *winv = (double *)h->ws;
+    double *U = (double *)((char *)h->ws + inv);
+    double *V = (double *)((char *)h->ws + inv + vec);
+    block_inverses<double>(h, dL, ldl, n, nullptr, winv, nullptr);
     if ((rc = solve_only<double>(h, dL, ldl, n, dXbar, ldxb, nrhs, winv, nullptr))) return rc;  // Bbar
     mi::launch_solve_adjoint_update(dL, ldl, n, nrhs, dX, ldx, dXbar, ldxb, dLbar, ldlb, U, V, s);
     return check_launch(h, "potrs_adjoint");
@@ -1255,9 +1242,8 @@ int mi_dpotrs_batched(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, int64
     hipStream_t s = h->stream;
     bl.bt.a = strideL;
     bl.bt.b = strideB;
-    mi::launch_leaf_inverses<double>(dL, ldl, n, bl.leaf, s, bl.bt);
     traced(h, s, MI_TRACE_TRTRI, (double)n * mi::kNB * mi::kNB / 3.0 * (double)batch,
-           [&] { mi::launch_block_inverses<double>(dL, ldl, n, bl.leaf, bl.inv, nullptr, s, true, bl.bt); });
+           [&] { mi::launch_block_inverses<double>(dL, ldl, n, nullptr, bl.inv, nullptr, s, true, bl.bt); });
     traced(h, s, MI_TRACE_SOLVE, 2.0 * (double)n * (double)n * (double)nrhs * (double)batch, [&] {
         mi::launch_solve_persistent<double>(dL, ldl, n, dB, ldb, nrhs, bl.inv, bl.pack,
                                             (int *)batch_sync(h) + mi::kSyncSolveTickets, nullptr, shared_status(h), s,
@@ -1293,9 +1279,8 @@ int mi_dpotrf_adjoint_batched(mi_llt_handle h, char uplo, int64_t n, int64_t bat
     traced(h, s, MI_TRACE_GEMM, nd * nd * nd / 3.0 * bd,
            [&] { mi::launch_trmm_tn_lower(Wt, n, W3, n, n, W3, n, W2, s, nb, sa, sa, sa, sa); });
     mi::launch_sym_tile(0, W3, n, n, W2, n, s, nb, sa, sa);  // M
-    mi::launch_leaf_inverses<double>(dL, ldl, n, bl.leaf, s, bl.bt);
     traced(h, s, MI_TRACE_TRTRI, nd * mi::kNB * mi::kNB / 3.0 * bd,
-           [&] { mi::launch_block_inverses<double>(dL, ldl, n, bl.leaf, bl.inv, nullptr, s, false, bl.bt); });
+           [&] { mi::launch_block_inverses<double>(dL, ldl, n, nullptr, bl.inv, nullptr, s, false, bl.bt); });
     traced(h, s, MI_TRACE_SOLVE, nd * nd * nd * bd,
            [&] { mi::launch_trsm_xl_multi(Wt, n, n, W2, n, n, bl.inv, false, s, nb, sa, sa, bl.bt.inv); });
     mi::launch_sym_tile(1, W2, n, n, W3, n, s, nb, sa, sa);  // Y^T
@@ -1331,8 +1316,7 @@ int mi_dpotrs_adjoint_batched(mi_llt_handle h, char uplo, int64_t n, int64_t nrh
     hipStream_t s = h->stream;
     bl.bt.a = strideL;
     bl.bt.b = strideXbar;
-    mi::launch_leaf_inverses<double>(dL, ldl, n, bl.leaf, s, bl.bt);
-    mi::launch_block_inverses<double>(dL, ldl, n, bl.leaf, bl.inv, nullptr, s, true, bl.bt);
+    mi::launch_block_inverses<double>(dL, ldl, n, nullptr, bl.inv, nullptr, s, true, bl.bt);
     traced(h, s, MI_TRACE_SOLVE, 2.0 * (double)n * (double)n * (double)nrhs * (double)batch, [&] {  // Bbar
         mi::launch_solve_persistent<double>(dL, ldl, n, dXbar, ldxb, nrhs, bl.inv, bl.pack,
                                             (int *)batch_sync(h) + mi::kSyncSolveTickets, nullptr, shared_status(h), s,
@@ -1413,9 +1397,8 @@ int mi_dposv_adjoint_batched(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs
     bl.bt.a = strideL;
     bl.bt.b = strideXbar;
     // one set of diagonal-block inverses (with the solve's couplings) serves both adjoints
-    mi::launch_leaf_inverses<double>(dL, ldl, n, bl.leaf, s, bl.bt);
     traced(h, s, MI_TRACE_TRTRI, nd * mi::kNB * mi::kNB / 3.0 * bd,
-           [&] { mi::launch_block_inverses<double>(dL, ldl, n, bl.leaf, bl.inv, nullptr, s, true, bl.bt); });
+           [&] { mi::launch_block_inverses<double>(dL, ldl, n, nullptr, bl.inv, nullptr, s, true, bl.bt); });
     if (nrhs > 0) {  // the solve's adjoint: Bbar = A^{-1} Xbar, Lbar -= tril(Bbar (L^T X)^T + X (L^T Bbar)^T)
         traced(h, s, MI_TRACE_SOLVE, 2.0 * nd * nd * (double)nrhs * bd, [&] {
             mi::launch_solve_persistent<double>(dL, ldl, n, dXbar, ldxb, nrhs, bl.inv, bl.pack,

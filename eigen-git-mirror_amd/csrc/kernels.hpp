@@ -14,7 +14,7 @@ constexpr int kNB = 128;
 //             (tile (ti, tj), ti > tj, at 256 * (ti(ti-1)/2 + tj), each column-major), then at
 //             kLeafOffset the 8 inverses of its 16 x 16 diagonal leaves (column-major).  The
 //             factorization's diagonal role publishes it for the panel solve, which copies it
-//             to LDS as it is; the solve-only path fills the leaf part alone.
+//             to LDS as it is.
 //   Winv[b] : L_bb^{-T}, 128 x 128, ld 128 (built for the solve)
 constexpr int64_t kPanelDoubles = 36 * 256;
 constexpr int64_t kLeafOffset = 28 * 256;
@@ -79,15 +79,12 @@ __host__ __device__ inline int64_t split_part_elems(int64_t n) { return ((n + 12
 // reads panels k-7..k (the 2-part split schedule), so 9 are in use at once.
 constexpr int kSplitRing = 16;
 __host__ __device__ inline int64_t split_slot_elems(int64_t n, int parts) { return parts * split_part_elems(n); }
-// Winv[b] = {X_b^T, X_b, M_b, N_b, M2_b, N2_b}, X_b = L_bb^{-1}, for every diagonal block (needs Wleaf).
+// Winv[b] = {X_b^T, X_b, M_b, N_b, M2_b, N2_b}, X_b = L_bb^{-1}, for every diagonal block
+// (Wleaf: the factorization's panel images, or null for a factor without them).
 // couplings = false: X_b^T and X_b only (for users of Winv other than the solve).
 template <typename T>
 void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wleaf, double *Winv, const int *info,
                            hipStream_t s, bool couplings = true, const Batch &bt = Batch());
-// Wleaf from an already factored matrix (standalone solve).
-template <typename T>
-void launch_leaf_inverses(const T *L, int64_t lda, int64_t n, double *Wleaf, hipStream_t s,
-                          const Batch &bt = Batch());
 // Solve: forward then backward sweep in place on B (one persistent launch each, each after a
 // small reset launch).  tickets: 2 ints; Ypk: solve_pack_doubles(n, nrhs) doubles of scratch
 // (each finished block's packed copy for its consumers), used by the two sweeps in turn: each

@@ -3,45 +3,132 @@
 // The diagonal-block Cholesky itself (llt_inplace<double,Lower>::unblocked on A11,
 // Eigen/src/Cholesky/LLT.h:312-336, called at :363) and the panel solve (LLT.h:364) run
 // inside the fused factorization step (factor_step.hip, potrf_device.hpp):
-//   * the 128 x 128 block is held in LDS and factored in 16-column panels; one wave holds
-//     a panel in registers, two rows per lane, and runs the column loop of LLT.h:320-334
-//     (pivot test, sqrt, scale, rank-1 update) with lane broadcasts (readlane) instead of
-//     barriers; then that wave inverts the 16 x 16 leaf while the other three apply the
-//     rank-16 update to the rest of the block with FP64 MFMA from LDS;
+//   * the 128 x 128 block is held in LDS and factored in 16-column panels: two waves run the
+//     column loop of LLT.h:320-334 (pivot test, sqrt, scale, rank-1 update) in registers on the
+//     row broadcast, which leaves the inverse of the 16 x 16 leaf too, while the other two
+//     apply the previous panel's rank-16 update to the rest of the block with FP64 MFMA;
 //   * the pivot test is Eigen's `x <= 0 -> fail at column k` (LLT.h:327-330), so a NaN
 //     pivot passes as in Eigen; the first failing column goes to `info` (LAPACK k+1); a last
 //     block narrower than 128 is padded with the identity (L_pad = [L 0; 0 I]);
 //   * the panel solve A21 <- A21 L11^{-T} (TriangularSolverMatrix.h:186-329) is blocked by
 //     16 columns with the leaf inverses; the MFMA result layout is the operand layout of the
 //     next k-step, so solved blocks feed the next MFMAs straight from registers.
-// The solve's block inverses L_bb^{-1} are built after the factor from its leaf inverses
-// (block_inverse_kernel), and the couplings from them (block_coupling_kernel).
+// The solve's block inverses L_bb^{-1} are built after the factor from its leaf inverses or from L
+// alone (block_inverse_kernel), and the couplings from them (block_coupling_kernel).
+#include "leaf_device.hpp"
 #include "potrf_device.hpp"
 
 namespace mi {
 
 // Packed lower 16 x 16 tiles of a 128 x 128 block in LDS, the diagonal included: tile (ti, tj),
-// ti >= tj, at 256 (ti (ti + 1) / 2 + tj), column-major.
-__device__ __forceinline__ int tile_at(int ti, int tj) { return 256 * ((ti * (ti + 1)) / 2 + tj); }
+// ti >= tj, at kTile (ti (ti + 1) / 2 + tj), column-major with a column every kTileLd doubles: one
+// more than the rows, so that 16 lanes reading along a row hit different banks.
+constexpr int kTileLd = 17, kTile = 16 * kTileLd;
+__device__ __forceinline__ constexpr int tile_at(int ti, int tj) { return kTile * ((ti * (ti + 1)) / 2 + tj); }
 
-// acc += A B for 16 x 16 tiles at LDS offsets a and bb (column-major): the MFMA operands are
-// P[i][k] = A[i][k] and Q[j][k] = B[k][j], k = 4s + lane/16; acc[r] is (lane%16, 4r + lane/16).
-__device__ __forceinline__ void tile_mma(const double *S, int a, int bb, dvec4 &acc)
+// The MFMA operands of 16 x 16 tiles at LDS offset o: of A in a product A B (P[i][k] = A[i][k]) and
+// of B (Q[j][k] = B[k][j]), k = 4s + lane/16.
+__device__ __forceinline__ void tile_p(const double *S, int o, double (&p)[4])
 {
-    const int l = lane_id(), i = l & 15, kl = l >> 4;
+    const int l = lane_id();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) acc = mfma_f64(S[bb + 4 * s + kl + 16 * i], S[a + i + 16 * (4 * s + kl)], acc);
+    for (int s = 0; s < 4; ++s) p[s] = S[o + (l & 15) + kTileLd * (4 * s + (l >> 4))];
+}
+__device__ __forceinline__ void tile_q(const double *S, int o, double (&q)[4])
+{
+    const int l = lane_id();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) q[s] = S[o + 4 * s + (l >> 4) + kTileLd * (l & 15)];
+}
+// acc += A B; acc[r] is element (lane%16, 4r + lane/16).
+__device__ __forceinline__ void tile_mma(const double (&p)[4], const double (&q)[4], dvec4 &acc)
+{
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = mfma_f64(q[s], p[s], acc);
+}
+__device__ __forceinline__ void tile_put(double *S, int o, const dvec4 &acc, bool negate)
+{
+    const int l = lane_id();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[o + (l & 15) + kTileLd * (4 * r + (l >> 4))] = negate ? -acc[r] : acc[r];
+}
+
+// One level of the tree over the diagonal: pairs of SZ-tile blocks A (tiles A0 ..) and B (tiles
+// A0 + SZ ..), T = L_BA X_AA and then X_BA = -X_BB T, in place of L_BA.  A wave takes a tile row of
+// T, then a tile column of X_BA, of pair w / SZ: equal shares, as X_AA and X_BB are triangular, and
+// each operand tile of the row or column is read once.
+template <int SZ>
+__device__ __forceinline__ void inverse_level(double *S, int w)
+{
+    const int A0 = (w / SZ) * 2 * SZ, B0 = A0 + SZ, x = w % SZ;
+    dvec4 acc[SZ];
+    double p[SZ][4], q[4];
+#pragma unroll
+    for (int k = 0; k < SZ; ++k) tile_p(S, tile_at(B0 + x, A0 + k), p[k]);
+#pragma unroll
+    for (int tj = 0; tj < SZ; ++tj) {
+        acc[tj] = dvec4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = tj; k < SZ; ++k) {
+            tile_q(S, tile_at(A0 + k, A0 + tj), q);
+            tile_mma(p[k], q, acc[tj]);
+        }
+    }
+    // only this wave reads its tile row of L_BA
+#pragma unroll
+    for (int tj = 0; tj < SZ; ++tj) tile_put(S, tile_at(B0 + x, A0 + tj), acc[tj], false);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < SZ; ++k) tile_q(S, tile_at(B0 + k, A0 + x), p[k]);
+#pragma unroll
+    for (int ti = 0; ti < SZ; ++ti) {
+        acc[ti] = dvec4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k <= ti; ++k) {
+            tile_p(S, tile_at(B0 + ti, B0 + k), q);
+            tile_mma(q, p[k], acc[ti]);
+        }
+    }
+    // only this wave reads its tile column of T
+#pragma unroll
+    for (int ti = 0; ti < SZ; ++ti) tile_put(S, tile_at(B0 + ti, A0 + x), acc[ti], true);
+    __syncthreads();
+}
+
+// Step K of the inverse of a lower 16 x 16 leaf: lane c of a row of 16 holds row c of the leaf in
+// v[0..15] and column c of the inverse in x[0..15].  x[K] is final after the division; rows M > K
+// take L_MK x[K] away.  (Lanes c > K are left alone: their x[K] is 0, but L_MK may be infinite.)
+template <int K, int M>
+__device__ __forceinline__ void leaf_inverse_rows(const double (&v)[16], double (&x)[16], int c)
+{
+    if constexpr (M < 16) {
+        double t = x[M];
+        row_fnma<M, M == K + 1>(t, v[K], x[K]);
+        x[M] = c <= K ? t : x[M];
+        leaf_inverse_rows<K, M + 1>(v, x, c);
+    }
+}
+template <int K>
+__device__ __forceinline__ void leaf_inverse_steps(const double (&v)[16], double (&x)[16], int c)
+{
+    if constexpr (K < 16) {
+        const double d = row_bcast<K>(v[K]);
+        x[K] = c <= K ? x[K] / d : 0.0;
+        leaf_inverse_rows<K, K + 1>(v, x, c);
+        leaf_inverse_steps<K + 1>(v, x, c);
+    }
 }
 
 // Workgroup b: X_b^T = L_bb^{-T} to Wout + b*kInvDoubles (ld 128) and X_b at + kInvX.
 // A triangular inverse by a tree over the diagonal 16 x 16 leaves (the recursive form of
-// LAPACK's dtrtri): from the 8 leaf inverses X_pp of the factorization, three levels double
-// the inverted diagonal blocks, X_BA = -X_BB (L_BA X_AA) for [A; B] of 16 + 16, 32 + 32 and
-// 64 + 64 rows, each level's products over 16 x 16 tiles on FP64 MFMA, in place in LDS (L_BA
-// is replaced by the product T = L_BA X_AA, then by X_BA).  Three levels of two products each
+// LAPACK's dtrtri): from the 8 leaf inverses X_pp, three levels double the inverted diagonal
+// blocks, X_BA = -X_BB (L_BA X_AA) for [A; B] of 16 + 16, 32 + 32 and 64 + 64 rows, each level's
+// products over 16 x 16 tiles on FP64 MFMA, in place in LDS.  Three levels of two products each
 // instead of eight dependent 16-column solve steps: the kernel is bound by one workgroup's
-// latency, not by its flops.  Beyond bs (a last block narrower than 128) L reads as 0 and the
-// leaf inverses are the identity's, so X is padded with the identity.
+// latency, not by its flops.  The leaf inverses come from the factorization's panel images, or,
+// without them (Wleaf null: a factor the caller kept), from the leaves, two per wave on the row
+// broadcast, where a kernel of its own took as long as this one.  Beyond bs (a last block narrower
+// than 128) L reads as the identity, so X is padded with the identity.
 // Batched launches (every kernel of this file): system z = blockIdx.z, its pointers advanced
 // by z times their strides (s*), its info at info + z.
 template <typename T>
@@ -50,10 +137,9 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict_
                                                             double *__restrict__ Wout, const int *info, int64_t sL,
                                                             int64_t sWl, int64_t sWo)
 {
-    __shared__ double S[kSmem];  // the 36 packed lower tiles
+    __shared__ double S[36 * kTile];  // the packed lower tiles
     const int64_t z = blockIdx.z;
     L += z * sL;
-    Wleaf += z * sWl;
     Wout += z * sWo;
     if (info) info += z;
     if (factor_failed(info)) return;
@@ -61,99 +147,73 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict_
     const int64_t kb = (int64_t)b * 128;
     const int bs = (int)((n - kb) < 128 ? (n - kb) : 128);
     const T *Lb = L + kb + kb * ldl;
-    const double *Xl = Wleaf + (size_t)b * kPanelDoubles + kLeafOffset;
     const int tid = threadIdx.x, l = lane_id();
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // the strictly lower tiles of L_bb (0 beyond bs) and the leaf inverses on the diagonal: a
-    // thread takes row r, columns of parity tid / 128, its loads issued 16 at a time (from
-    // clamped, in-bounds addresses) before their LDS stores
+    // the lower tiles of L_bb: a thread takes row r, columns of parity tid / 128, all its loads in
+    // flight (from clamped, in-bounds addresses) before their LDS stores
     {
         const int r = tid & 127, ch = tid >> 7, rt = r >> 4;
         double x[8];
+        if (Wleaf) {
+            const double *Xl = Wleaf + z * sWl + (size_t)b * kPanelDoubles + kLeafOffset;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) x[q] = Xl[tid + 256 * q];
+            for (int q = 0; q < 8; ++q) x[q] = Xl[tid + 256 * q];
+        }
+        T v[64];
 #pragma unroll
-        for (int q0 = 0; q0 < 64; q0 += 16) {
-            double v[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int c = 2 * (q0 + q) + ch;
-                const bool in = r < bs && c < bs;
-                v[q] = (double)Lb[(in ? r : 0) + (int64_t)(in ? c : 0) * ldl];
-            }
-#pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int c = 2 * (q0 + q) + ch;
-                const bool in = r < bs && c < bs;
-                if ((c >> 4) < rt) S[tile_at(rt, c >> 4) + (r & 15) + 16 * (c & 15)] = in ? v[q] : 0.0;
-            }
+        for (int q = 0; q < 64; ++q) {
+            const int c = 2 * q + ch;
+            const bool in = r < bs && c <= r;
+            v[q] = Lb[(in ? r : 0) + (int64_t)(in ? c : 0) * ldl];
         }
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {  // element tid of leaf q: (tid % 16, tid / 16)
-            const int i = tid & 15, j = tid >> 4;
-            S[tile_at(q, q) + tid] = j <= i ? x[q] : 0.0;
+        for (int q = 0; q < 64; ++q) {
+            const int c = 2 * q + ch;
+            const bool in = r < bs && c <= r;
+            if ((q >> 3) <= rt) S[tile_at(rt, q >> 3) + (r & 15) + kTileLd * (c & 15)] = in ? (double)v[q] : r == c ? 1.0 : 0.0;
+        }
+        __syncthreads();
+        if (Wleaf) {  // element tid of leaf q: (tid % 16, tid / 16)
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                S[tile_at(q, q) + (tid & 15) + kTileLd * (tid >> 4)] = (tid >> 4) <= (tid & 15) ? x[q] : 0.0;
+        } else {
+            const int c = l & 15, o = tile_at(2 * w, 2 * w) + ((l >> 4) & 1) * (tile_at(2 * w + 1, 2 * w + 1) - tile_at(2 * w, 2 * w));
+            double u[16], y[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                u[k] = S[o + c + kTileLd * k];
+                y[k] = k == c ? 1.0 : 0.0;
+            }
+            leaf_inverse_steps<0>(u, y, c);
+            if (l < 32) {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) S[o + k + kTileLd * c] = y[k];
+            }
         }
     }
     __syncthreads();
+    inverse_level<1>(S, w);
+    inverse_level<2>(S, w);
+    inverse_level<4>(S, w);
 
-    // level v: pairs of sz-tile blocks A (tiles A0 ..) and B (tiles A0 + sz ..); 4 sz output
-    // tiles (B0 + ti, A0 + tj) per level, dealt over the 4 waves
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-        const int sz = 1 << v, nout = 4 * sz;
-        dvec4 acc[4];
-        // T = L_BA X_AA (X_AA lower: k >= tj)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc[q] = dvec4{0.0, 0.0, 0.0, 0.0};
-            const int o = w + 4 * q;
-            if (o < nout) {
-                const int A0 = (o / (sz * sz)) * 2 * sz, B0 = A0 + sz, ti = (o % (sz * sz)) / sz, tj = o % sz;
-                for (int k = tj; k < sz; ++k) tile_mma(S, tile_at(B0 + ti, A0 + k), tile_at(A0 + k, A0 + tj), acc[q]);
-            }
-        }
-        __syncthreads();  // every wave has read L_BA
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int o = w + 4 * q;
-            if (o < nout) {
-                const int A0 = (o / (sz * sz)) * 2 * sz, B0 = A0 + sz, ti = (o % (sz * sz)) / sz, tj = o % sz;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) S[tile_at(B0 + ti, A0 + tj) + (l & 15) + 16 * (4 * r + (l >> 4))] = acc[q][r];
-            }
-        }
-        __syncthreads();
-        // X_BA = -X_BB T (X_BB lower: k <= ti)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            acc[q] = dvec4{0.0, 0.0, 0.0, 0.0};
-            const int o = w + 4 * q;
-            if (o < nout) {
-                const int A0 = (o / (sz * sz)) * 2 * sz, B0 = A0 + sz, ti = (o % (sz * sz)) / sz, tj = o % sz;
-                for (int k = 0; k <= ti; ++k) tile_mma(S, tile_at(B0 + ti, B0 + k), tile_at(B0 + k, A0 + tj), acc[q]);
-            }
-        }
-        __syncthreads();  // every wave has read T
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int o = w + 4 * q;
-            if (o < nout) {
-                const int A0 = (o / (sz * sz)) * 2 * sz, B0 = A0 + sz, ti = (o % (sz * sz)) / sz, tj = o % sz;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) S[tile_at(B0 + ti, A0 + tj) + (l & 15) + 16 * (4 * r + (l >> 4))] = -acc[q][r];
-            }
-        }
-        __syncthreads();
-    }
-
-    // X to Wout + kInvX and X^T to Wout (ld 128), zeros above the diagonal
+    // X to Wout + kInvX and X^T to Wout (ld 128), zeros above the diagonal; two elements a store
     double *Wt = Wout + (size_t)b * kInvDoubles, *Wx = Wt + kInvX;
-    for (int e = tid; e < 128 * 128; e += 256) {
-        const int r = e & 127, c = e >> 7;
-        const double x = (r >> 4) >= (c >> 4) ? S[tile_at(r >> 4, c >> 4) + (r & 15) + 16 * (c & 15)] : 0.0;
-        Wx[r + 128 * c] = x;
-        Wt[c + 128 * r] = x;
+#pragma unroll 8
+    for (int e = tid; e < 128 * 64; e += 256) {
+        const int f = 2 * (e & 63), c = e >> 6;  // elements (f, c), (f + 1, c) of X and of X^T
+        dvec2 x = {0.0, 0.0}, xt = {0.0, 0.0};
+        if ((f >> 4) >= (c >> 4)) {
+            const double *t = S + tile_at(f >> 4, c >> 4) + (f & 15) + kTileLd * (c & 15);
+            x = dvec2{t[0], t[1]};
+        }
+        if ((c >> 4) >= (f >> 4)) {
+            const double *t = S + tile_at(c >> 4, f >> 4) + (c & 15) + kTileLd * (f & 15);
+            xt = dvec2{t[0], t[kTileLd]};
+        }
+        *(dvec2 *)(Wx + f + 128 * c) = x;
+        *(dvec2 *)(Wt + f + 128 * c) = xt;
     }
 }
 
@@ -223,53 +283,6 @@ __global__ __launch_bounds__(256) void block_coupling_kernel(const T *__restrict
                 C[(64 * wr + 16 * a + (l & 15)) + 128 * (64 * wc + 16 * q + 4 * r + kl)] = acc[a][q][r];
 }
 
-// Leaf inverses of the diagonal blocks of an already factored matrix: workgroup b, wave w
-// inverts leaves 2w and 2w+1 of block b (lane i < 16 holds row i of the leaf).
-template <typename T>
-__global__ __launch_bounds__(256) void leaf_inverse_kernel(const T *__restrict__ L, int64_t lda, int64_t n,
-                                                           double *__restrict__ Wleaf, int64_t sL, int64_t sWl)
-{
-    L += (int64_t)blockIdx.z * sL;
-    Wleaf += (int64_t)blockIdx.z * sWl;
-    const int l = lane_id(), w = threadIdx.x >> 6;
-    const int64_t kb = (int64_t)blockIdx.x * 128;
-    const int bs = (int)((n - kb) < 128 ? (n - kb) : 128);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int p = 2 * w + h;
-        const int c0 = 16 * p;
-        double v[16], x[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const int r = c0 + l, cc = c0 + c;
-            double val = 0.0;
-            const bool in = l < 16 && r < bs && cc < bs;
-            const double lraw = (double)L[kb + (in ? r : 0) + (kb + (in ? cc : 0)) * lda];
-            if (l < 16 && c <= l) val = in ? lraw : (r == cc ? 1.0 : 0.0);
-            v[c] = val;
-            x[c] = (c == l) ? 1.0 : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const double lkk = readlane_d(v[k], k);
-            if (l == k) {
-#pragma unroll
-                for (int c = 0; c <= k; ++c) x[c] = x[c] / lkk;
-            }
-#pragma unroll
-            for (int c = 0; c <= k; ++c) {
-                const double xkc = readlane_d(x[c], k);
-                if (l > k) x[c] -= v[k] * xkc;
-            }
-        }
-        if (l < 16) {
-#pragma unroll
-            for (int c = 0; c < 16; ++c)
-                Wleaf[(size_t)blockIdx.x * kPanelDoubles + kLeafOffset + p * 256 + l + 16 * c] = (c <= l) ? x[c] : 0.0;
-        }
-    }
-}
-
 template <typename T>
 void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wleaf, double *Winv, const int *info,
                            hipStream_t s, bool couplings, const Batch &bt)
@@ -282,19 +295,9 @@ void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wle
                            s, L, lda, n, Winv, info, bt.a, bt.inv);
 }
 
-template <typename T>
-void launch_leaf_inverses(const T *L, int64_t lda, int64_t n, double *Wleaf, hipStream_t s, const Batch &bt)
-{
-    const unsigned nblk = (unsigned)((n + 127) / 128);
-    hipLaunchKernelGGL(leaf_inverse_kernel<T>, dim3(nblk, 1, bt.count), dim3(256), 0, s, L, lda, n, Wleaf, bt.a,
-                       bt.leaf);
-}
-
 template void launch_block_inverses<double>(const double *, int64_t, int64_t, const double *, double *, const int *,
                                             hipStream_t, bool, const Batch &);
 template void launch_block_inverses<float>(const float *, int64_t, int64_t, const double *, double *, const int *,
                                            hipStream_t, bool, const Batch &);
-template void launch_leaf_inverses<double>(const double *, int64_t, int64_t, double *, hipStream_t, const Batch &);
-template void launch_leaf_inverses<float>(const float *, int64_t, int64_t, double *, hipStream_t, const Batch &);
 
 }  // namespace mi
