@@ -1425,4 +1425,36 @@ int mi_dposv_adjoint_batched(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs
     return check_launch(h, "posv_adjoint_batched");
 }
 
+int mi_dgp_gradient_batched(mi_llt_handle h, int64_t n, int64_t batch, const double *dL, int64_t ldl, int64_t strideL,
+                            const double *dAlpha, int64_t strideAlpha, const double *dG, double *dK, int64_t ldk,
+                            int64_t strideK)
+{
+    if (!valid(h)) return MI_LLT_E_HANDLE;
+    if (n < 0) return -2;
+    if (batch < 0 || batch > 65535) return -3;
+    if (int e = check_batch_args(n, n, batch, ldl, strideL, dL)) return e == 2 ? -4 : (e == 3 ? -5 : -6);
+    if (int e = check_batch_args(n, 1, batch, n > 1 ? n : 1, strideAlpha, dAlpha)) return e == 2 ? -7 : -8;
+    if (dG == nullptr && n > 0 && batch > 0) return -9;
+    if (int e = check_batch_args(n, n, batch, ldk, strideK, dK)) return e == 2 ? -10 : (e == 3 ? -11 : -12);
+    if (n == 0 || batch == 0) return 0;
+    const size_t np = (size_t)(n + mi::kNB - 1) / mi::kNB * mi::kNB, edge = (size_t)mi::inverse_pairs_edge(n);
+    const size_t v = np * (np + mi::kNB), w = edge * edge;
+    int rc = reserve(h, (v + w) * (size_t)batch * sizeof(double));
+    if (rc) return rc;
+    double *V = (double *)h->ws, *W = V + v * (size_t)batch;
+    mi::Batch bt;
+    bt.count = (unsigned)batch;
+    bt.a = strideL;
+    bt.b = strideAlpha;
+    bt.g = strideK;
+    bt.aux = (int64_t)v;
+    bt.aux2 = (int64_t)w;
+    hipStream_t s = h->stream;
+    const double nd = (double)n, bd = (double)batch;
+    traced(h, s, MI_TRACE_TRTRI, nd * nd * nd / 3.0 * bd, [&] { mi::launch_factor_inverse(dL, ldl, n, V, W, s, bt); });
+    traced(h, s, MI_TRACE_GEMM, nd * nd * nd / 3.0 * bd,
+           [&] { mi::launch_gp_gradient(V, n, dAlpha, dG, dK, ldk, s, bt); });
+    return check_launch(h, "gp_gradient_batched");
+}
+
 }  // extern "C"

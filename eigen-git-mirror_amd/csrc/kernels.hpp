@@ -85,6 +85,18 @@ __host__ __device__ inline int64_t split_slot_elems(int64_t n, int parts) { retu
 template <typename T>
 void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wleaf, double *Winv, const int *info,
                            hipStream_t s, bool couplings = true, const Batch &bt = Batch());
+// X_b^T to Wt + b stride and X_b to Wx + b stride (ld ldw, even like stride; systems sW apart).
+void launch_block_inverses_to(const double *L, int64_t lda, int64_t n, double *Wt, double *Wx, int64_t ldw,
+                              int64_t stride, hipStream_t s, unsigned count, int64_t sL, int64_t sW);
+// V (np x (np + 128), ld np = n rounded up to 128s) <- L^{-1} in its block-lower part and its
+// transpose one block column to the right; W: inverse_pairs_edge(n)^2 doubles of scratch.
+// bt: a (L), aux (V), aux2 (W).
+int64_t inverse_pairs_edge(int64_t n);
+void launch_factor_inverse(const double *L, int64_t ldl, int64_t n, double *V, double *W, hipStream_t st,
+                           const Batch &bt);
+// G <- g/2 (a a^T - X^T X), full, X = the inverse in V.  bt: aux (V), b (a), g (G); one g a system.
+void launch_gp_gradient(const double *V, int64_t n, const double *a, const double *g, double *G, int64_t ldg,
+                        hipStream_t st, const Batch &bt);
 // Solve: forward then backward sweep in place on B (one persistent launch each, each after a
 // small reset launch).  tickets: 2 ints; Ypk: solve_pack_doubles(n, nrhs) doubles of scratch
 // (each finished block's packed copy for its consumers), used by the two sweeps in turn: each

@@ -119,7 +119,7 @@ __device__ __forceinline__ void leaf_inverse_steps(const double (&v)[16], double
     }
 }
 
-// Workgroup b: X_b^T = L_bb^{-T} to Wout + b*kInvDoubles (ld 128) and X_b at + kInvX.
+// Workgroup b: X_b^T = L_bb^{-T} to Wt + b sBlk and X_b to Wx + b sBlk (ld ldw).
 // A triangular inverse by a tree over the diagonal 16 x 16 leaves (the recursive form of
 // LAPACK's dtrtri): from the 8 leaf inverses X_pp, three levels double the inverted diagonal
 // blocks, X_BA = -X_BB (L_BA X_AA) for [A; B] of 16 + 16, 32 + 32 and 64 + 64 rows, each level's
@@ -133,14 +133,15 @@ __device__ __forceinline__ void leaf_inverse_steps(const double (&v)[16], double
 // by z times their strides (s*), its info at info + z.
 template <typename T>
 __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict__ L, int64_t ldl, int64_t n,
-                                                            const double *__restrict__ Wleaf,
-                                                            double *__restrict__ Wout, const int *info, int64_t sL,
+                                                            const double *__restrict__ Wleaf, double *Wt, double *Wx,
+                                                            int64_t ldw, int64_t sBlk, const int *info, int64_t sL,
                                                             int64_t sWl, int64_t sWo)
 {
     __shared__ double S[36 * kTile];  // the packed lower tiles
     const int64_t z = blockIdx.z;
     L += z * sL;
-    Wout += z * sWo;
+    Wt += z * sWo;
+    Wx += z * sWo;
     if (info) info += z;
     if (factor_failed(info)) return;
     const int b = (int)blockIdx.x;
@@ -198,8 +199,9 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict_
     inverse_level<2>(S, w);
     inverse_level<4>(S, w);
 
-    // X to Wout + kInvX and X^T to Wout (ld 128), zeros above the diagonal; two elements a store
-    double *Wt = Wout + (size_t)b * kInvDoubles, *Wx = Wt + kInvX;
+    // X and X^T, zeros above and below the diagonal; two elements a store (ldw and sBlk are even)
+    Wt += b * sBlk;
+    Wx += b * sBlk;
 #pragma unroll 8
     for (int e = tid; e < 128 * 64; e += 256) {
         const int f = 2 * (e & 63), c = e >> 6;  // elements (f, c), (f + 1, c) of X and of X^T
@@ -212,8 +214,8 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict_
             const double *t = S + tile_at(c >> 4, f >> 4) + (c & 15) + kTileLd * (f & 15);
             xt = dvec2{t[0], t[kTileLd]};
         }
-        *(dvec2 *)(Wx + f + 128 * c) = x;
-        *(dvec2 *)(Wt + f + 128 * c) = xt;
+        *(dvec2 *)(Wx + f + ldw * c) = x;
+        *(dvec2 *)(Wt + f + ldw * c) = xt;
     }
 }
 
@@ -289,10 +291,18 @@ void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wle
 {
     const unsigned nblk = (unsigned)((n + 127) / 128);
     hipLaunchKernelGGL(block_inverse_kernel<T>, dim3(nblk, 1, bt.count), dim3(256), 0, s, L, lda, n, Wleaf, Winv,
-                       info, bt.a, bt.leaf, bt.inv);
+                       Winv + kInvX, (int64_t)128, kInvDoubles, info, bt.a, bt.leaf, bt.inv);
     if (couplings && solve_couplings(nblk) > 0)
         hipLaunchKernelGGL(block_coupling_kernel<T>, dim3(2 * solve_couplings(nblk) * nblk, 1, bt.count), dim3(256), 0,
                            s, L, lda, n, Winv, info, bt.a, bt.inv);
+}
+
+void launch_block_inverses_to(const double *L, int64_t lda, int64_t n, double *Wt, double *Wx, int64_t ldw,
+                              int64_t stride, hipStream_t s, unsigned count, int64_t sL, int64_t sW)
+{
+    const unsigned nblk = (unsigned)((n + 127) / 128);
+    hipLaunchKernelGGL(block_inverse_kernel<double>, dim3(nblk, 1, count), dim3(256), 0, s, L, lda, n,
+                       (const double *)nullptr, Wt, Wx, ldw, stride, (const int *)nullptr, sL, (int64_t)0, sW);
 }
 
 template void launch_block_inverses<double>(const double *, int64_t, int64_t, const double *, double *, const int *,

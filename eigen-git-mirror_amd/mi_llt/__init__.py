@@ -96,6 +96,7 @@ def lib() -> ctypes.CDLL:
                                              _VP]
         L.mi_dposv_adjoint_batched.argtypes = [_VP, ctypes.c_char, _I64, _I64, _I64, _VP, _I64, _I64, _VP, _I64,
                                                _I64, _VP, _I64, _I64, _VP, _I64, _I64]
+        L.mi_dgp_gradient_batched.argtypes = [_VP, _I64, _I64, _VP, _I64, _I64, _VP, _I64, _VP, _VP, _I64, _I64]
         L.LAPACKE_spotrf.argtypes = [_INT, ctypes.c_char, _INT, _VP, _INT]
         L.LAPACKE_spotrs.argtypes = [_INT, ctypes.c_char, _INT, _INT, _VP, _INT, _VP, _INT]
         _PI = ctypes.POINTER(_INT)
@@ -122,7 +123,7 @@ def lib() -> ctypes.CDLL:
                      "mi_spotrf_async", "mi_spotrs", "mi_dtrsm", "mi_dsyrk", "mi_dpocon", "mi_dllt_rank_update",
                      "LAPACKE_spotrf", "LAPACKE_spotrs", "mi_dpotrf_batched_async", "mi_dpotrs_batched",
                      "mi_dpotrf_adjoint_batched", "mi_dpotrs_adjoint_batched", "mi_dposv_noalloc",
-                     "mi_dposv_batched_async", "mi_dposv_adjoint_batched"):
+                     "mi_dposv_batched_async", "mi_dposv_adjoint_batched", "mi_dgp_gradient_batched"):
             getattr(L, name).restype = _INT
         L.dpotrf_.restype = None
         L.dpotrs_.restype = None

@@ -9,12 +9,12 @@ symmetric input is returned as a full symmetric matrix.
 * :class:`CholeskySolve` (B, L) -> X = (L L^T)^{-1} B, backward = mi_dpotrs_adjoint
 * :class:`CholeskyBatched`, :class:`CholeskySolveBatched`: the same for a (batch, n, n) stack
   of systems of one order, through the batched entry points (every kernel launch covers the
-  whole batch); :class:`GPLogMarginalBatched` / :func:`gp_log_marginal_batched` the fused
-  log marginal likelihood of a batch (mi_dposv_batched_async forward, mi_dposv_adjoint_batched
-  backward)
-* :func:`gp_log_marginal` the Gaussian-process log marginal likelihood
-  -1/2 y^T K^{-1} y - sum log L_ii - n/2 log(2 pi), whose gradient is 1/2 (a a^T - K^{-1}),
-  a = K^{-1} y.
+  whole batch)
+* :class:`GPLogMarginal` / :func:`gp_log_marginal`, :class:`GPLogMarginalBatched` /
+  :func:`gp_log_marginal_batched` the Gaussian-process log marginal likelihood
+  -1/2 y^T K^{-1} y - sum log L_ii - n/2 log(2 pi) of one system or a batch, fused: factor and
+  solve forward; its gradient 1/2 (a a^T - K^{-1}), a = K^{-1} y, backward by
+  mi_dgp_gradient_batched, which forms K^{-1} from the factor.
 All tensors are float64 on the GPU; inputs are copied to column-major storage.
 """
 from __future__ import annotations
@@ -23,8 +23,8 @@ import math
 
 import torch
 
-from . import (_VP, _batched_ld, _ld, colmajor, colmajor_batched, default_handle, lib, posv_batched_async_, potrf_,
-               potrf_batched_async_, potrs_, potrs_batched_)
+from . import (_VP, _batched_ld, _ld, colmajor, colmajor_batched, default_handle, lib, posv_async_,
+               posv_batched_async_, potrf_, potrf_batched_async_, potrs_, potrs_batched_)
 
 
 def _cm(t: torch.Tensor) -> torch.Tensor:
@@ -88,12 +88,58 @@ def cholesky_solve(b: torch.Tensor, l: torch.Tensor) -> torch.Tensor:
     return CholeskySolve.apply(b, l)
 
 
+def _row_major(k: torch.Tensor) -> bool:
+    return k.stride(-1) == 1 and k.stride(-2) != 1
+
+
+def _gp_gradient(l: torch.Tensor, a: torch.Tensor, g: torch.Tensor, row_major: bool) -> torch.Tensor:
+    """g_z/2 (a_z a_z^T - (L_z L_z^T)^{-1}) for column-major l (batch, n, n), a (batch, n, 1) and g
+    (batch,).  It is symmetric, so it comes in the strides of a row- or column-major K without a
+    copy (autograd would copy a gradient into its input's strides)."""
+    b, n = int(l.shape[0]), int(l.shape[1])
+    g = g.to(torch.float64).contiguous()
+    out = torch.empty_strided((b, n, n), (n * n, 1, max(n, 1)), dtype=torch.float64, device=l.device)
+    h = default_handle()
+    ldl, sl = _batched_ld(l)
+    ldo, so = _batched_ld(out)
+    h.check(lib().mi_dgp_gradient_batched(h.ptr, n, b, _VP(l.data_ptr()), ldl, sl, _VP(a.data_ptr()),
+                                          _batched_ld(a)[1], _VP(g.data_ptr()), _VP(out.data_ptr()), ldo, so),
+            "mi_dgp_gradient_batched")
+    return out.transpose(1, 2) if row_major else out
+
+
+class GPLogMarginal(torch.autograd.Function):
+    """(K, y) -> log N(y | 0, K); dK = g/2 (a a^T - K^{-1}), dy = -g a, a = K^{-1} y."""
+
+    @staticmethod
+    def forward(ctx, k: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
+        l = _cm(k)  # the lower triangle becomes L
+        a = _cm(y.reshape(y.shape[0], -1))
+        d_info = torch.zeros(1, dtype=torch.int32, device=l.device)
+        posv_async_(l, a, d_info)
+        info = int(d_info.item())
+        if info != 0:
+            raise torch.linalg.LinAlgError(f"Cholesky: the leading minor of order {info} is not positive definite")
+        ctx.save_for_backward(l, a)
+        ctx.row_major = _row_major(k)
+        return (-0.5 * torch.dot(y, a.reshape(-1) if y.dim() == 1 else a) - torch.log(torch.diagonal(l)).sum()
+                - 0.5 * k.shape[0] * math.log(2.0 * math.pi))
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g: torch.Tensor):
+        l, a = ctx.saved_tensors
+        dk = dy = None
+        if ctx.needs_input_grad[0]:
+            dk = _gp_gradient(l.unsqueeze(0), a.unsqueeze(0), g.reshape(1), ctx.row_major)[0]
+        if ctx.needs_input_grad[1]:
+            dy = -g * a.reshape(-1)
+        return dk, dy
+
+
 def gp_log_marginal(k: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
-    """log N(y | 0, K) through the library's factorization and solve (differentiable in K)."""
-    n = k.shape[0]
-    l = cholesky(k)
-    alpha = cholesky_solve(y, l)
-    return -0.5 * torch.dot(y, alpha) - torch.log(torch.diagonal(l)).sum() - 0.5 * n * math.log(2.0 * math.pi)
+    """log N(y | 0, K) through the library's factorization and solve (differentiable in K and y)."""
+    return GPLogMarginal.apply(k, y)
 
 
 class CholeskyBatched(torch.autograd.Function):
@@ -166,9 +212,8 @@ def cholesky_solve_batched(b: torch.Tensor, l: torch.Tensor) -> torch.Tensor:
 
 class GPLogMarginalBatched(torch.autograd.Function):
     """(K (batch, n, n), y (batch, n)) -> log N(y_z | 0, K_z) per system, fused: the forward is
-    one factor + solve per system (mi_dposv_batched_async: L and a = K^{-1} y), the backward one
-    call of mi_dposv_adjoint_batched with the gradients the log-likelihood sends into a and L
-    (abar = -g/2 y, Lbar = -g diag(1/L_ii)), which returns dL/dK = g/2 (a a^T - K^{-1})."""
+    one factor + solve per system (mi_dposv_batched_async: L and a = K^{-1} y), the backward
+    dK_z = g_z/2 (a_z a_z^T - K_z^{-1}) (mi_dgp_gradient_batched)."""
 
     @staticmethod
     def forward(ctx, k: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
@@ -184,30 +229,18 @@ class GPLogMarginalBatched(torch.autograd.Function):
                                            "positive definite")
         d = torch.diagonal(l, dim1=-2, dim2=-1)
         ya = a.squeeze(-1)
-        ctx.save_for_backward(l, a, y.detach().to(torch.float64))
+        ctx.save_for_backward(l, a)
+        ctx.row_major = _row_major(k)
         return -0.5 * (y.detach() * ya).sum(-1) - torch.log(d).sum(-1) - 0.5 * n * math.log(2.0 * math.pi)
 
     @staticmethod
     def backward(ctx, g: torch.Tensor):
-        l, a, y = ctx.saved_tensors
-        b, n = int(l.shape[0]), int(l.shape[1])
-        g = g.to(torch.float64)
-        xbar = colmajor_batched((-0.5 * g)[:, None] * y)
-        lbar = torch.zeros_like(l)  # same (column-major) strides as l
-        torch.diagonal(lbar, dim1=-2, dim2=-1).copy_(-g[:, None] / torch.diagonal(l, dim1=-2, dim2=-1))
-        h = default_handle()
-        ldl, sl = _batched_ld(l)
-        ldx, sx = _batched_ld(a)
-        ldb, sb = _batched_ld(xbar)
-        ldlb, slb = _batched_ld(lbar)
-        h.check(lib().mi_dposv_adjoint_batched(h.ptr, b"L", n, 1, b, _VP(l.data_ptr()), ldl, sl, _VP(a.data_ptr()), ldx,
-                                               sx, _VP(xbar.data_ptr()), ldb, sb, _VP(lbar.data_ptr()), ldlb, slb),
-                "mi_dposv_adjoint_batched")
-        return lbar, None
+        l, a = ctx.saved_tensors
+        return _gp_gradient(l, a, g, ctx.row_major), None
 
 
 def gp_log_marginal_batched(k: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
     """log N(y_z | 0, K_z) for a (batch, n, n) stack K and (batch, n) targets y: a (batch,)
-    tensor, differentiable in K (one batched factor + solve forward, one batched adjoint
+    tensor, differentiable in K (one batched factor + solve forward, one batched inverse
     backward)."""
     return GPLogMarginalBatched.apply(k, y)

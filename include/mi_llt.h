@@ -291,6 +291,15 @@ int mi_dposv_adjoint_batched(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs
                              int64_t ldl, int64_t strideL, const double *dX, int64_t ldx, int64_t strideX,
                              double *dXbar, int64_t ldxb, int64_t strideXbar, double *dLbar, int64_t ldlb,
                              int64_t strideLbar);
+/* mi_dgp_gradient_batched: per system the gradient of log N(y | 0, A) = -1/2 y^T A^{-1} y
+ *   - sum log L_ii - n/2 log(2 pi) with respect to A, times dG[z]: dK_z <- dG[z]/2 (a a^T - A^{-1}),
+ *   full symmetric, with L_z as left by mi_dpotrf(_batched_async) (lower) in dL and a = A^{-1} y in
+ *   dAlpha (n doubles a system, strideAlpha apart); dG: `batch` doubles on the device.  Asynchronous.
+ *   Workspace per system: np (np + 128) doubles and a quarter to all of np^2 (np = n rounded up to
+ *   128s). */
+int mi_dgp_gradient_batched(mi_llt_handle h, int64_t n, int64_t batch, const double *dL, int64_t ldl, int64_t strideL,
+                            const double *dAlpha, int64_t strideAlpha, const double *dG, double *dK, int64_t ldk,
+                            int64_t strideK);
 
 #ifdef __cplusplus
 }

@@ -174,6 +174,34 @@ def test_batched_gp_gradient_closed_form_and_single(dev):
         assert dif <= 1e-13, f"system {z}: batched gradient differs from the single path by {dif}"
 
 
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 128, 129, 191, 200, 257, 385, 513, 641])
+@pytest.mark.parametrize("row_major", [False, True])
+def test_gp_gradient_inverse_tree(dev, n, row_major):
+    """Around the 64 x 64 tiles, the 128-row blocks and the levels of the inverse's tree (the last
+    pair's second half shorter, rows beyond n), each gradient in K's own strides, against FP64 on the
+    CPU: |d A^{-1}| <= 8 n u kappa |A^{-1}| for kappa <= 45 (gram_spd: spectrum in [0.1, 4.2])."""
+    say(f"[gpu] GP gradient tree n={n} row_major={row_major}")
+    batch = 3
+    ks = torch.stack([torch.from_numpy(workloads.gram_spd(n, seed=40 * n + z)) for z in range(batch)])
+    ys = torch.from_numpy(np.random.default_rng(n).standard_normal((batch, n)))
+    g = torch.tensor([1.0, -0.5, 3.0], dtype=torch.float64)
+    inv = torch.stack([torch.linalg.inv(k) for k in ks])
+    al = torch.stack([inv[z] @ ys[z] for z in range(batch)])
+    ref = 0.5 * g[:, None, None] * (al[:, :, None] * al[:, None, :] - inv)
+    tol = 8 * (n + 8) * 45 * 2.0 ** -53
+    kd = ks.to(dev)
+    kd = (kd.contiguous() if row_major else mi_llt.colmajor_batched(kd)).requires_grad_(True)
+    (mad.gp_log_marginal_batched(kd, ys.to(dev)) * g.to(dev)).sum().backward()
+    assert torch.equal(kd.grad, kd.grad.transpose(1, 2))
+    for z in range(batch):
+        assert float((kd.grad[z].cpu() - ref[z]).abs().max()) <= tol * float(ref[z].abs().max()), z
+    k1 = kd.detach()[1].clone().requires_grad_(True)
+    y1 = ys[1].to(dev).requires_grad_(True)
+    (mad.gp_log_marginal(k1, y1) * g[1].to(dev)).backward()
+    assert torch.equal(k1.grad, kd.grad[1])
+    assert float((y1.grad.cpu() + g[1] * al[1]).abs().max()) <= tol * float(al[1].abs().max())
+
+
 def test_batched_argument_errors(dev):
     h = mi_llt.default_handle()
     L = mi_llt.lib()
