@@ -27,10 +27,14 @@
 // storage a launch's update is MFMA work, and the deeper tiles would leave the last round of
 // each launch emptier: the FP64 factorization keeps the two-panel alternation.
 //
-// Workgroups take roles from a ticket counter, in the order: the diagonal role of the panel
-// (the critical path, always running before anyone waits for it), the trailing-update tiles,
-// then the panel's row roles -- which wait for the diagonal block, so they should not hold
-// CUs while it is being factored.
+// Workgroup 0 and those past the tiles are the panel's: they take its roles from a ticket counter,
+// the first to start the diagonal role (the critical path, always running before anyone waits for
+// it), the others the row roles -- which wait for the diagonal block, so they come last in the
+// grid and do not hold CUs while it is being factored.  The workgroups between are the trailing
+// update's tiles, by their place in the grid: with a ticket for each, the last of the 512 that start
+// together came 9 us late (17.5 ns an atomic on one address), 6282 against 6120 us at n = 8192 and
+// 14.2 against 13.85 ms in the FP32-storage factor at n = 16384.  (Raised wave priorities for the
+// panel's roles, or for the earlier of the two workgroups of a CU, changed nothing.)
 #include "factor_plan.hpp"
 #include "potrf_device.hpp"
 #include "syrk_device.hpp"
@@ -88,33 +92,36 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
         info += z;
     }
     __shared__ int s_role, s_ok, s_stop;
-    // Every workgroup draws its ticket, even when it then stops: the host counts them.  The
-    // failure words (info, status) are read in the same round trip as the ticket, so a
-    // workgroup starts after one memory latency, not three.
-    if (threadIdx.x == 0) {
-        const uint32_t tk = atomicAdd(tickets, 1u);
-        const int iv = __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int sv = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_role = (int)(tk - ticket_base);
-        s_stop = iv | sv;
-    }
-    __syncthreads();
-    if (s_stop) return;
-    const int t = __builtin_amdgcn_readfirstlane(s_role);  // uniform: every derived address is scalar
-    // A role outside this launch means the counter was not reset with the host's accounting
-    // (never in a correct call sequence): record it and touch nothing, rather than turn the
-    // ticket into an address.
-    if (t < 0 || t >= Gp + nsyrk) {
-        if (threadIdx.x == 0) atomicOr(status, MI_FACTOR_TICKET);
-        return;
-    }
-    if (Gp > 0 && (t == 0 || t > nsyrk)) {  // ticket 0: diagonal role; last Gp-1: row roles
+    const int bx = (int)blockIdx.x;
+    if (Gp > 0 && (bx == 0 || bx > nsyrk)) {
+        // The panel's workgroups draw tickets, even those that then stop: the host counts them.  The
+        // failure words (info, status) are read in the same round trip as the ticket, so a
+        // workgroup starts after one memory latency, not three.
+        if (threadIdx.x == 0) {
+            const uint32_t tk = atomicAdd(tickets, 1u);
+            const int iv = __hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int sv = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_role = (int)(tk - ticket_base);
+            s_stop = iv | sv;
+        }
+        __syncthreads();
+        if (s_stop) return;
+        const int t = __builtin_amdgcn_readfirstlane(s_role);  // uniform: every derived address is scalar
+        // A role outside this launch means the counter was not reset with the host's accounting
+        // (never in a correct call sequence): record it and touch nothing, rather than turn the
+        // ticket into an address.
+        if (t < 0 || t >= Gp) {
+            if (threadIdx.x == 0) atomicOr(status, MI_FACTOR_TICKET);
+            return;
+        }
         __bf16 *split = Wsplit ? Wsplit + ((kp / kNB) & (kSplitRing - 1)) * slot_elems : nullptr;
-        panel_role<S, PREC>(t == 0 ? 0 : t - nsyrk, smem, &s_ok, A, lda, n, kp, Wleaf, info, flag, epoch,
-                            status, split, split_part_elems(n));
+        panel_role<S, PREC>(t, smem, &s_ok, A, lda, n, kp, Wleaf, info, flag, epoch, status, split, split_part_elems(n));
         return;
     }
-    const int u = xcd_remap(Gp > 0 ? t - 1 : t, nsyrk);
+    // A tile waits for nothing and depends on nothing in this launch, so it needs no ticket, and the
+    // failure words as earlier launches left them are enough.
+    if (*info | *status) return;
+    const int u = xcd_remap(Gp > 0 ? bx - 1 : bx, nsyrk);
     const int nblk = (int)((n + kNB - 1) / kNB);
     constexpr bool OCT = KQ > 0 && PREC == kPrecBF16x3;
     int i, c;
@@ -283,7 +290,7 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
         slabo = q.slabo;
     }
     const unsigned grid = (unsigned)(Gp + nsyrk);
-    *grid_out = grid;
+    *grid_out = (uint32_t)Gp;  // tickets drawn
     if (grid == 0) return;
     const dim3 g(grid, 1, bt.count);
     const int64_t slot = split_slot_elems(n, prec == kPrecBF16x6 ? 3 : 2);

@@ -43,7 +43,7 @@ struct Batch {
 };
 
 // Synchronisation words of a handle (32-bit words in device memory).  Each group sits on its
-// own 128-byte line: every starting workgroup of a factorization step takes an atomic on the
+// own 128-byte line: the starting panel workgroups of a factorization step take an atomic on the
 // ticket counter and the waiting ones poll the flag, and a read of another word of that line
 // (the status, read by every workgroup as it starts) waits behind those atomics.
 constexpr int kSyncStatus = 0;          // status bits (MI_SOLVE_TIMEOUT, ...)
