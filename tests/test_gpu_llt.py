@@ -74,6 +74,33 @@ def test_row_role_edges(dev, n, pad):
     assert_status_ok()
 
 
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 300, 897, 1025, 2049])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_one_column_solve_edges(dev, n, pad):
+    """One right-hand side (its own product and copies) beside two, at the ends of the couplings' ranges
+    (none below 8 blocks, two below 16, three), leading dimensions of any parity; FP64 by the oracle's
+    bound, FP32 storage by |B - A X| <= 3 (n + 2) u max a_ii |X|."""
+    say(f"[gpu] one-column solve n={n} pad={pad}")
+    a = workloads.gram_spd(n, seed=n + 1)
+    b = workloads.rhs(n, 2, seed=n)
+    for dtype, factor, solve in ((torch.float64, mi_llt.potrf_, mi_llt.potrs_), (torch.float32, mi_llt.spotrf_, mi_llt.spotrs_)):
+        m = torch.full((n, n + pad), 7.0, dtype=dtype, device=dev).t()[:n, :] if pad else \
+            mi_llt.colmajor(torch.zeros(n, n, dtype=dtype, device=dev))
+        m.copy_(torch.from_numpy(a).to(dev))
+        assert factor(m) == 0
+        for cols in ([0], [0, 1]):
+            x = mi_llt.colmajor(torch.from_numpy(b[:, cols].copy()).to(dev).to(dtype))
+            solve(m, x)
+            xs = x.cpu().numpy().astype(np.float64)
+            if dtype == torch.float64:
+                assert oracle.solve_berr(a, xs, b[:, cols]) <= TOL_BERR
+            else:
+                a32, b32 = a.astype(np.float32).astype(np.float64), b[:, cols].astype(np.float32).astype(np.float64)
+                lim = 3 * (n + 2) * 2.0 ** -24 * a32.diagonal().max() * np.abs(xs).sum(0).max()
+                assert np.abs(b32 - a32 @ xs).max() <= lim
+    assert_status_ok()
+
+
 @pytest.mark.parametrize("tag", ["kat3"] + [f"spd{n}" for n in (1, 2, 3, 7, 8, 16, 31, 32, 33, 64, 100, 127,
                                                                 128, 129, 200)])
 def test_factor_solve_matches_eigen_golden(dev, tag):
