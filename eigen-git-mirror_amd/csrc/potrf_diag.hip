@@ -225,12 +225,15 @@ __global__ __launch_bounds__(256) void block_inverse_kernel(const T *__restrict_
 // so everything else is done before they are published (solve_couplings: none below 8 blocks,
 // the third only from 16 blocks on).  Workgroup q nblk + b, distance d = 1 + q / 2: q even, M_b / M2_b / M3_b = X_b L_{b,b-d} (b >= d); q odd, N_b / N2_b / N3_b
 // = X_b^T L_{b+d,b}^T (b + d < nblk).  128 x 128 each at Winv[b] + kInvM / kInvN / kInvM2 /
-// kInvN2 / kInvM3 / kInvN3 (ld 128); entries of L outside the matrix read as 0.  4 waves of
-// 64 x 64 (4 x 4 FP64 MFMA tiles), depth 128.
+// kInvN2 / kInvM3 / kInvN3 (ld 128); entries of L outside the matrix read as 0.
+//
+// Bound by latency: a workgroup takes a 64 x 64 quadrant (blockIdx.y), a wave 32 x 32 of it, so that
+// a few blocks' products still use the chip, and the k outside the triangle of X (whole chunks of 32)
+// is not multiplied.  Two chunks' operands are in flight: 8 k-steps of 4 MFMAs each.
 template <typename T>
-__global__ __launch_bounds__(256) void block_coupling_kernel(const T *__restrict__ L, int64_t ldl, int64_t n,
-                                                             double *__restrict__ Winv, const int *info, int64_t sL,
-                                                             int64_t sWo)
+__global__ __launch_bounds__(256, 2) void block_coupling_kernel(const T *__restrict__ L, int64_t ldl, int64_t n,
+                                                                double *__restrict__ Winv, const int *info, int64_t sL,
+                                                                int64_t sWo)
 {
     const int64_t z = blockIdx.z;
     L += z * sL;
@@ -243,46 +246,63 @@ __global__ __launch_bounds__(256) void block_coupling_kernel(const T *__restrict
     const int d = 1 + q / 2;
     if (fwd ? b < d : b + d > nblk - 1) return;
     double *Wb = Winv + (size_t)b * kInvDoubles;
-    const double *P = Wb + (fwd ? kInvX : 0);  // P[i][k] = X_b[i][k] or X_b^T[i][k] at P + i + 128 k
+    const int l = lane_id(), kl = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i0 = 64 * ((int)blockIdx.y >> 1) + 32 * (w >> 1), j0 = 64 * ((int)blockIdx.y & 1) + 32 * (w & 1);
+    // P[i][k] = X_b[i][k] (forward; 0 for k > i) or X_b^T[i][k] (0 for k < i) at P + i + 128 k;
     // Q[j][k] = L[128 b + k][128 (b-d) + j] (forward; rows k < lim exist) or
     //           L[128 (b+d) + j][128 b + k] (backward; rows j < lim exist)
+    const double *P = Wb + (fwd ? kInvX : 0) + i0 + (l & 15) + 128 * kl;
     const int64_t r0 = fwd ? 128 * (int64_t)b : 128 * (int64_t)(b + d);
     const int64_t c0 = fwd ? 128 * (int64_t)(b - d) : 128 * (int64_t)b;
     const int lim = (int)((n - r0) < 128 ? (n - r0) : 128);
-    const int l = lane_id(), w = threadIdx.x >> 6, wr = w >> 1, wc = w & 1, kl = l >> 4;
-    dvec4 acc[4][4];
+    const int clo = fwd ? 0 : i0 / 32, chi = fwd ? i0 / 32 + 1 : 4;  // chunks of the triangle
+    double pv[2][8][2];
+    T qv[2][8][2];
+    bool in[2][8][2];
+    auto load = [&](int u, int c) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+        for (int s = 0; s < 8; ++s) {
+            const int k = 32 * c + 4 * s;  // + kl
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[a][q] = dvec4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 2
-    for (int s = 0; s < 32; ++s) {
-        const int k = 4 * s + kl;
-        double pv[4], qv[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) pv[a] = P[64 * wr + 16 * a + (l & 15) + 128 * k];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int j = 64 * wc + 16 * q + (l & 15);
-            const int rr = fwd ? k : j;  // the row of L read, relative to r0
-            const bool in = rr < lim;
-            const int64_t off = fwd ? (r0 + (in ? k : 0)) + (c0 + j) * ldl : (r0 + (in ? j : 0)) + (c0 + k) * ldl;
-            const double v = (double)L[off];
-            qv[q] = in ? v : 0.0;
+            for (int a = 0; a < 2; ++a) {
+                pv[u][s][a] = P[16 * a + 128 * k];
+                const int j = j0 + 16 * a + (l & 15);
+                in[u][s][a] = (fwd ? k + kl : j) < lim;
+                const bool i = in[u][s][a];
+                qv[u][s][a] = L[fwd ? (r0 + (i ? k + kl : 0)) + (c0 + j) * ldl : (r0 + (i ? j : 0)) + (c0 + k + kl) * ldl];
+            }
         }
+    };
+    dvec4 acc[2][2];
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) acc[a][q] = mfma_f64(qv[q], pv[a], acc[a][q]);
+        for (int e = 0; e < 2; ++e) acc[a][e] = dvec4{0.0, 0.0, 0.0, 0.0};
+    load(0, 0);
+    load(1, 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (c >= clo && c < chi) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const double qe = in[c & 1][s][e] ? (double)qv[c & 1][s][e] : 0.0;
+#pragma unroll
+                    for (int a = 0; a < 2; ++a) acc[a][e] = mfma_f64(qe, pv[c & 1][s][a], acc[a][e]);
+                }
+        }
+        if (c < 2) load(c & 1, c + 2);
     }
     double *C = Wb + (fwd ? (d == 1 ? kInvM : d == 2 ? kInvM2 : kInvM3) : (d == 1 ? kInvN : d == 2 ? kInvN2 : kInvN3));
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                C[(64 * wr + 16 * a + (l & 15)) + 128 * (64 * wc + 16 * q + 4 * r + kl)] = acc[a][q][r];
+                C[(i0 + 16 * a + (l & 15)) + 128 * (j0 + 16 * e + 4 * r + kl)] = acc[a][e][r];
 }
 
 template <typename T>
@@ -293,7 +313,7 @@ void launch_block_inverses(const T *L, int64_t lda, int64_t n, const double *Wle
     hipLaunchKernelGGL(block_inverse_kernel<T>, dim3(nblk, 1, bt.count), dim3(256), 0, s, L, lda, n, Wleaf, Winv,
                        Winv + kInvX, (int64_t)128, kInvDoubles, info, bt.a, bt.leaf, bt.inv);
     if (couplings && solve_couplings(nblk) > 0)
-        hipLaunchKernelGGL(block_coupling_kernel<T>, dim3(2 * solve_couplings(nblk) * nblk, 1, bt.count), dim3(256), 0,
+        hipLaunchKernelGGL(block_coupling_kernel<T>, dim3(2 * solve_couplings(nblk) * nblk, 4, bt.count), dim3(256), 0,
                            s, L, lda, n, Winv, info, bt.a, bt.inv);
 }
 
