@@ -42,13 +42,13 @@ __device__ __forceinline__ double readlane_d(double x, int lane)
 // up to 112 rows below the leaf (row c0+16+64w+l), for which they are the panel solve A_ip
 // L_pp^{-T}, and in the last 16 lanes of wave 1 (never a row below) the rows of the 16 x 16
 // identity, which become L_pp^{-T}, i.e. column i of X_pp = L_pp^{-1} in lane 48+i, written to xleaf
-// column-major.  (With readlane broadcasts and the leaf in lanes 0..15, three waves took a panel in
+// (LDS) column-major.  (With readlane broadcasts and the leaf in lanes 0..15, three waves took a panel in
 // 4300 cycles; this form takes 2900, and two waves are left for the deferred updates.)
 //
 // Returns the failing panel column or -1, the same in both waves.  The factored leaf is left in u:
 // it is written back to S only after a barrier, since the other wave reads the unfactored leaf from
 // S here and may still be doing so when one wave is done.
-__device__ __forceinline__ int panel_factor2(double *S, int c0, double *__restrict__ xleaf, double (&u)[16])
+__device__ __forceinline__ int panel_factor2(double *S, int c0, double *xleaf, double (&u)[16])
 {
     const int l = lane_id(), w = threadIdx.x >> 6;
     const int rb = c0 + 16 + 64 * w + l;
@@ -127,26 +127,38 @@ __device__ __forceinline__ void lds_tile_update(double *C, const double (&Pi)[4]
     for (int r = 0; r < 4; ++r) C[64 * r] = old[r] - acc[r];
 }
 
+// Image stores reach memory by themselves (agent-scope stores are written through), so publishing
+// them takes the wait for them and the flag's store, no L2 writeback.
+__device__ __forceinline__ void image_store(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The panel flag of the launch with epoch e goes from 4 (e - 1) to 4 e: + 1 by each of two waves once
+// the image's block columns below kEarlyPanels are in memory, 4 e when all of it is.
+constexpr int kEarlyPanels = 4;
+
 // Cholesky of the 128 x 128 lower block in S (all 256 threads), in eight 16-column panels with
 // a one-panel lookahead inside the block.  After panel p is factored, with T = 7-p tile rows
-// below it and their operands P_x (tile (p+1+x, p), x < T) in every wave's registers:
+// below it and their operands P_x = tile (p+1+x, p), x < T:
 //   A(p): the leaf of p goes back to S; the T tiles of column p+1 get panel p's update (the
 //         waves round-robin), barrier;
-//   B(p): waves 0 and 1 factor panel p+1 (panel_factor2: VALU) while waves 2 and 3 apply panel p
-//         to the tiles right of column p+1 on the matrix core (21 tiles at most), barrier.
+//   B(p): waves 0 and 1 factor panel p+1 (panel_factor2: VALU) while waves 2 and 3 store panel p
+//         (its tiles and its leaf's inverse) to the panel image W and apply it to the tiles right of
+//         column p+1 on the matrix core (21 tiles at most), barrier.
 // Column p+1 thus has every earlier panel's update before its factor, the tiles beyond it get
 // panel p's before phase A(p+1) touches them, and the rank-16 updates mostly run under the
-// column loop.  Returns the first failing column or -1 (uniform); writes the 8 leaf inverses
-// to Xl and the strictly lower tiles to the panel image W (sls order), each panel's from the operands
-// in the registers of phase A, so that only the stores' end is left to wait for when the block is done.
-// s_fail: an LDS int.
-__device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, int *s_fail, double *__restrict__ W)
+// column loop.  The panels below kEarlyPanels are published in B(kEarlyPanels), a panel's time after
+// their last store, so that the rows waiting for the block solve their part by them meanwhile.
+// Returns the first failing column or -1 (uniform).  xs: 2 x 256 doubles of LDS, s_fail: an LDS int.
+__device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, double *__restrict__ W, uint32_t *flag)
 {
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id();
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane_id();
+    double *Xl = W + kLeafOffset;
     double lv[16];
     __syncthreads();
     if (w < 2) {
-        const int f = panel_factor2(S, 0, Xl, lv);
+        const int f = panel_factor2(S, 0, xs, lv);
         if (w == 0 && l == 0) *s_fail = f;
     }
     __syncthreads();
@@ -157,37 +169,42 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
     for (int p = 0; p < 7; ++p) {
         const int T = 7 - p;
         const int tb = p + 1;  // first trailing tile row / column
+        auto operand = [&](int x, double (&P)[4]) {
+            const double *src = S + 256 * (((tb + x) * (tb + x + 1)) / 2 + p) + l;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) P[s] = src[64 * s];
+        };
         // ---- A(p)
+        {
+            double P0[4], Pw[2][4];
+            operand(0, P0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (w + 4 * h < T) operand(w + 4 * h, Pw[h]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int x = w + 4 * h;
+                if (x < T) lds_tile_update(S + 256 * (((tb + x) * (tb + x + 1)) / 2 + tb) + l, Pw[h], P0);
+            }
+        }
         if (w == 0 && l < 16) {  // the leaf of p: read by nobody until the final copy out
 #pragma unroll
             for (int c = 0; c < 16; ++c) S[sl(16 * p + l, 16 * p + c)] = lv[c];
         }
-        double P[7][4];
-#pragma unroll
-        for (int x = 0; x < 7; ++x) {
-            if (x < T) {
-                const double *src = S + 256 * (((tb + x) * (tb + x + 1)) / 2 + p) + l;
-#pragma unroll
-                for (int s = 0; s < 4; ++s) P[x][s] = src[64 * s];
-            }
-        }
-        // the panel's tiles to the image
-#pragma unroll
-        for (int x = 0; x < 7; ++x)
-            if (x < T && (x & 3) == w) {
-                double *dst = W + 256 * (((tb + x) * (tb + x - 1)) / 2 + p) + l;
-#pragma unroll
-                for (int s = 0; s < 4; ++s) dst[64 * s] = P[x][s];
-            }
-#pragma unroll
-        for (int x = 0; x < 7; ++x)
-            if (x < T && (x & 3) == w) lds_tile_update(S + 256 * (((tb + x) * (tb + x + 1)) / 2 + tb) + l, P[x], P[0]);
         __syncthreads();
         // ---- B(p)
         if (w < 2) {
-            const int f = panel_factor2(S, 16 * tb, Xl + 256 * tb, lv);
+            const int f = panel_factor2(S, 16 * tb, xs + 256 * (tb & 1), lv);
             if (w == 0 && l == 0) *s_fail = f;
         } else {
+            if (p == kEarlyPanels) {  // this wave's stores of the panels before p
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                if (l == 0) __hip_atomic_fetch_add(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            double P[7][4];
+#pragma unroll
+            for (int x = 0; x < 7; ++x)
+                if (x < T) operand(x, P[x]);
 #pragma unroll
             for (int ti = 1; ti < 7; ++ti) {
 #pragma unroll
@@ -197,11 +214,24 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *__restrict__ Xl, 
                         lds_tile_update(S + 256 * (((tb + ti) * (tb + ti + 1)) / 2 + tb + tj) + l, P[ti], P[tj]);
                 }
             }
+#pragma unroll
+            for (int x = 0; x < 7; ++x)
+                if (x < T && w == 2 + (x & 1)) {
+                    double *dst = W + 256 * (((tb + x) * (tb + x - 1)) / 2 + p) + l;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) image_store(dst + 64 * s, P[x][s]);
+                }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int e = (tid & 127) + 128 * s;
+                image_store(Xl + 256 * p + e, xs[256 * (p & 1) + e]);
+            }
         }
         __syncthreads();
         const int f = __builtin_amdgcn_readfirstlane(*s_fail);
         if (f >= 0) return 16 * tb + f;
     }
+    image_store(Xl + 256 * 7 + tid, xs[256 + tid]);
     if (w == 0 && l < 16) {  // the last leaf
 #pragma unroll
         for (int c = 0; c < 16; ++c) S[sl(112 + l, 112 + c)] = lv[c];
@@ -224,78 +254,130 @@ constexpr int kRowTiles = 1;
 // 8 leaf inverses (Xs, 256 doubles each, column-major): the panel image of kernels.hpp.
 //
 // X <- X L^{-T} in place, strip by strip (TriangularSolverMatrix.h:186-329, blocked by 16):
-//   X_p <- (X_p - sum_{q<p} X_q L_pq^T) X_pp^T,   X_pp = L_pp^{-1}
+//   X_q <- X_q X_qq^T, then X_p <- X_p - X_q L_pq^T for the strips p > q,   X_qq = L_qq^{-1}
 // with the accumulator of a solved strip used directly as the operand of the next ones (its
-// layout is that of an MFMA P operand with k = 4s + lane/16).
-template <int RT>
+// layout is that of an MFMA P operand with k = 4s + lane/16).  Strips Q0 .. Q1-1 here.
+template <int Q0, int Q1, int RT>
 __device__ __forceinline__ void trsm_in_registers(const double *smem, dvec4 (&X)[RT][8])
 {
     const int l = lane_id();
     const double *Ls = smem;
     const double *Xs = smem + kLeafOffset;
 #pragma unroll
-    for (int p = 0; p < 8; ++p) {
-#pragma unroll
-        for (int q = 0; q < p; ++q) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const double lv = Ls[256 * ((p * (p - 1)) / 2 + q) + l + 64 * s];  // L[16p + l%16][16q + 4s + l/16]
-#pragma unroll
-                for (int t = 0; t < RT; ++t) X[t][p] = mfma_f64(-lv, X[t][q][s], X[t][p]);
-            }
-        }
+    for (int q = Q0; q < Q1; ++q) {
         dvec4 z[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t) z[t] = dvec4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const double xv = Xs[256 * p + l + 64 * s];  // X_pp[l%16][4s + l/16]
+            const double xv = Xs[256 * q + l + 64 * s];  // X_qq[l%16][4s + l/16]
 #pragma unroll
-            for (int t = 0; t < RT; ++t) z[t] = mfma_f64(xv, X[t][p][s], z[t]);
+            for (int t = 0; t < RT; ++t) z[t] = mfma_f64(xv, X[t][q][s], z[t]);
         }
 #pragma unroll
-        for (int t = 0; t < RT; ++t) X[t][p] = z[t];
+        for (int t = 0; t < RT; ++t) X[t][q] = z[t];
+#pragma unroll
+        for (int p = q + 1; p < 8; ++p) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const double lv = Ls[256 * ((p * (p - 1)) / 2 + q) + l + 64 * s];  // L[16p + l%16][16q + 4s + l/16]
+#pragma unroll
+                for (int t = 0; t < RT; ++t) X[t][p] = mfma_f64(-lv, z[t][s], X[t][p]);
+            }
+        }
     }
 }
 
-// L (128 x 128 lower, ld ldl, valid order bs, identity beyond; T = float widens) and the leaf
-// inverses Xl -> the panel image in LDS.
-template <typename T>
-__device__ __forceinline__ void stage_factor_image(double *smem, const T *__restrict__ L, int64_t ldl, int bs,
-                                                   const double *__restrict__ Xl)
-{
-    for (int e = threadIdx.x; e < 128 * 128; e += 256) {  // strictly lower tiles of L
-        const int r = e & 127, c = e >> 7;
-        if ((r >> 4) > (c >> 4)) {
-            const bool in = r < bs && c < bs;
-            const double v = (double)L[(in ? r : 0) + (int64_t)(in ? c : 0) * ldl];
-            smem[sls(r, c)] = in ? v : 0.0;
-        }
-    }
-    for (int e = threadIdx.x; e < 8 * 256; e += 256) smem[kLeafOffset + e] = Xl[e];
-}
-
-// A published panel image (kPanelDoubles, 16-byte aligned) -> LDS, 16 bytes per load.
+// Block columns Q0 .. Q1-1 of a published panel image (16-byte aligned) -> LDS, two tiles at a time,
+// 16 bytes per load.
+template <int Q0, int Q1>
 __device__ __forceinline__ void stage_panel_image(double *smem, const double *__restrict__ W)
 {
-    const double2 *src = reinterpret_cast<const double2 *>(W);
-    double2 *dst = reinterpret_cast<double2 *>(smem);
+    constexpr int kTiles = 28 + 8;
+    constexpr auto wanted = [](int t) constexpr -> bool {  // tile t of the image: (ti, tj), then the leaves
+        if (t >= 28) return t - 28 >= Q0 && t - 28 < Q1;
+        int ti = 1;
+        while ((ti + 1) * ti / 2 <= t) ++ti;
+        const int tj = t - ti * (ti - 1) / 2;
+        return tj >= Q0 && tj < Q1;
+    };
+    const int half = threadIdx.x >> 7, e = 2 * (threadIdx.x & 127);
+    int first = -1;  // of a pair
 #pragma unroll
-    for (int i = 0; i < (int)(kPanelDoubles / 2 / 256); ++i) dst[threadIdx.x + 256 * i] = src[threadIdx.x + 256 * i];
+    for (int t = 0; t < kTiles; ++t) {
+        if (!wanted(t)) continue;
+        if (first < 0) {
+            first = t;
+        } else {
+            const int o = 256 * (half ? t : first) + e;
+            *(double2 *)(smem + o) = *(const double2 *)(W + o);
+            first = -1;
+        }
+    }
+    if (first >= 0 && half == 0) *(double2 *)(smem + 256 * first + e) = *(const double2 *)(W + 256 * first + e);
 }
 
-// Rows 0..64 kRowTiles - 1 of P (valid m) <- P * L^{-T} with L and its 8 leaf inverses Xl (read from
-// global into the LDS panel image).  Each wave owns 16 kRowTiles rows.  T = float: P and L are read as
-// FP32 and widened, the arithmetic is FP64, the result is rounded back to FP32.  If IMAGE is given, the panel image is copied from there instead of built from
-// L and Xl.  If SPLIT (a split-panel slot) is given (T = float), the rounded rows are also
+// Waits (thread 0) until *flag has reached `want`, then every wave acquires: each invalidates its own
+// view of the caches, so that the loads it issues next see what was published.  Returns the flag's
+// value less `base` (uniform), 0 on a timeout, recorded as MI_PANEL_TIMEOUT.
+__device__ __forceinline__ int wait_panel_flag(int *s_seen, const uint32_t *flag, uint32_t base, int want, int *status)
+{
+    if (threadIdx.x == 0) {
+        uint32_t spins = 0;
+        int seen;
+        while ((seen = (int)(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - base)) < want) {
+            __builtin_amdgcn_s_sleep(2);
+            if (++spins > (1u << 22)) {
+                atomicOr(status, MI_PANEL_TIMEOUT);
+                seen = 0;
+                break;
+            }
+        }
+        *s_seen = seen;
+    }
+    __syncthreads();
+    const int seen = *s_seen;
+    if (seen > 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    return seen;
+}
+
+// The rows' solve, X as in trsm_in_registers: by the panels published early while the others are being
+// factored, if the block is not done yet, then by those.  Returns false if the factor failed or a wait
+// timed out.
+template <int RT>
+__device__ __forceinline__ bool solve_rows(double *smem, int *s_seen, dvec4 (&X)[RT][8], const double *__restrict__ W,
+                                           const uint32_t *flag, uint32_t epoch, const int *info, int *status)
+{
+    const uint32_t base = 4 * (epoch - 1);
+    int seen = wait_panel_flag(s_seen, flag, base, 2, status);
+    if (seen <= 0) return false;
+    if (seen >= 4) {
+        if (factor_failed(info)) return false;
+        stage_panel_image<0, 8>(smem, W);
+        __syncthreads();
+        trsm_in_registers<0, 8>(smem, X);
+        return true;
+    }
+    stage_panel_image<0, kEarlyPanels>(smem, W);
+    __syncthreads();
+    trsm_in_registers<0, kEarlyPanels>(smem, X);
+    if (wait_panel_flag(s_seen, flag, base, 4, status) <= 0 || factor_failed(info)) return false;
+    stage_panel_image<kEarlyPanels, 8>(smem, W);
+    __syncthreads();
+    trsm_in_registers<kEarlyPanels, 8>(smem, X);
+    return true;
+}
+
+// Rows 0..64 kRowTiles - 1 of P (valid m) <- P * L^{-T} by the panel image (solve_rows).  Each wave
+// owns 16 kRowTiles rows.  T = float: P is read as FP32 and widened, the arithmetic is FP64, the result
+// is rounded back to FP32.  If SPLIT (a split-panel slot) is given (T = float), the rounded rows are also
 // written split into split_parts BF16 parts (2 or 3), row i as row split_row0 + i of the slot
 // (split_store_row; part t at split + t * split_lo).
 template <typename T>
-__device__ __forceinline__ void trsm_rows(double *smem, T *__restrict__ P, int64_t ldp, int m,
-                                          const T *__restrict__ L, int64_t ldl, int bs,
-                                          const double *__restrict__ Xl,
-                                          const double *__restrict__ image = nullptr, __bf16 *split = nullptr,
-                                          int64_t split_lo = 0, int64_t split_row0 = 0, int split_parts = 2)
+__device__ __forceinline__ void trsm_rows(double *smem, int *s_seen, T *__restrict__ P, int64_t ldp, int m,
+                                          const double *__restrict__ image, const uint32_t *flag, uint32_t epoch,
+                                          const int *info, int *status, __bf16 *split, int64_t split_lo,
+                                          int64_t split_row0, int split_parts)
 {
     const int l = lane_id(), w = threadIdx.x >> 6;
     const int row0 = 16 * kRowTiles * w;
@@ -312,12 +394,7 @@ __device__ __forceinline__ void trsm_rows(double *smem, T *__restrict__ P, int64
                 X[t][p][r] = (i < m) ? pv : 0.0;
             }
     }
-    if (image)
-        stage_panel_image(smem, image);
-    else
-        stage_factor_image<T>(smem, L, ldl, bs, Xl);
-    __syncthreads();
-    trsm_in_registers(smem, X);
+    if (!solve_rows(smem, s_seen, X, image, flag, epoch, info, status)) return;
 #pragma unroll
     for (int t = 0; t < kRowTiles; ++t) {
         const int i = row0 + 16 * t + (l & 15);
@@ -418,36 +495,12 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
     }
 }
 
-// Waits (thread 0) until *flag >= epoch, then every wave acquires: each invalidates its own
-// view of the caches, so that the loads it issues next see what the flag's release published.
-// Returns false (uniformly) on a timeout, recorded as MI_PANEL_TIMEOUT.
-__device__ __forceinline__ bool wait_panel_flag(int *s_ok, const uint32_t *flag, uint32_t epoch, int *status)
-{
-    if (threadIdx.x == 0) {
-        uint32_t spins = 0;
-        int ok = 1;
-        while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
-            __builtin_amdgcn_s_sleep(2);
-            if (++spins > (1u << 22)) {
-                atomicOr(status, MI_PANEL_TIMEOUT);
-                ok = 0;
-                break;
-            }
-        }
-        *s_ok = ok;
-    }
-    __syncthreads();
-    const bool ok = *s_ok != 0;
-    if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    return ok;
-}
-
 // The panel role of one block step; g is the role from the ticket:
 //   role 0   : C = A_kk - P_0 P_0^T straight into LDS, Cholesky in LDS, the panel image
-//              (L11's strictly lower tiles and the leaf inverses) to the workspace, publish
-//              `flag` = epoch (release), then L11 into A;
-//   role g>0 : the g-th 64 kRowTiles rows below the block: C = A_gk - P_g P_0^T, wait for the flag,
-//              then rows <- rows * L11^{-T} with the published image, stored once.
+//              (L11's strictly lower tiles and the leaf inverses) to the workspace, published by
+//              `flag` in two parts, then L11 into A;
+//   role g>0 : the g-th 64 kRowTiles rows below the block: C = A_gk - P_g P_0^T, then rows <-
+//              rows * L11^{-T} with the published image as it comes, stored once.
 // The diagonal role publishes even on a failing pivot, so that no waiter is left behind;
 // waiters then see `info` and stop.  (LLT.h:350-366: the update of block column k by all
 // earlier panels precedes its unblocked factor and the right-side solve.)
@@ -468,9 +521,9 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
     const int bs = (int)((n - k0) < 128 ? (n - k0) : 128);
     T *Ck = A + R0 + k0 * lda;  // this role's rows of block column k0
     double *Wp = Wleaf + (size_t)(k0 / 128) * kPanelDoubles;  // the panel image
-    double *Xl = Wp + kLeafOffset;
 
     if (g == 0) {
+        __shared__ double xs[2 * 256];  // potrf_in_lds
         if (k0 > 0) {
             if constexpr (sizeof(T) == 8) {
                 const double *P0 = A + k0 + (k0 - 128) * lda;
@@ -486,10 +539,10 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
         } else {
             block_to_lds(smem, Ck, lda, bs);
         }
-        const int f = potrf_in_lds(smem, Xl, s_ok, Wp);  // begins with a barrier
+        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag);  // begins with a barrier
         if (f >= 0 && tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
-        global_barrier();  // every wave's stores of the image have reached L2
-        if (tid == 0) publish_flag(flag, epoch);
+        global_barrier();  // every wave's stores of the image are in memory
+        if (tid == 0) __hip_atomic_store(flag, 4 * epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (f < 0) lds_to_block(smem, Ck, lda, bs);  // read by later launches only
         return;
     }
@@ -505,10 +558,7 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
             t.setup_rows(A + R0 + (k0 - 128) * lda, lda, r2, rows, A + k0 + (k0 - 128) * lda, lda, 0, 128, 128);
             t.template run_fixed<32>();
         }
-        if (!wait_panel_flag(s_ok, flag, epoch, status) || factor_failed(info)) return;
-        stage_panel_image(smem, Wp);
-        __syncthreads();
-        trsm_in_registers(smem, t.acc);
+        if (!solve_rows(smem, s_ok, t.acc, Wp, flag, epoch, info, status)) return;
         const int l = lane_id();
 #pragma unroll
         for (int a = 0; a < kRowTiles; ++a) {
@@ -532,9 +582,8 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
             t.template store<false, false>(Ck, lda, wr * H, wc * 64, rows, 128);
         }
         global_barrier();  // this role's updated rows are in L2 before other waves read them back
-        if (!wait_panel_flag(s_ok, flag, epoch, status) || factor_failed(info)) return;
-        trsm_rows<T>(smem, Ck, lda, rows, (const T *)nullptr, 0, 128, nullptr, Wp, split, split_lo,
-                            R0, PREC == kPrecBF16x6 ? 3 : 2);
+        trsm_rows<T>(smem, s_ok, Ck, lda, rows, Wp, flag, epoch, info, status, split, split_lo, R0,
+                     PREC == kPrecBF16x6 ? 3 : 2);
     }
 }
 
