@@ -27,9 +27,9 @@
 // storage a launch's update is MFMA work, and the deeper tiles would leave the last round of
 // each launch emptier: the FP64 factorization keeps the two-panel alternation.
 //
-// Workgroup 0 and those past the tiles are the panel's: they take its roles from a ticket counter,
-// the first to start the diagonal role (the critical path, always running before anyone waits for
-// it), the others the row roles -- which wait for the diagonal block, so they come last in the
+// The first workgroups and those past the tiles are the panel's: they take its roles from a ticket
+// counter, the first to start the diagonal role (the critical path, always running before anyone waits
+// for it), the next two its helpers (FP64), the others the row roles -- which wait for the diagonal block, so they come last in the
 // grid and do not hold CUs while it is being factored.  The workgroups between are the trailing
 // update's tiles, by their place in the grid: with a ticket for each, the last of the 512 that start
 // together came 9 us late (17.5 ns an atomic on one address), 6282 against 6120 us at n = 8192 and
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
                                                           double *__restrict__ Wleaf, int *info, uint32_t *tickets,
                                                           uint32_t ticket_base, uint32_t *flag, uint32_t epoch,
                                                           int *status, __bf16 *Wsplit, int64_t slot_elems,
-                                                          int64_t sA, int64_t sW, int64_t sSync)
+                                                          int64_t sA, int64_t sW, int64_t sSync, int halves, int nh)
 {
     __shared__ __align__(16) double smem[kSmem];
     {  // batched launches: system z = blockIdx.z (its matrix, panel images, tickets, flag, info)
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
     }
     __shared__ int s_role, s_ok, s_stop;
     const int bx = (int)blockIdx.x;
-    if (Gp > 0 && (bx == 0 || bx > nsyrk)) {
+    if (Gp > 0 && (bx <= nh || bx > nsyrk + nh)) {
         // The panel's workgroups draw tickets, even those that then stop: the host counts them.  The
         // failure words (info, status) are read in the same round trip as the ticket, so a
         // workgroup starts after one memory latency, not three.
@@ -114,14 +114,23 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
             if (threadIdx.x == 0) atomicOr(status, MI_FACTOR_TICKET);
             return;
         }
+        uint32_t *helped = tickets + (kSyncHelped - kSyncFactorTickets);
+        if constexpr (sizeof(S) == 8) {
+            if (t >= 1 && t <= nh) {
+                diag_helper(t - 1, A, lda, n, kp, helped, epoch);
+                return;
+            }
+        }
         __bf16 *split = Wsplit ? Wsplit + ((kp / kNB) & (kSplitRing - 1)) * slot_elems : nullptr;
-        panel_role<S, PREC>(t, smem, &s_ok, A, lda, n, kp, Wleaf, info, flag, epoch, status, split, split_part_elems(n));
+        panel_role<S, PREC>(t == 0 ? 0 : t - nh, nh, smem, &s_ok, A, lda, n, kp, Wleaf, info, flag, helped, epoch, status,
+                            split, split_part_elems(n));
         return;
     }
     // A tile waits for nothing and depends on nothing in this launch, so it needs no ticket, and the
     // failure words as earlier launches left them are enough.
     if (*info | *status) return;
-    const int u = xcd_remap(Gp > 0 ? bx - 1 : bx, nsyrk);
+    const int hu = xcd_remap(Gp > 0 ? bx - 1 - nh : bx, nsyrk);
+    const int u = hu >> halves, half = hu & halves;
     const int nblk = (int)((n + kNB - 1) / kNB);
     constexpr bool OCT = KQ > 0 && PREC == kPrecBF16x3;
     int i, c;
@@ -167,9 +176,16 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
     }
     if constexpr (KQ > 0) {
         if (quad) {
-            syrk_tile<KQ, S, PREC>(A + r + r * lda, lda, A + r + slabq * lda, lda, (int)m, ncol, i - c, 0);
+            if (halves)
+                syrk_tile<KQ, S, PREC, true>(A + r + r * lda, lda, A + r + slabq * lda, lda, (int)m, ncol, i - c, 0, half);
+            else
+                syrk_tile<KQ, S, PREC>(A + r + r * lda, lda, A + r + slabq * lda, lda, (int)m, ncol, i - c, 0);
             return;
         }
+    }
+    if (halves) {
+        syrk_tile<K, S, PREC, true>(A + r + r * lda, lda, A + r + slab * lda, lda, (int)m, ncol, i - c, 0, half);
+        return;
     }
     syrk_tile<K, S, PREC>(A + r + r * lda, lda, A + r + slab * lda, lda, (int)m, ncol, i - c, 0);
 }
@@ -179,6 +195,7 @@ __global__ void factor_reset_kernel(uint32_t *sync, int64_t sSync)
     sync += (int64_t)blockIdx.z * sSync;
     if (threadIdx.x == 0) sync[kSyncFactorTickets] = 0u;
     if (threadIdx.x == 1) sync[kSyncFlag] = 0u;
+    if (threadIdx.x >= 2 && threadIdx.x < 4) sync[kSyncHelped + threadIdx.x - 2] = 0u;
 }
 
 void launch_factor_reset(uint32_t *sync, hipStream_t s, const Batch &bt)
@@ -230,11 +247,11 @@ template <typename S, int PREC, int K, int KQ>
 static void launch_one(dim3 grid, hipStream_t s, S *A, int64_t lda, int64_t n, int64_t kp, int Gp, int c0, int nsyrk,
                        int64_t slab, int cq0, int64_t slabq, int co0, int64_t slabo, int nko, double *Wleaf, int *info, uint32_t *tickets,
                        uint32_t ticket_base, uint32_t *flag, uint32_t epoch, int *status, __bf16 *Wsplit,
-                       int64_t slot_elems, const Batch &bt)
+                       int64_t slot_elems, const Batch &bt, int halves, int nh)
 {
     hipLaunchKernelGGL((factor_step_kernel<S, PREC, K, KQ>), grid, dim3(256), 0, s, A, lda, n, kp, Gp, c0, nsyrk, slab,
                        cq0, slabq, co0, slabo, nko, Wleaf, info, tickets, ticket_base, flag, epoch, status, Wsplit, slot_elems, bt.a,
-                       bt.leaf, bt.sync);
+                       bt.leaf, bt.sync, halves, nh);
 }
 
 template <typename S, int PREC>
@@ -242,11 +259,11 @@ static void launch_prec(dim3 grid, hipStream_t s, int K, int KQ, S *A, int64_t l
                         int c0, int nsyrk, int64_t slab, int cq0, int64_t slabq, int co0, int64_t slabo, int nko,
                         double *Wleaf, int *info,
                         uint32_t *tickets, uint32_t ticket_base, uint32_t *flag, uint32_t epoch, int *status,
-                        __bf16 *Wsplit, int64_t slot_elems, const Batch &bt)
+                        __bf16 *Wsplit, int64_t slot_elems, const Batch &bt, int halves, int nh)
 {
 #define MI_FS_ARGS grid, s, A, lda, n, kp, Gp, c0, nsyrk, slab, cq0, slabq, co0, slabo, nko, Wleaf, info, tickets, \
                    ticket_base, flag, \
-                   epoch, status, Wsplit, slot_elems, bt
+                   epoch, status, Wsplit, slot_elems, bt, halves, nh
     if constexpr (sizeof(S) == 8) {
         if (K == 256)
             launch_one<S, PREC, 256, 0>(MI_FS_ARGS);
@@ -271,7 +288,11 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
                         hipStream_t s, uint32_t *grid_out, int prec, __bf16 *Wsplit, const Batch &bt)
 {
     const int64_t below = n - kp - kNB;  // rows below the panel's diagonal block
-    const int Gp = kp < 0 ? 0 : 1 + (below > 0 ? (int)((below + 64 * kRowTiles - 1) / (64 * kRowTiles)) : 0);
+    // Helpers of the diagonal role (diag_helper), while the launch waits for one system's panel: a large
+    // batch's diagonal roles fill the chip by themselves (120 systems of order 512: 1600 us for the
+    // Gaussian processes without, 1665 with).
+    const int nh = sizeof(S) == 8 && kp > 0 && bt.count <= 16 ? 2 : 0;
+    const int Gp = kp < 0 ? 0 : 1 + nh + (below > 0 ? (int)((below + 64 * kRowTiles - 1) / (64 * kRowTiles)) : 0);
     int c0 = 0, nsyrk = 0, K = k >= 1 ? 256 : 128, KQ = 0, cq0 = 0, co0 = 0, nko = 0;
     int64_t slab = k >= 1 ? (k - 1) * kNB : 0, slabq = 0, slabo = 0;
     if constexpr (sizeof(S) == 8) {
@@ -289,6 +310,11 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
         slabq = q.slabq;
         slabo = q.slabo;
     }
+    // Half tiles (64 x 128) while each still gets a CU of its own: a tile alone on its CU takes 27 us in
+    // FP64 (28 in FP32 at depth 512), as long as the panel.  The split arithmetic's tiles stage their
+    // operands for the whole tile.
+    const int halves = (prec != kPrecBF16x3 && prec != kPrecBF16x6) && 2 * (int64_t)nsyrk * bt.count <= 256 ? 1 : 0;
+    nsyrk <<= halves;
     const unsigned grid = (unsigned)(Gp + nsyrk);
     *grid_out = (uint32_t)Gp;  // tickets drawn
     if (grid == 0) return;
@@ -297,15 +323,15 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
 #define MI_FS_ARGS g, s, K, KQ, A, lda, n, kp, Gp, c0, nsyrk, slab, cq0, slabq, co0, slabo, nko, Wleaf, info, \
                    tickets, ticket_base, flag, epoch, status
     if constexpr (sizeof(S) == 8) {
-        launch_prec<S, kPrecF64>(MI_FS_ARGS, nullptr, slot, bt);
+        launch_prec<S, kPrecF64>(MI_FS_ARGS, nullptr, slot, bt, halves, nh);
     } else if (prec == kPrecBF16) {
-        launch_prec<S, kPrecBF16>(MI_FS_ARGS, nullptr, slot, bt);
+        launch_prec<S, kPrecBF16>(MI_FS_ARGS, nullptr, slot, bt, halves, nh);
     } else if (prec == kPrecBF16x6) {
-        launch_prec<S, kPrecBF16x6>(MI_FS_ARGS, Wsplit, slot, bt);
+        launch_prec<S, kPrecBF16x6>(MI_FS_ARGS, Wsplit, slot, bt, halves, nh);
     } else if (prec == kPrecBF16x3) {
-        launch_prec<S, kPrecBF16x3>(MI_FS_ARGS, Wsplit, slot, bt);
+        launch_prec<S, kPrecBF16x3>(MI_FS_ARGS, Wsplit, slot, bt, halves, nh);
     } else {
-        launch_prec<S, kPrecF32>(MI_FS_ARGS, nullptr, slot, bt);
+        launch_prec<S, kPrecF32>(MI_FS_ARGS, nullptr, slot, bt, halves, nh);
     }
 #undef MI_FS_ARGS
 }

@@ -50,6 +50,7 @@ constexpr int kSyncStatus = 0;          // status bits (MI_SOLVE_TIMEOUT, ...)
 constexpr int kSyncSolveTickets = 32;   // 2 words: the forward and the backward sweep
 constexpr int kSyncRankTicket = 34;     // the rank update's ticket
 constexpr int kSyncFactorTickets = 64;  // the factorization's ticket counter
+constexpr int kSyncHelped = 80;         // 2 words: the diagonal role's helpers (that counter's line)
 constexpr int kSyncFlag = 96;           // the factorization's panel flag
 constexpr int kSyncWords = 128;
 

@@ -127,6 +127,47 @@ __device__ __forceinline__ void lds_tile_update(double *C, const double (&Pi)[4]
     for (int r = 0; r < 4; ++r) C[64 * r] = old[r] - acc[r];
 }
 
+// Tiles (i, j), i = i0, i0 + 2, ... (NT of them), of the block in S: C[x] (the tile's elements l + 64 r)
+// less its products with the panels 0 .. p, in turn, to S.  Each product's operands are read during the
+// one before.
+template <int NT>
+__device__ __forceinline__ void column_products(double *S, int i0, int j, int p, double (&C)[3][4])
+{
+    const int l = lane_id();
+    const double *pj = S + 256 * ((j * (j + 1)) / 2) + l;
+    const double *pi[NT];
+    double Pj[4], Pi[NT][4];
+#pragma unroll
+    for (int x = 0; x < NT; ++x) pi[x] = S + 256 * (((i0 + 2 * x) * (i0 + 2 * x + 1)) / 2) + l;
+    auto operands = [&](int q) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) Pj[s] = pj[256 * q + 64 * s];
+#pragma unroll
+        for (int x = 0; x < NT; ++x)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) Pi[x][s] = pi[x][256 * q + 64 * s];
+    };
+    operands(0);
+    for (int q = 0; q <= p; ++q) {
+        dvec4 acc[NT];
+#pragma unroll
+        for (int x = 0; x < NT; ++x) acc[x] = dvec4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int x = 0; x < NT; ++x) acc[x] = mfma_f64(Pj[s], Pi[x][s], acc[x]);
+        operands(q < p ? q + 1 : p);
+#pragma unroll
+        for (int x = 0; x < NT; ++x)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) C[x][r] -= acc[x][r];
+    }
+#pragma unroll
+    for (int x = 0; x < NT; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[256 * (((i0 + 2 * x) * (i0 + 2 * x + 1)) / 2 + j) + l + 64 * r] = C[x][r];
+}
+
 // Image stores reach memory by themselves (agent-scope stores are written through), so publishing
 // them takes the wait for them and the flag's store, no L2 writeback.
 __device__ __forceinline__ void image_store(double *p, double v)
@@ -134,9 +175,14 @@ __device__ __forceinline__ void image_store(double *p, double v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The panel flag of the launch with epoch e goes from 4 (e - 1) to 4 e: + 1 by each of two waves once
-// the image's block columns below kEarlyPanels are in memory, 4 e when all of it is.
-constexpr int kEarlyPanels = 4;
+// The panel flag of the launch with epoch e goes from 8 (e - 1) to 8 e: + 1 by each of two waves once
+// the image's block columns below kPart1, then below kPart2, are in memory, 8 e when all of it is.
+// The rows take about as long for the first part (2.8 us of MFMAs, and the image's tiles from memory)
+// as the diagonal role for the rest, and are left with 12 of their 144 MFMAs a row tile when the block
+// is done.  One part, two, and three with diag_helper and half tiles (syrk_tile): 41, 38 and 33 us a
+// launch in FP64 at n <= 1024; factor and solve at n = 3001 1330, 1230 and 1123 us, FP32 at n = 4001
+// 1979, 1850 and 1735 us.
+constexpr int kPart1 = 4, kPart2 = 6;
 
 // Cholesky of the 128 x 128 lower block in S (all 256 threads), in eight 16-column panels with
 // a one-panel lookahead inside the block.  After panel p is factored, with T = 7-p tile rows
@@ -144,28 +190,66 @@ constexpr int kEarlyPanels = 4;
 //   A(p): the leaf of p goes back to S; the T tiles of column p+1 get panel p's update (the
 //         waves round-robin), barrier;
 //   B(p): waves 0 and 1 factor panel p+1 (panel_factor2: VALU) while waves 2 and 3 store panel p
-//         (its tiles and its leaf's inverse) to the panel image W and apply it to the tiles right of
-//         column p+1 on the matrix core (21 tiles at most), barrier.
-// Column p+1 thus has every earlier panel's update before its factor, the tiles beyond it get
-// panel p's before phase A(p+1) touches them, and the rank-16 updates mostly run under the
-// column loop.  The panels below kEarlyPanels are published in B(kEarlyPanels), a panel's time after
-// their last store, so that the rows waiting for the block solve their part by them meanwhile.
-// Returns the first failing column or -1 (uniform).  xs: 2 x 256 doubles of LDS, s_fail: an LDS int.
-__device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, double *__restrict__ W, uint32_t *flag)
+//         (its tiles and its leaf's inverse) to the panel image W and bring column p+2 up to
+//         panel p on the matrix core (its tiles by panels 0 .. p), barrier.
+// Column p+1 thus has every earlier panel's update before its factor, and B's products, 12 tile
+// products at most, run under the column loop (1.4 us; applying panel p to all the tiles right of column
+// p+1 instead took up to 21, 2.8 us).  The panels below kPart1 and kPart2 are published in B of that
+// panel, a panel's time after their last store.
+// Returns the first failing column or -1 (uniform); the columns after it are then factored all the same,
+// to no use (a test of the failure in each panel took longer).  xs: 2 x 256 doubles of LDS, s_fail: an
+// LDS int.
+//
+// Akk: null when S holds the whole block; else S has tile columns 0 and 1 of it, and the others are
+// read from Akk (ld lda, order bs, identity beyond), each one phase ahead, columns 2, 3 and 4 .. 7 once
+// helped[0] and helped[1] have reached `epoch` (diag_helper).
+__device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, double *__restrict__ W, uint32_t *flag,
+                                            const double *Akk, int64_t lda, int bs, const uint32_t *helped,
+                                            uint32_t epoch, int *status)
 {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane_id();
     double *Xl = W + kLeafOffset;
     double lv[16];
-    __syncthreads();
+    double next[3][4];  // waves 2 and 3: this wave's tiles (i, j), i = j + w - 2, + 2, + 4, of the next column
+    auto fetch = [&](int j) {
+        if (Akk && (j == 2 || j == 4)) {
+            uint32_t spins = 0;
+            while (__hip_atomic_load(helped + (j == 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
+                __builtin_amdgcn_s_sleep(1);
+                if (++spins > (1u << 22)) {
+                    atomicOr(status, MI_PANEL_TIMEOUT);
+                    break;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // the loads stay behind the flag's
+        }
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            const int i = j + w - 2 + 2 * x;
+            if (i < 8) {
+                if (Akk) {
+                    const int gi = 16 * i + (l & 15), ci = gi < bs ? gi : bs - 1;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int gj = 16 * j + 4 * r + (l >> 4), cj = gj < bs ? gj : bs - 1;
+                        next[x][r] = coherent_load(Akk + ci + (int64_t)cj * lda);
+                    }
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) next[x][r] = S[256 * ((i * (i + 1)) / 2 + j) + l + 64 * r];
+                }
+            }
+        }
+    };
+    if (tid == 0) *s_fail = -1;
+    lds_barrier();
     if (w < 2) {
         const int f = panel_factor2(S, 0, xs, lv);
-        if (w == 0 && l == 0) *s_fail = f;
+        if (w == 0 && l == 0 && f >= 0) *s_fail = f;
+    } else {
+        fetch(2);
     }
-    __syncthreads();
-    {
-        const int f = __builtin_amdgcn_readfirstlane(*s_fail);
-        if (f >= 0) return f;
-    }
+    lds_barrier();
     for (int p = 0; p < 7; ++p) {
         const int T = 7 - p;
         const int tb = p + 1;  // first trailing tile row / column
@@ -191,53 +275,69 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, 
 #pragma unroll
             for (int c = 0; c < 16; ++c) S[sl(16 * p + l, 16 * p + c)] = lv[c];
         }
-        __syncthreads();
+        lds_barrier();
         // ---- B(p)
         if (w < 2) {
             const int f = panel_factor2(S, 16 * tb, xs + 256 * (tb & 1), lv);
-            if (w == 0 && l == 0) *s_fail = f;
+            if (w == 0 && l == 0 && f >= 0 && *s_fail < 0) *s_fail = 16 * tb + f;
         } else {
-            if (p == kEarlyPanels) {  // this wave's stores of the panels before p
+            if (p == kPart1 || p == kPart2) {  // this wave's stores of the panels before p
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 if (l == 0) __hip_atomic_fetch_add(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            double P[7][4];
+            // column j = p + 2: tile rows i = j + w - 2, + 2, + 4 of this wave
+            const int j = p + 2, i0 = j + w - 2;
+            double C[3][4];
 #pragma unroll
-            for (int x = 0; x < 7; ++x)
-                if (x < T) operand(x, P[x]);
+            for (int x = 0; x < 3; ++x)
 #pragma unroll
-            for (int ti = 1; ti < 7; ++ti) {
-#pragma unroll
-                for (int tj = 1; tj <= ti; ++tj) {
-                    const int t = ((ti - 1) * ti) / 2 + (tj - 1);  // enumerates the deferred tiles
-                    if (ti < T && w == 2 + (t & 1))
-                        lds_tile_update(S + 256 * (((tb + ti) * (tb + ti + 1)) / 2 + tb + tj) + l, P[ti], P[tj]);
+                for (int r = 0; r < 4; ++r) {
+                    const int gi = 16 * (i0 + 2 * x) + (l & 15), gj = 16 * j + 4 * r + (l >> 4);
+                    C[x][r] = !Akk || (gi < bs && gj < bs) ? next[x][r] : gi == gj ? 1.0 : 0.0;
                 }
-            }
+            // Panel p to the image, tile rows p + 1 + w - 2, + 2, ..., and its leaf's inverse; then the next
+            // column's loads.  In front of the products, so that the next phase, which waits for all of
+            // them when it takes up `next`, finds them done.
+            {
+                double im[4][4], xi[2];
 #pragma unroll
-            for (int x = 0; x < 7; ++x)
-                if (x < T && w == 2 + (x & 1)) {
-                    double *dst = W + 256 * (((tb + x) * (tb + x - 1)) / 2 + p) + l;
+                for (int x = 0; x < 4; ++x) {
+                    const int i = tb + w - 2 + 2 * x;
+                    if (i < 8) {
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) image_store(dst + 64 * s, P[x][s]);
+                        for (int s = 0; s < 4; ++s) im[x][s] = S[256 * ((i * (i + 1)) / 2 + p) + l + 64 * s];
+                    }
                 }
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int e = (tid & 127) + 128 * s;
-                image_store(Xl + 256 * p + e, xs[256 * (p & 1) + e]);
+                for (int s = 0; s < 2; ++s) xi[s] = xs[256 * (p & 1) + (tid & 127) + 128 * s];
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const int i = tb + w - 2 + 2 * x;
+                    if (i < 8) {
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) image_store(W + 256 * ((i * (i - 1)) / 2 + p) + l + 64 * s, im[x][s]);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < 2; ++s) image_store(Xl + 256 * p + (tid & 127) + 128 * s, xi[s]);
             }
+            fetch(j + 1);
+            const int nt = (9 - i0) / 2;  // this wave's tiles of the column
+            if (nt == 3)
+                column_products<3>(S, i0, j, p, C);
+            else if (nt == 2)
+                column_products<2>(S, i0, j, p, C);
+            else if (nt == 1)
+                column_products<1>(S, i0, j, p, C);
         }
-        __syncthreads();
-        const int f = __builtin_amdgcn_readfirstlane(*s_fail);
-        if (f >= 0) return 16 * tb + f;
+        lds_barrier();
     }
     image_store(Xl + 256 * 7 + tid, xs[256 + tid]);
     if (w == 0 && l < 16) {  // the last leaf
 #pragma unroll
         for (int c = 0; c < 16; ++c) S[sl(112 + l, 112 + c)] = lv[c];
     }
-    __syncthreads();
-    return -1;
+    return __builtin_amdgcn_readfirstlane(*s_fail);
 }
 
 // Row tiles of 16 per wave in the panel solve: a row role is 64 kRowTiles rows.  With one, the solve
@@ -288,9 +388,9 @@ __device__ __forceinline__ void trsm_in_registers(const double *smem, dvec4 (&X)
     }
 }
 
-// Block columns Q0 .. Q1-1 of a published panel image (16-byte aligned) -> LDS, two tiles at a time,
-// 16 bytes per load.
-template <int Q0, int Q1>
+// Block columns Q0 .. Q1-1 of a published panel image (16-byte aligned) -> LDS.  COHERENT: by loads that
+// are served from memory, as they stand behind no acquire; else two tiles at a time, 16 bytes per load.
+template <int Q0, int Q1, bool COHERENT>
 __device__ __forceinline__ void stage_panel_image(double *smem, const double *__restrict__ W)
 {
     constexpr int kTiles = 28 + 8;
@@ -301,6 +401,16 @@ __device__ __forceinline__ void stage_panel_image(double *smem, const double *__
         const int tj = t - ti * (ti - 1) / 2;
         return tj >= Q0 && tj < Q1;
     };
+    if constexpr (COHERENT) {
+        double v[kTiles];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+            if (wanted(t)) v[t] = coherent_load(W + 256 * t + threadIdx.x);
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t)
+            if (wanted(t)) smem[256 * t + threadIdx.x] = v[t];
+        return;
+    }
     const int half = threadIdx.x >> 7, e = 2 * (threadIdx.x & 127);
     int first = -1;  // of a pair
 #pragma unroll
@@ -317,9 +427,8 @@ __device__ __forceinline__ void stage_panel_image(double *smem, const double *__
     if (first >= 0 && half == 0) *(double2 *)(smem + 256 * first + e) = *(const double2 *)(W + 256 * first + e);
 }
 
-// Waits (thread 0) until *flag has reached `want`, then every wave acquires: each invalidates its own
-// view of the caches, so that the loads it issues next see what was published.  Returns the flag's
-// value less `base` (uniform), 0 on a timeout, recorded as MI_PANEL_TIMEOUT.
+// Waits (thread 0) until *flag has reached `want`.  Returns the flag's value less `base` (uniform), 0 on
+// a timeout, recorded as MI_PANEL_TIMEOUT.
 __device__ __forceinline__ int wait_panel_flag(int *s_seen, const uint32_t *flag, uint32_t base, int want, int *status)
 {
     if (threadIdx.x == 0) {
@@ -336,35 +445,40 @@ __device__ __forceinline__ int wait_panel_flag(int *s_seen, const uint32_t *flag
         *s_seen = seen;
     }
     __syncthreads();
-    const int seen = *s_seen;
-    if (seen > 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    return seen;
+    return *s_seen;
 }
 
 // The rows' solve, X as in trsm_in_registers: by the panels published early while the others are being
-// factored, if the block is not done yet, then by those.  Returns false if the factor failed or a wait
-// timed out.
+// factored, if the block is not done yet, then by those.  A block that is done is read after an acquire
+// (each wave invalidates its own view of the caches), through the L2 that the rows share; its parts by
+// coherent loads, since three acquires a role cost the tiles beside them their cached operands (a batch of
+// 120 systems of order 512 took 3% longer).  Returns false if the factor failed or a wait timed out.
 template <int RT>
 __device__ __forceinline__ bool solve_rows(double *smem, int *s_seen, dvec4 (&X)[RT][8], const double *__restrict__ W,
                                            const uint32_t *flag, uint32_t epoch, const int *info, int *status)
 {
-    const uint32_t base = 4 * (epoch - 1);
+    const uint32_t base = 8 * (epoch - 1);
     int seen = wait_panel_flag(s_seen, flag, base, 2, status);
     if (seen <= 0) return false;
-    if (seen >= 4) {
+    if (seen >= 8) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if (factor_failed(info)) return false;
-        stage_panel_image<0, 8>(smem, W);
+        stage_panel_image<0, 8, false>(smem, W);
         __syncthreads();
         trsm_in_registers<0, 8>(smem, X);
         return true;
     }
-    stage_panel_image<0, kEarlyPanels>(smem, W);
+    stage_panel_image<0, kPart1, true>(smem, W);
     __syncthreads();
-    trsm_in_registers<0, kEarlyPanels>(smem, X);
-    if (wait_panel_flag(s_seen, flag, base, 4, status) <= 0 || factor_failed(info)) return false;
-    stage_panel_image<kEarlyPanels, 8>(smem, W);
+    trsm_in_registers<0, kPart1>(smem, X);
+    if (wait_panel_flag(s_seen, flag, base, 4, status) <= 0) return false;
+    stage_panel_image<kPart1, kPart2, true>(smem, W);
     __syncthreads();
-    trsm_in_registers<kEarlyPanels, 8>(smem, X);
+    trsm_in_registers<kPart1, kPart2>(smem, X);
+    if (wait_panel_flag(s_seen, flag, base, 8, status) <= 0 || factor_failed(info)) return false;
+    stage_panel_image<kPart2, 8, true>(smem, W);
+    __syncthreads();
+    trsm_in_registers<kPart2, 8>(smem, X);
     return true;
 }
 
@@ -420,16 +534,18 @@ __device__ __forceinline__ void trsm_rows(double *smem, int *s_seen, T *__restri
     }
 }
 
-// FP64 update of the diagonal block straight into LDS: S = A_kk - P_0 P_0^T for tile rows W
-// and 7-W, their tiles at and left of the diagonal -- 9 tiles per wave, the 36 lower tiles
-// over the 4 waves -- with acc starting from A_kk; identity beyond bs.  A diagonal tile is
-// written whole (its upper entries are never read as data).
-template <int W>
-__device__ __forceinline__ void diag_update_f64(double *S, const double *__restrict__ Akk,
-                                                const double *__restrict__ P0, int64_t lda, int bs)
+// FP64 update of tile columns [C0, C1) of the diagonal block, A_kk - P_0 P_0^T, for tile rows W and
+// 7-W, their tiles at and left of the diagonal, with acc starting from A_kk: to S (identity beyond bs; a
+// diagonal tile is written whole, its upper entries are never read as data) for C0 = 0, written
+// through to A_kk (its lower entries) for the others.
+template <int W, int C0, int C1>
+__device__ __forceinline__ void diag_update_f64(double *S, double *__restrict__ Akk, const double *__restrict__ P0,
+                                                int64_t lda, int bs)
 {
-    constexpr uint32_t kActive = ((1u << (W + 1)) - 1u) | (((1u << (8 - W)) - 1u) << 8);
-    WaveTile<2, 8, 5, true, kActive> t;  // 72 accumulator registers: room for five k-steps in flight
+    constexpr uint32_t kCols = ((1u << C1) - 1u) & ~((1u << C0) - 1u);
+    constexpr uint32_t kActive = (((1u << (W + 1)) - 1u) & kCols) | ((((1u << (8 - W)) - 1u) & kCols) << 8);
+    // registers for eight k-steps in flight with four tiles at most, for five with nine
+    WaveTile<2, 8, C1 - C0 == 8 ? 5 : 8, true, kActive> t;
     const int rows[2] = {16 * W, 16 * (7 - W)};
     t.zero();
     t.load_acc(Akk, lda, rows, 0, bs, bs);
@@ -446,9 +562,23 @@ __device__ __forceinline__ void diag_update_f64(double *S, const double *__restr
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = 16 * ti + (l & 15), j = 16 * b + 4 * r + (l >> 4);
-                    C[64 * r] = (i < bs && j < bs) ? t.acc[a][b][r] : (i == j ? 1.0 : 0.0);
+                    if (C0 == 0)
+                        C[64 * r] = (i < bs && j < bs) ? t.acc[a][b][r] : (i == j ? 1.0 : 0.0);
+                    else if (i < bs && j <= i)
+                        image_store(Akk + i + (int64_t)j * lda, t.acc[a][b][r]);
                 }
             }
+    }
+}
+template <int C0, int C1>
+__device__ __forceinline__ void diag_update_columns(int w, double *S, double *__restrict__ Akk,
+                                                    const double *__restrict__ P0, int64_t lda, int bs)
+{
+    switch (w) {
+    case 0: diag_update_f64<0, C0, C1>(S, Akk, P0, lda, bs); break;
+    case 1: diag_update_f64<1, C0, C1>(S, Akk, P0, lda, bs); break;
+    case 2: diag_update_f64<2, C0, C1>(S, Akk, P0, lda, bs); break;
+    default: diag_update_f64<3, C0, C1>(S, Akk, P0, lda, bs); break;
     }
 }
 
@@ -495,10 +625,10 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
     }
 }
 
-// The panel role of one block step; g is the role from the ticket:
+// The panel role of one block step; g is the role from the ticket, less the nh helpers' (diag_helper):
 //   role 0   : C = A_kk - P_0 P_0^T straight into LDS, Cholesky in LDS, the panel image
 //              (L11's strictly lower tiles and the leaf inverses) to the workspace, published by
-//              `flag` in two parts, then L11 into A;
+//              `flag` in three parts, then L11 into A;
 //   role g>0 : the g-th 64 kRowTiles rows below the block: C = A_gk - P_g P_0^T, then rows <-
 //              rows * L11^{-T} with the published image as it comes, stored once.
 // The diagonal role publishes even on a failing pivot, so that no waiter is left behind;
@@ -508,11 +638,30 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
 // (the diagonal factor and the panel solve are FP64 for every T).  With T = double the row
 // role keeps its rows in registers from the update to the store; with T = float the update
 // is rounded to FP32 storage first (as the mixed-precision trailing updates are) and read back.
+// Helper h of the diagonal role (FP64, k0 > 0): tile columns 2, 3 (h = 0) or 4 .. 7 of A_kk - P_0 P_0^T
+// into A_kk, then helped[h] = epoch.  The update's 36 tiles are 18400 cycles of MFMA on one CU, in front
+// of everything else on the chain; the diagonal role computes the 15 tiles of columns 0 and 1 and needs
+// column 2 a panel's time later, column 4 three panels' time.
+__device__ __forceinline__ void diag_helper(int h, double *__restrict__ A, int64_t lda, int64_t n, int64_t k0,
+                                            uint32_t *helped, uint32_t epoch)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int bs = (int)((n - k0) < 128 ? (n - k0) : 128);
+    double *Akk = A + k0 + k0 * lda;
+    const double *P0 = A + k0 + (k0 - 128) * lda;
+    if (h == 0)
+        diag_update_columns<2, 4>(w, nullptr, Akk, P0, lda, bs);
+    else
+        diag_update_columns<4, 8>(w, nullptr, Akk, P0, lda, bs);
+    global_barrier();  // every wave's stores are in memory
+    if (threadIdx.x == 0) __hip_atomic_store(helped + h, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <typename T, int PREC>
-__device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__restrict__ A,
+__device__ __forceinline__ void panel_role(int g, int nh, double *smem, int *s_ok, T *__restrict__ A,
                                            int64_t lda, int64_t n, int64_t k0, double *__restrict__ Wleaf, int *info,
-                                           uint32_t *flag, uint32_t epoch, int *status, __bf16 *split = nullptr,
-                                           int64_t split_lo = 0)
+                                           uint32_t *flag, const uint32_t *helped, uint32_t epoch, int *status,
+                                           __bf16 *split = nullptr, int64_t split_lo = 0)
 {
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -526,23 +675,22 @@ __device__ __forceinline__ void panel_role(int g, double *smem, int *s_ok, T *__
         __shared__ double xs[2 * 256];  // potrf_in_lds
         if (k0 > 0) {
             if constexpr (sizeof(T) == 8) {
-                const double *P0 = A + k0 + (k0 - 128) * lda;
-                switch (w) {
-                case 0: diag_update_f64<0>(smem, Ck, P0, lda, bs); break;
-                case 1: diag_update_f64<1>(smem, Ck, P0, lda, bs); break;
-                case 2: diag_update_f64<2>(smem, Ck, P0, lda, bs); break;
-                default: diag_update_f64<3>(smem, Ck, P0, lda, bs); break;
-                }
+                if (nh)
+                    diag_update_columns<0, 2>(w, smem, Ck, A + k0 + (k0 - 128) * lda, lda, bs);
+                else
+                    diag_update_columns<0, 8>(w, smem, Ck, A + k0 + (k0 - 128) * lda, lda, bs);
             } else {
                 diag_update_lowp<T, PREC>(smem, A, lda, k0, bs);
             }
         } else {
             block_to_lds(smem, Ck, lda, bs);
         }
-        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag);  // begins with a barrier
+        const double *Akk = nullptr;
+        if constexpr (sizeof(T) == 8) Akk = nh ? Ck : nullptr;
+        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag, Akk, lda, bs, helped, epoch, status);  // a barrier first
         if (f >= 0 && tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
         global_barrier();  // every wave's stores of the image are in memory
-        if (tid == 0) __hip_atomic_store(flag, 4 * epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) __hip_atomic_store(flag, 8 * epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (f < 0) lds_to_block(smem, Ck, lda, bs);  // read by later launches only
         return;
     }

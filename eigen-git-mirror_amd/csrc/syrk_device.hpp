@@ -13,27 +13,32 @@
 
 namespace mi {
 
-// Tile (ti, tj) of C (m x m, lower), columns restricted to j < ncol; depth K (compile time).
+// Tile (ti, tj) of C (m x m, lower), columns restricted to j < ncol; depth K (compile time).  HALF: its
+// rows 64 half .. + 63 alone, wave tiles of 32 x 64.
 // T = double: FP64 MFMA; T = float: FP32 storage with the low-precision MFMA of PREC.
-template <int K, typename T = double, int PREC = kPrecF64>
+template <int K, typename T = double, int PREC = kPrecF64, bool HALF = false>
 __device__ __forceinline__ void syrk_tile(T *__restrict__ C, int64_t ldc, const T *__restrict__ P, int64_t ldp,
-                                          int m, int ncol, int ti, int tj)
+                                          int m, int ncol, int ti, int tj, int half = 0)
 {
+    constexpr int TA = HALF ? 2 : 4;
     const int w = threadIdx.x >> 6, wr = w >> 1, wc = w & 1;
-    if (ti == tj && wr == 0 && wc == 1) return;
-    const int i0 = ti * 128 + wr * 64, j0 = tj * 128 + wc * 64;
+    if (ti == tj && wc == 1 && (HALF ? half : wr) == 0) return;  // strictly upper
+    const int i0 = ti * 128 + half * 64 + wr * 16 * TA, j0 = tj * 128 + wc * 64;
+    if (HALF && i0 >= m) return;
     if constexpr (sizeof(T) == 8) {
         // C is read into the accumulators first, so its loads overlap the first operand
         // prefetch, and the negated product accumulates into it: the tile ends with stores only
         // (about 2% off the factorization at n = 8192 against a read of C after the last MFMA)
-        WaveTile<4, 4, 3, true> t;
-        const int rows[4] = {i0, i0 + 16, i0 + 32, i0 + 48};
+        WaveTile<TA, 4, HALF ? 5 : 3, true> t;
+        int rows[TA];
+#pragma unroll
+        for (int a = 0; a < TA; ++a) rows[a] = i0 + 16 * a;
         t.load_acc(C, ldc, rows, j0, m, ncol);
         t.setup(P, ldp, i0, m, P, ldp, j0, m, K);
         t.template run_fixed<K / 4>();
         t.template store<true, true>(C, ldc, i0, j0, m, ncol);
     } else {
-        using Tile = typename TileSel<T, PREC>::type;
+        using Tile = typename TileSel<T, PREC, TA>::type;
         Tile t;
         t.zero();
         t.setup(P, ldp, i0, m, P, ldp, j0, m, K);

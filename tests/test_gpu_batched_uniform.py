@@ -202,6 +202,22 @@ def test_gp_gradient_inverse_tree(dev, n, row_major):
     assert float((y1.grad.cpu() + g[1] * al[1]).abs().max()) <= tol * float(al[1].abs().max())
 
 
+@pytest.mark.parametrize("n", [128, 129, 200, 257, 400])
+def test_large_batch_factor_is_the_single_one(dev, n):
+    """A batch above the diagonal role's helpers (17 systems), whose diagonal blocks one workgroup
+    updates whole, against single systems, whose helpers do most of it: the same bits."""
+    say(f"[gpu] batch of 17 against singles n={n}")
+    a = torch.stack([torch.from_numpy(workloads.gram_spd(n, seed=z)) for z in range(17)]).to(dev)
+    l = mi_llt.colmajor_batched(a)
+    info = torch.zeros(17, dtype=torch.int32, device=dev)
+    mi_llt.potrf_batched_async_(l, info)
+    assert int(info.abs().sum()) == 0
+    for z in (0, 7, 16):
+        one = mi_llt.colmajor(a[z])
+        assert mi_llt.potrf_(one) == 0
+        assert torch.equal(one, l[z]), z
+
+
 def test_batched_argument_errors(dev):
     h = mi_llt.default_handle()
     L = mi_llt.lib()
