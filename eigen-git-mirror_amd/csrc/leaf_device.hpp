@@ -73,7 +73,7 @@ __device__ __forceinline__ void leaf_updates(T (&u)[16], T (&v)[16])
 
 // Column J with its pivot x on every lane.  The next column's chain -- estimate, Newton step -- is
 // laid between the updates, which do not depend on it.
-template <int J, bool LAID, typename T>
+template <int J, typename T>
 __device__ __forceinline__ void leaf_columns(T (&u)[16], T (&v)[16], T rd, int &bad)
 {
     u[J] *= rd;
@@ -86,29 +86,24 @@ __device__ __forceinline__ void leaf_columns(T (&u)[16], T (&v)[16], T rd, int &
         // LLT.h:327-330; a NaN pivot passes.  (A vector minimum: a scalar test would put a branch and a
         // vector-to-scalar round trip into every column, half the column's time.)
         bad = min(bad, x <= (T)0 ? J + 1 : 16);
-        if constexpr (LAID) {
-            constexpr int N = 14 - J, C = J + 2;  // updates left, in four parts
-            const T r = rsqrt_estimate(x);
-            const T h = (T)0.5 * x;
-            __builtin_amdgcn_sched_barrier(0);
-            leaf_updates<J, C, C + N / 4>(u, v);
-            __builtin_amdgcn_sched_barrier(0);
-            const T hr = h * r;
-            __builtin_amdgcn_sched_barrier(0);
-            leaf_updates<J, C + N / 4, C + N / 2>(u, v);
-            __builtin_amdgcn_sched_barrier(0);
-            const T f = (T)1.5 - hr * r;
-            __builtin_amdgcn_sched_barrier(0);
-            leaf_updates<J, C + N / 2, C + 3 * N / 4>(u, v);
-            __builtin_amdgcn_sched_barrier(0);
-            const T rn = r * f;
-            __builtin_amdgcn_sched_barrier(0);
-            leaf_updates<J, C + 3 * N / 4, 16>(u, v);
-            leaf_columns<J + 1, LAID>(u, v, rn, bad);
-        } else {
-            leaf_updates<J, J + 2, 16>(u, v);
-            leaf_columns<J + 1, LAID>(u, v, rsqrt_newton(x), bad);
-        }
+        constexpr int N = 14 - J, C = J + 2;  // updates left, in four parts
+        const T r = rsqrt_estimate(x);
+        const T h = (T)0.5 * x;
+        __builtin_amdgcn_sched_barrier(0);
+        leaf_updates<J, C, C + N / 4>(u, v);
+        __builtin_amdgcn_sched_barrier(0);
+        const T hr = h * r;
+        __builtin_amdgcn_sched_barrier(0);
+        leaf_updates<J, C + N / 4, C + N / 2>(u, v);
+        __builtin_amdgcn_sched_barrier(0);
+        const T f = (T)1.5 - hr * r;
+        __builtin_amdgcn_sched_barrier(0);
+        leaf_updates<J, C + N / 2, C + 3 * N / 4>(u, v);
+        __builtin_amdgcn_sched_barrier(0);
+        const T rn = r * f;
+        __builtin_amdgcn_sched_barrier(0);
+        leaf_updates<J, C + 3 * N / 4, 16>(u, v);
+        leaf_columns<J + 1>(u, v, rn, bad);
     }
 }
 
@@ -116,12 +111,12 @@ __device__ __forceinline__ void leaf_columns(T (&u)[16], T (&v)[16], T rd, int &
 // v: rows that take the same column operations, v <- v L^{-T}.  With the identity (v[c] = c ==
 // l % 16) lane l is left with column l % 16 of X = L^{-1}: v[c] = X[c][l % 16].  Returns the failing
 // column or -1 (uniform); entries of u right of a lane's diagonal change but are never read.
-template <bool LAID = true, typename T>
+template <typename T>
 __device__ __forceinline__ int leaf_factor(T (&u)[16], T (&v)[16])
 {
     const T x = row_bcast<0>(u[0]);
     int bad = x <= (T)0 ? 0 : 16;
-    leaf_columns<0, LAID>(u, v, rsqrt_newton(x), bad);
+    leaf_columns<0>(u, v, rsqrt_newton(x), bad);
     bad = __builtin_amdgcn_readfirstlane(bad);
     return bad < 16 ? bad : -1;
 }

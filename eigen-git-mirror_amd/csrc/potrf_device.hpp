@@ -19,22 +19,6 @@ __device__ __forceinline__ int sl(int r, int c)
     const int ti = r >> 4, tj = c >> 4;
     return 256 * ((ti * (ti + 1)) / 2 + tj) + (r & 15) + 16 * (c & 15);
 }
-// The strictly lower tiles only (the panel solve keeps L11 without its diagonal tiles, whose
-// inverses it uses instead): r >> 4 > c >> 4.
-__device__ __forceinline__ int sls(int r, int c)
-{
-    const int ti = r >> 4, tj = c >> 4;
-    return 256 * ((ti * (ti - 1)) / 2 + tj) + (r & 15) + 16 * (c & 15);
-}
-
-__device__ __forceinline__ double readlane_d(double x, int lane)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, x);
-    const int lo = __builtin_amdgcn_readlane((int)(uint32_t)u, lane);
-    const int hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
-    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
 // Panel p (columns c0..c0+15 of the 128 x 128 block in S, tiled: sl), waves 0 and 1 (2 and 3 are
 // meanwhile busy with the previous panel's deferred update, see potrf_in_lds).  Each row of 16
 // lanes holds the whole 16 x 16 leaf in u (leaf_device.hpp), so its broadcasts need no barrier and
@@ -350,7 +334,8 @@ constexpr int kRowTiles = 1;
 
 // The panel solve works on a wave's 16 RT rows x 128 columns in the FP64 MFMA result layout:
 // X[t][p][r] is row 16t + lane%16, column 16p + 4r + lane/16 (t < RT row tiles, p = 0..7
-// column strips).  It needs, in LDS, the 28 strictly lower tiles of L (Ls, sls order) and the
+// column strips).  It needs, in LDS, the 28 strictly lower tiles of L (Ls: tile (ti, tj) at
+// 256 * (ti(ti-1)/2 + tj)) and the
 // 8 leaf inverses (Xs, 256 doubles each, column-major): the panel image of kernels.hpp.
 //
 // X <- X L^{-T} in place, strip by strip (TriangularSolverMatrix.h:186-329, blocked by 16):
