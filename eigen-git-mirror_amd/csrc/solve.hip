@@ -75,6 +75,13 @@ __device__ __forceinline__ bool await_written(double (&v)[M], const double *p, i
 // case on the chain: the consumer finishes its previous product after the producer publishes)
 // costs one round trip.  Small copies (N < ST): every
 // thread polls its own elements, so a copy that was waited for costs one round trip too.
+//
+// Every wave passes a barrier after its last put, so all of the copy is there on return.  Large
+// copies have another between the poll and the first put: whatever the waves read of the destination
+// before the call is read by then.  Small copies have none, and a thread that finds its element
+// written puts it at once, beside waves that are still multiplying the previous copy: their
+// destination must be one that nobody has read since the barrier of an earlier call (two used in
+// turn are; Sums::NY).
 template <int N, class Put>
 __device__ __forceinline__ bool fetch_published(const double *src, int *status, int *s_ok, int *s_fail, Put put)
 {
@@ -143,6 +150,7 @@ struct Sums;
 template <>
 struct Sums<1> {
     static constexpr int NE = 1;          // elements a lane ends with
+    static constexpr int NY = 2;          // staged copies in LDS, used in turn (fetch_published)
     static constexpr int NC = 4, NA = 4;  // chains of dependent sums: of a coupling's product, of the others
     double v;
     __device__ __forceinline__ void zero() { v = 0.0; }
@@ -176,7 +184,7 @@ struct Sums<1> {
 };
 template <>
 struct Sums<16> {
-    static constexpr int NE = 4, NC = 4, NA = 1;
+    static constexpr int NE = 4, NY = 1, NC = 4, NA = 1;
     dvec4 v;
     __device__ __forceinline__ void zero() { v = dvec4{0.0, 0.0, 0.0, 0.0}; }
     __device__ __forceinline__ void mac(const double *col, double p) { v = mfma_f64(*col, p, v); }
@@ -249,7 +257,8 @@ __global__ __launch_bounds__(ST, 2) void solve_sweep_kernel(const T *__restrict_
     // Ys[c + SC (k + k / 32)]: the published block being consumed, one padding row per
     // 32 k, so that lanes reading k = 32 q + s (q = lane / 16, the permuted order below) hit
     // distinct banks
-    __shared__ double Ys[SP + 4 * SC];
+    constexpr int YS = SP + 4 * SC;
+    __shared__ double Ys[Sums<SC>::NY * YS];
     __shared__ double Ts[SP];         // Ts[c + SC*r]: the block's residual before the inverse
     __shared__ int s_item, s_ok, s_fail;
     const int nblk = (int)((n + SB - 1) / SB);
@@ -301,10 +310,14 @@ __global__ __launch_bounds__(ST, 2) void solve_sweep_kernel(const T *__restrict_
     const double *M2p = Wi + (BACKWARD ? kInvN2 : kInvM2) + r + SB * kl;
     const double *M3p = Wi + (BACKWARD ? kInvN3 : kInvM3) + r + SB * kl;
 
-    // Stages packed block jb into Ys once it is written (false: given up).
-    auto stage = [&](int jb) -> bool {
+    // Stages packed block jb into copy y of Ys once it is written (false: given up).  The plain
+    // contributions use copy 0, each followed by a barrier; of the couplings the second uses copy 1,
+    // so that where a stage may overwrite a copy that is still being read (fetch_published), it writes
+    // the other one, and the next write of the first is behind its barrier.
+    constexpr int Y1 = (Sums<SC>::NY - 1) * YS;
+    auto stage = [&](int jb, int y = 0) -> bool {
         return fetch_published<SP>(gpk + (size_t)jb * SP, status, &s_ok, &s_fail,
-                                   [&](int e, double v) { Ys[e + SC * (e / (32 * SC))] = v; });
+                                   [&](int e, double v) { Ys[y + e + SC * (e / (32 * SC))] = v; });
     };
 
     // P operand of a contributing block, k-step s: P[row][k] = L_ij[row][k] (forward) or
@@ -497,12 +510,12 @@ __global__ __launch_bounds__(ST, 2) void solve_sweep_kernel(const T *__restrict_
         for (int e = 0; e < NE; ++e) y[e] -= ct[e];
     }
     if (crit2) {
-        if (!stage(ib - 2 * jstep)) return;
+        if (!stage(ib - 2 * jstep, Y1)) return;
 #pragma unroll
         for (int q = 0; q < NC; ++q) cq[q].zero();
 #pragma unroll
         for (int s = 0; s < SB / 4; ++s) {
-            cq[s & (NC - 1)].mac(ys(yo4, s), pv[s]);
+            cq[s & (NC - 1)].mac(ys(yo4, s) + Y1, pv[s]);
             pv[s] = M1p[(size_t)4 * SB * s];
             Sums<SC>::step(s, yo4);
         }

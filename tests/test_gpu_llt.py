@@ -101,6 +101,31 @@ def test_one_column_solve_edges(dev, n, pad):
     assert_status_ok()
 
 
+@pytest.mark.parametrize("n", [1025, 2049, 4000])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_one_column_solve_repeats_bit_for_bit(dev, n, dtype):
+    """One right-hand side solved 300 times with one factor, two of them in turn: every block's copy in
+    LDS must stay until all four waves are done with it, so each pass gives the first one's bits (the
+    sums run in a fixed order)."""
+    say(f"[gpu] one-column solve repeated n={n} {dtype}")
+    a, b = workloads.gram_spd(n, seed=n + 2), workloads.rhs(n, 2, seed=n + 3)
+    m = mi_llt.colmajor(torch.from_numpy(a).to(dev).to(dtype))
+    bd = torch.from_numpy(b).to(dev).to(dtype)
+    factor, solve = (mi_llt.potrf_, mi_llt.potrs_) if dtype == torch.float64 else (mi_llt.spotrf_, mi_llt.spotrs_)
+    assert factor(m) == 0
+    first = []
+    for it in range(300):
+        x = mi_llt.colmajor(bd[:, it % 2:it % 2 + 1])
+        solve(m, x)
+        if it < 2:
+            first.append(x)
+            if dtype == torch.float64:
+                assert oracle.solve_berr(a, x.cpu().numpy(), b[:, it:it + 1]) <= TOL_BERR
+        else:
+            assert torch.equal(x, first[it % 2]), f"pass {it}"
+    assert_status_ok()
+
+
 @pytest.mark.parametrize("tag", ["kat3"] + [f"spd{n}" for n in (1, 2, 3, 7, 8, 16, 31, 32, 33, 64, 100, 127,
                                                                 128, 129, 200)])
 def test_factor_solve_matches_eigen_golden(dev, tag):
