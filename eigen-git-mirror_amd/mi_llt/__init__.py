@@ -67,6 +67,7 @@ def lib() -> ctypes.CDLL:
         L.mi_llt_trace_reset.argtypes = [_VP]
         L.mi_llt_status.argtypes = [_VP, ctypes.POINTER(_INT)]
         L.mi_llt_inject_status.argtypes = [_VP, _INT]
+        L.mi_llt_wait_info.argtypes = [_VP, _I64, _VP, ctypes.POINTER(_I64), ctypes.POINTER(_INT)]
         L.mi_dposv_vbatched.argtypes = [_VP, ctypes.c_char, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP]
         L.mi_sposv_vbatched.argtypes = [_VP, ctypes.c_char, _I64, _VP, _VP, _VP, _VP, _VP, _VP, _VP]
         L.mi_llt_set_vbatched_config.argtypes = [_VP, _INT, _INT, _INT]
@@ -118,6 +119,7 @@ def lib() -> ctypes.CDLL:
         for name in ("mi_llt_create", "mi_llt_destroy", "mi_llt_set_stream", "mi_dpotrf", "mi_dpotrf_async",
                      "mi_dpotrs", "mi_dposv_async", "mi_dsy_l1norm", "mi_ssy_l1norm", "LAPACKE_dpotrf", "LAPACKE_dpotrs",
                      "mi_llt_trace", "mi_llt_trace_read", "mi_llt_trace_reset", "mi_llt_status", "mi_llt_inject_status",
+                     "mi_llt_wait_info",
                      "mi_dposv_mixed", "mi_dposv_vbatched", "mi_sposv_vbatched", "mi_llt_set_vbatched_config",
                      "mi_llt_get_vbatched_config", "mi_dpotrf_adjoint", "mi_dpotrs_adjoint", "mi_spotrf",
                      "mi_spotrf_async", "mi_spotrs", "mi_dtrsm", "mi_dsyrk", "mi_dpocon", "mi_dllt_rank_update",
@@ -203,6 +205,15 @@ class Handle:
         v = ctypes.c_int(0)
         self.check(lib().mi_llt_status(self._h, ctypes.byref(v)), "mi_llt_status")
         return int(v.value)
+
+    def wait_info(self, info: torch.Tensor) -> tuple[int, int]:
+        """Waits for the asynchronous calls that write ``info`` (int32, on the device): the index and the
+        value of its first word that is not 0 (``(info.numel(), 0)`` if none).  Raises (``E_DEVICE``) when
+        the device recorded a failure, which leaves the info words at 0."""
+        z, v = _I64(0), ctypes.c_int(0)
+        self.check(lib().mi_llt_wait_info(self._h, int(info.numel()), _VP(info.data_ptr()), ctypes.byref(z),
+                                          ctypes.byref(v)), "mi_llt_wait_info")
+        return int(z.value), int(v.value)
 
     def inject_status(self, bits: int):
         """Sets device status bits on the handle's stream (tests of the failure path)."""

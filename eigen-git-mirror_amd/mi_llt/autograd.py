@@ -31,6 +31,15 @@ def _cm(t: torch.Tensor) -> torch.Tensor:
     return colmajor(t.to(torch.float64))
 
 
+def _check_factor(info: torch.Tensor, batched: bool) -> None:
+    """Waits for the factor; raises if the device recorded a failure (a timeout: the kernels then stop or
+    skip their work and leave the info at 0) or a system is not positive definite."""
+    z, i = default_handle().wait_info(info)
+    if i != 0:
+        raise torch.linalg.LinAlgError(f"Cholesky: {f'system {z}: ' if batched else ''}the leading minor of order "
+                                       f"{i} is not positive definite")
+
+
 class Cholesky(torch.autograd.Function):
     @staticmethod
     def forward(ctx, a: torch.Tensor) -> torch.Tensor:
@@ -117,9 +126,7 @@ class GPLogMarginal(torch.autograd.Function):
         a = _cm(y.reshape(y.shape[0], -1))
         d_info = torch.zeros(1, dtype=torch.int32, device=l.device)
         posv_async_(l, a, d_info)
-        info = int(d_info.item())
-        if info != 0:
-            raise torch.linalg.LinAlgError(f"Cholesky: the leading minor of order {info} is not positive definite")
+        _check_factor(d_info, False)
         ctx.save_for_backward(l, a)
         ctx.row_major = _row_major(k)
         return (-0.5 * torch.dot(y, a.reshape(-1) if y.dim() == 1 else a) - torch.log(torch.diagonal(l)).sum()
@@ -150,11 +157,7 @@ class CholeskyBatched(torch.autograd.Function):
         l = colmajor_batched(a.to(torch.float64))
         info = torch.zeros(l.shape[0], dtype=torch.int32, device=l.device)
         potrf_batched_async_(l, info)
-        bad = torch.nonzero(info).flatten()
-        if bad.numel():
-            z = int(bad[0])
-            raise torch.linalg.LinAlgError(f"Cholesky: system {z}: the leading minor of order {int(info[z])} is not "
-                                           "positive definite")
+        _check_factor(info, True)
         l = colmajor_batched(torch.tril(l))
         ctx.save_for_backward(l)
         return l
@@ -222,11 +225,7 @@ class GPLogMarginalBatched(torch.autograd.Function):
         a = colmajor_batched(y.detach().to(torch.float64))
         info = torch.zeros(l.shape[0], dtype=torch.int32, device=l.device)
         posv_batched_async_(l, a, info)
-        bad = torch.nonzero(info).flatten()
-        if bad.numel():
-            z = int(bad[0])
-            raise torch.linalg.LinAlgError(f"Cholesky: system {z}: the leading minor of order {int(info[z])} is not "
-                                           "positive definite")
+        _check_factor(info, True)
         d = torch.diagonal(l, dim1=-2, dim2=-1)
         ya = a.squeeze(-1)
         ctx.save_for_backward(l, a)

@@ -78,6 +78,10 @@ int64_t mi_llt_workspace_bytes(mi_llt_handle h);
 #define MI_LLT_STATUS_PANEL_TIMEOUT 2
 #define MI_LLT_STATUS_FACTOR_TICKET 4
 int mi_llt_status(mi_llt_handle h, int *status);
+/* Waits for asynchronous calls that leave `count` info words at d_info: *info is the first that is
+ * not 0 and *index its place (0 and `count` if all are), or MI_LLT_E_DEVICE is returned and the status
+ * word cleared when the device recorded a failure, which leaves the info words at 0. */
+int mi_llt_wait_info(mi_llt_handle h, int64_t count, const int *d_info, int64_t *index, int *info);
 /* Sets `bits` in the handle's status word on its stream, as a device failure would (no
  * reference counterpart: for tests of the failure path, which must not make a kernel fail). */
 int mi_llt_inject_status(mi_llt_handle h, int bits);

@@ -14,6 +14,7 @@ import pytest
 import torch
 
 import mi_llt
+from mi_llt import autograd as mad
 from mi_llt import workloads
 
 pytestmark = pytest.mark.gpu
@@ -130,3 +131,21 @@ def test_device_status_is_reported_and_cleared(dev):
     assert ei.value.code == mi_llt.E_DEVICE
     _, iters, berr, info = mi_llt.posv_mixed(a0, b0, prec="fp32", handle=h)
     assert info == 0 and berr <= 1e-14
+
+
+def test_autograd_forwards_report_device_status(dev):
+    """A failure that the device recorded (the kernels skip their work, info stays 0) is raised by every
+    forward that factors asynchronously, before its result is used, and cleared."""
+    n = 200
+    k = torch.from_numpy(workloads.gram_spd(n, seed=9)).to(dev)
+    y = torch.from_numpy(workloads.rhs(n, 1, seed=9)[:, 0].copy()).to(dev)
+    calls = [lambda: mad.gp_log_marginal(k, y), lambda: mad.gp_log_marginal_batched(k[None], y[None]),
+             lambda: mad.cholesky_batched(k[None])]
+    for i, call in enumerate(calls):
+        print(f"[gpu] device status in autograd forward {i}", flush=True)
+        want = call()
+        mi_llt.default_handle().inject_status(mi_llt.STATUS_PANEL_TIMEOUT)
+        with pytest.raises(mi_llt.MiLLTError) as ei:
+            call()
+        assert ei.value.code == mi_llt.E_DEVICE
+        assert torch.equal(call(), want)
