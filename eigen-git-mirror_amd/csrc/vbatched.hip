@@ -8,23 +8,26 @@
 // A system is factored by a group of W waves, W = 1, 2 or 4 by its order (n <= 64, 128, 256), in
 // block columns of 64, left-looking: a wave holds its rows' part of the block column -- up to 4
 // tile rows of 16 (dealt round-robin over the group's waves) x 4 tile columns -- in registers:
-//   accumulate: C_ic = A_ic - sum_k L_ik L_ck^T over the finished columns (the wave's rows and the
+//   accumulate: S_ic = sum_k L_ik L_ck^T over the finished columns (the wave's rows and the
 //               block's own four tile rows are read back once per block column), MFMA
 //   then for each of the 4 tile columns c, right-looking inside the block:
+//   subtract: C_ic = A_ic - S_ic, once all earlier columns are in S: a sum has its own rounding, not A's
+//             (in single precision the products of the block's own columns, added to A one by one, made
+//             the whole call's error 7.7e-7 instead of 6.1e-7)
 //   leaf:   L_cc = chol(C_cc), X_cc = L_cc^{-1} in one column loop (leaf_device.hpp), by the wave
-//           that owns the row; X_cc to LDS
+//           that owns the row; X_cc to LDS.  The next column of A is read meanwhile
 //   panel:  L_ic = C_ic X_cc^T for the wave's rows below, the block's own rows to LDS
-//   update: C_ic' -= L_ic L_c'c^T, c' > c.
+//   update: S_ic' += L_ic L_c'c^T, c' > c.
 // The MFMA result layout (element r of lane l: row l%16, column kx(r, l/16)) is the operand layout of
 // k-step r of the next product, so C_ic feeds C_ic X_cc^T and L_ic the update from registers.
 // What used to bound this path was re-reading the system, 14 times its size (one wave per system,
 // left-looking by single tile columns: 26.6 GB a launch of 20,000 systems, 5.7 TB/s beyond L2):
 // with 64-column blocks held by the group a factor of 256 reads its finished columns about twice,
 // and a CU has 2 to 12 systems in flight instead of 8 of any size.  20,000 systems, n ~ U[8, 256]:
-// FP64 4.6 -> 3.5 ms, FP32 3.0 -> 2.2 ms; 700 systems FP64 0.60 -> 0.19 ms.  What bounds it now is
-// the chain of a system's steps (about 6.5k cycles per 16 columns with two workgroups on a CU: leaf,
+// FP64 4.6 -> 3.1 ms, FP32 3.0 -> 1.9 ms; 700 systems FP64 0.60 -> 0.20 ms.  What bounds it now is
+// the chain of a system's steps (about 6k cycles per 16 columns with two workgroups on a CU: leaf,
 // two barriers, panel, update; then 3.5k per step of each substitution), not memory: one workgroup
-// per CU takes 5.7 ms.
+// per CU takes 4.8 ms.
 // The substitutions run over the same blocks: the tiles of a block are dealt over the waves, each
 // sums the finished part on its own, and the block's 4 steps pass through LDS.  A partial last tile
 // is padded with the identity.
@@ -83,8 +86,9 @@ struct VbArith<float> {  // v_mfma_f32_16x16x4f32
 };
 
 // Workgroups per CU: FP64 holds 4 x 4 tiles in 128 registers a lane and two workgroups; FP32 fits
-// three, which measured 2.17 ms against 2.70 with two (20,000 systems).  FP64 blocks of two tile
-// columns with three workgroups measured 3.7 ms against 3.5.
+// three, which measured 1.96 ms against 2.40 with two (20,000 systems).  FP64 blocks of two tile
+// columns with three workgroups took 6% longer (3.7 ms, 3.5 then).  The compiler spills 21 (FP64) and
+// 40 (FP32) registers and 82 to 84 scalars, mostly at a system's start and end, none in the leaf.
 template <typename T>
 constexpr int kVbPerCu = sizeof(T) == 8 ? 2 : 3;
 
@@ -281,64 +285,75 @@ struct VbGroup {
                 else if (ns == 1)
                     accumulate<1>(C, A, lda, J, offp, offq);
             }
-            // A minus the sum: the tiles at and left of the diagonal (the strictly upper part of a
-            // diagonal tile is read but never used: every lane stops at its own diagonal entry).  The
-            // sum is formed by itself first: in FP32 it keeps its own rounding, not A's.
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
+            // A's tile column c of the block, this wave's tiles at and left of the diagonal (the strictly
+            // upper part of a diagonal tile is read but never used: every lane stops at its own diagonal
+            // entry).  Rows past n, rows above the diagonal and empty slots: a row that is read anyway.
+            // The loads are issued in front of the barrier that ends the leaf: behind it, a launch of 20,000
+            // took 0.15 ms longer in FP64; in front of the leaf, its registers spilled (6.8 ms a call against 4.8).
+            auto read_column = [&](T(&a)[4][4], int c) {
                 const int col = 16 * (4 * J + c);
                 if (col + 16 <= n) {
-                    T a[4][4];
+                    uint32_t off[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        off[r] = r < ns && r * W + w >= c ? offp[r] : offp[0];
+                        asm volatile("" : "+v"(off[r]));  // or each load gets branches of its own
+                    }
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const gptr<T> base = A + (int64_t)(col + M::step(e)) * lda;
-                        // rows above the block's diagonal and empty slots: a row that is read anyway
 #pragma unroll
-                        for (int r = 0; r < 4; ++r)
-                            a[r][e] = *elem_at(base, r < ns && r * W + w >= c ? offp[r] : offp[0]);
+                        for (int r = 0; r < 4; ++r) a[r][e] = *elem_at(base, off[r]);
                     }
+                } else {  // the last, partial tile column (its diagonal tile alone): columns past n - 1 read n - 1's
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
+                    for (int e = 0; e < 4; ++e) {
+                        const int i = col + li, cc = col + M::kx(e, g);
+                        const T x = A[(i < n ? i : n - 1) + (int64_t)(cc < n ? cc : n - 1) * lda];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) C[r][c][e] = a[r][e] - C[r][c][e];
-                } else if (c < nb) {  // the last, partial tile column: columns past n - 1 read n - 1's
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (r < ns && r * W + w == c) {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int i = col + li, cc = col + M::kx(e, g);
-                                C[r][c][e] = A[(i < n ? i : n - 1) + (int64_t)(cc < n ? cc : n - 1) * lda] - C[r][c][e];
-                            }
-                        }
+                        for (int r = 0; r < 4; ++r) a[r][e] = x;
+                    }
                 }
-            }
-            // rows past n: zero, the identity on the diagonal
+            };
+            // a <- A's column less S, the sum of all earlier columns' products, which is formed by itself: it
+            // keeps its own rounding, not A's.  Rows past n: zero, the identity on the diagonal.
+            auto subtract = [&](T(&a)[4][4], int c, int h) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int q = r * W + w, i = 16 * (4 * J + q) + li;
-                if (r < ns && 16 * (4 * J + q) + 16 > n) {
+                for (int r = 0; r < 4; ++r) {
+                    const int q = r * W + w;
 #pragma unroll
-                    for (int c = 0; c < 4; ++c)
+                    for (int e = 0; e < 4; ++e) a[r][e] -= C[r][h][e];
+                    if (r < ns && 16 * (4 * J + q) + 16 > n) {
+                        const int i = 16 * (4 * J + q) + li;
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
                             const int col = 16 * (4 * J + c) + M::kx(e, g);
-                            C[r][c][e] = i < n && col < n ? C[r][c][e] : (i == col ? one : zero);
+                            a[r][e] = i < n && col < n ? a[r][e] : (i == col ? one : zero);
                         }
+                    }
                 }
-            }
-            // this wave's diagonal tile of the block column at hand, in C[r][0]: to LDS for the leaf
-            auto give_leaf = [&](int c) {
+            };
+            // this wave's diagonal tile of the block column at hand: to LDS for the leaf
+            auto give_leaf = [&](const T(&a)[4][4], int c) {
                 T *xs = X + 16 * LS * (4 * J + c);
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     if (r * W + w == c) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) xs[LS * li + M::kx(e, g)] = C[r][0][e];
+                        for (int e = 0; e < 4; ++e) xs[LS * li + M::kx(e, g)] = a[r][e];
                     }
             };
-            give_leaf(0);
-            // the column at hand is always C[.][0]; the others move up after each
+            {
+                T a[4][4];
+                read_column(a, 0);
+                subtract(a, 0, 0);
+                give_leaf(a, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) C[r][0][e] = a[r][e];
+            }
+            // the column at hand is always C[.][0]; the others, sums so far, move up after each
 #pragma unroll 1
             for (int c = 0; c < nb; ++c) {
                 const int k = 4 * J + c, k0 = 16 * k;
@@ -363,6 +378,8 @@ struct VbGroup {
                         for (int m = 0; m < 16; ++m) xs[LS * li + m] = v[m];
                     }
                 }
+                T a[4][4] = {};  // the next column
+                if (c + 1 < nb) read_column(a, c + 1);  // in flight during the other waves' leaf and the panel
                 barrier();
                 {
                     const int f = __builtin_amdgcn_readfirstlane(sy->fail);
@@ -400,25 +417,28 @@ struct VbGroup {
                 if (c + 1 == nb) break;
                 barrier();
                 // ---- update, and the columns move up
-                T np[4][4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) np[r][e] = -C[r][0][e];
 #pragma unroll
                 for (int h = 1; h < 4; ++h) {  // tile column c + h
                     T pq[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) pq[e] = Y[256 * ((c + h) & 3) + 64 * e + l];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        C[r][h - 1] = C[r][h];
+                    for (int r = 0; r < 4; ++r)
                         if (r < ns && c + h < nb && r * W + w >= c + h) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) C[r][h - 1] = M::mma(pq[e], np[r][e], C[r][h - 1]);
+                            for (int e = 0; e < 4; ++e) C[r][h] = M::mma(pq[e], C[r][0][e], C[r][h]);
                         }
+                    if (h == 1) {
+                        subtract(a, c + 1, 1);
+                        give_leaf(a, c + 1);
                     }
-                    if (h == 1) give_leaf(c + 1);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) C[r][0][e] = a[r][e];
+                    C[r][1] = C[r][2];
+                    C[r][2] = C[r][3];
                 }
             }
             barrier_global();  // the next block reads this one's columns (and the panel tiles are free)

@@ -226,3 +226,88 @@ def test_vbatched_group_edges(dev, dtype):
             x = big.B(i)[:n].cpu().double().numpy()
             res = np.linalg.norm(asym @ x - b, axis=0) / (np.linalg.norm(asym) * np.linalg.norm(x, axis=0))
             assert res.max() <= (2e-6 * n / 16 if f32 else 1e-14), (i, n, rs[i], res.max())
+
+
+def _fma32(a, b, c):
+    """a b + c with one rounding to float32 (a product of two floats is exact in double)."""
+    return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
+
+
+def _factor32(a):
+    """Lower factors of a (m, n, n), n a multiple of 16, in float32 by tile columns of 16: A's column less
+    the sum over all earlier columns, formed by itself; the tile's column loop with the reciprocal square
+    root and one Newton step; the rows below by the tile's inverse."""
+    f32 = np.float32
+    m, n, _ = a.shape
+    out = np.zeros_like(a)
+    for k0 in range(0, n, 16):
+        s = np.zeros((m, n - k0, 16), f32)
+        for k in range(k0):
+            s = _fma32(out[:, k0:, k, None], out[:, None, k0:k0 + 16, k], s)
+        c = a[:, k0:, k0:k0 + 16] - s
+        u, v = c[:, :16].copy(), np.broadcast_to(np.eye(16, dtype=f32), (m, 16, 16)).copy()
+        for j in range(16):
+            x = u[:, j, j].copy()
+            r = (1 / np.sqrt(x.astype(np.float64))).astype(f32)
+            r = r * _fma32(-(f32(0.5) * x * r), r, np.full_like(x, 1.5))
+            u[:, :, j] *= r[:, None]
+            v[:, :, j] *= r[:, None]
+            for i in range(j + 1, 16):
+                v[:, :, i] = _fma32(-u[:, i, j, None], v[:, :, j], v[:, :, i])
+                u[:, :, i] = _fma32(-u[:, i, j, None], u[:, :, j], u[:, :, i])
+        out[:, k0:k0 + 16, k0:k0 + 16] = np.tril(u)
+        p = np.zeros((m, n - k0 - 16, 16), f32)
+        for k in range(16):  # v[i][k] is the inverse's [k][i]
+            p = _fma32(c[:, 16:, k, None], v[:, k, None, :], p)
+        out[:, k0 + 16:, k0:k0 + 16] = p
+    return out
+
+
+@pytest.mark.parametrize("n,count", [(64, 200), (128, 60), (200, 30)])
+def test_vbatched_float_sums_keep_their_own_rounding(dev, n, count):
+    """The error of the single precision factor (one, two and four waves a system) against 64 bits is no
+    more than 1.1 times that of the same arithmetic on the CPU with each column's sum formed by itself and
+    subtracted from A once.  Products added to A one by one, within a block of 64 columns, would be
+    rounded at A's magnitude: 1.5 times at n = 64 by the same emulation."""
+    print(f"[gpu] float sums n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    g = rng.standard_normal((count, n, n))
+    a = (g @ g.swapaxes(1, 2) / n + 0.1 * np.eye(n)).astype(np.float32)
+    a = np.tril(a) + np.tril(a, -1).swapaxes(1, 2)
+    vb = batched.VBatch([n] * count, [0] * count, dtype=torch.float32, device=dev)
+    for i in range(count):
+        vb.A(i).copy_(torch.from_numpy(a[i]))
+    assert int(batched.posv_vbatched_(vb, mi_llt.Handle()).abs().sum()) == 0
+    got = np.stack([np.tril(vb.A(i).cpu().numpy()) for i in range(count)]).astype(np.float64)
+    want = np.linalg.cholesky(a.astype(np.float64))
+    pad = -n % 16
+    ap = np.zeros((count, n + pad, n + pad), np.float32)
+    ap[:, :n, :n] = a
+    ap[:, range(n, n + pad), range(n, n + pad)] = 1
+    emu = _factor32(ap)[:, :n, :n].astype(np.float64)
+    assert np.linalg.norm(got - want) <= 1.1 * np.linalg.norm(emu - want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_vbatched_leaves_everything_else(dev, dtype):
+    """Bytes outside the lower triangles and the right-hand sides -- the strictly upper triangles, the rows
+    from n on of A and of B -- stay as they were, at the edges of tiles, blocks and groups."""
+    ns = [1, 15, 16, 17, 48, 63, 64, 65, 127, 128, 129, 177, 193, 255, 256]
+    pads = [(3 * i + 1) % 5 for i in range(len(ns))]
+    rs = [(1, 16, 17)[i % 3] for i in range(len(ns))]
+    vb = batched.VBatch([n + p for n, p in zip(ns, pads)], rs, dtype=dtype, device=dev)
+    vb.d_n.copy_(torch.tensor(ns, dtype=torch.int32))
+    gen = torch.Generator(device=dev).manual_seed(4)
+    vb.a_flat.copy_(torch.randn(vb.a_flat.numel(), device=dev, generator=gen))
+    vb.b_flat.copy_(torch.randn(vb.b_flat.numel(), device=dev, generator=gen))
+    for i, n in enumerate(ns):
+        spd = torch.from_numpy(workloads.gram_spd(n, seed=80 + i)).to(dev).to(dtype)
+        vb.A(i)[:n, :n] = torch.where(torch.ones(n, n, device=dev).tril().bool(), spd, vb.A(i)[:n, :n])
+    a0, b0 = [vb.A(i).clone() for i in range(len(ns))], [vb.B(i).clone() for i in range(len(ns))]
+    assert int(batched.posv_vbatched_(vb, mi_llt.Handle()).abs().sum()) == 0
+    for i, n in enumerate(ns):
+        keep = torch.ones(n + pads[i], n + pads[i], device=dev).tril().bool()
+        keep[n:], keep[:, n:] = False, False  # the system's lower triangle
+        assert torch.equal(torch.where(keep, a0[i], vb.A(i)), a0[i]), n
+        assert torch.equal(vb.B(i)[n:], b0[i][n:]), n
+        assert bool((vb.B(i)[:n] != b0[i][:n]).any()), n
