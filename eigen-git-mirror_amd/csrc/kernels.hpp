@@ -143,10 +143,8 @@ void launch_add_in_place(double *X, int64_t ldx, const double *D, int64_t ldd, i
                          hipStream_t s);
 
 // Batched uneven factor + solve (vbatched.hip): plan (argument checks, queues by order) + one
-// persistent launch of `grid` workgroups (vb_workgroups_per_cu fit a CU).  plan: vb_plan_bytes(batch) bytes.
+// persistent launch of `grid` workgroups.  plan: vb_plan_bytes(batch) bytes.
 int64_t vb_plan_bytes(int64_t batch);
-template <typename T>
-int vb_workgroups_per_cu();
 template <typename T>
 void launch_vbatched(int64_t batch, const int *d_n, T *const *d_A, const int *d_lda, const int *d_nrhs,
                      T *const *d_B, const int *d_ldb, int *d_info, void *plan, int grid, int lpt, hipStream_t s);

@@ -743,14 +743,6 @@ void launch_vbatched(int64_t batch, const int *d_n, T *const *d_A, const int *d_
     hipLaunchKernelGGL(vb_persistent_kernel<T>, dim3(grid), dim3(256), 0, s, desc, queue, d_info);
 }
 
-template <typename T>
-int vb_workgroups_per_cu()
-{
-    return kVbPerCu<T>;
-}
-template int vb_workgroups_per_cu<double>();
-template int vb_workgroups_per_cu<float>();
-
 template void launch_vbatched<double>(int64_t, const int *, double *const *, const int *, const int *,
                                       double *const *, const int *, int *, void *, int, int, hipStream_t);
 template void launch_vbatched<float>(int64_t, const int *, float *const *, const int *, const int *, float *const *,

@@ -232,8 +232,7 @@ int mi_dposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n,
 int mi_sposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n, float *const *d_A,
                       const int *d_lda, const int *d_nrhs, float *const *d_B, const int *d_ldb, int *d_info);
 /* Schedule of the batched launch (no reference counterpart; set by the autotuner in
- * mi_llt.batched): workgroups of 4 waves launched per CU (1..64; until it is set, as many as fit
- * a CU: 2 for FP64, 3 for FP32), a register-block size (0, 2 or 4; accepted and kept, the kernel's
+ * mi_llt.batched): workgroups of 4 waves launched per CU (1..64; 3 until it is set), a register-block size (0, 2 or 4; accepted and kept, the kernel's
  * blocks are fixed per precision), and longest-first ordering within the size classes (1) or the
  * given order (0). */
 int mi_llt_set_vbatched_config(mi_llt_handle h, int wg_per_cu, int group, int longest_first);

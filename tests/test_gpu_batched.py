@@ -228,6 +228,17 @@ def test_vbatched_group_edges(dev, dtype):
             assert res.max() <= (2e-6 * n / 16 if f32 else 1e-14), (i, n, rs[i], res.max())
 
 
+def test_vbatched_schedule_round_trip(dev):
+    """What a handle reports is what it launches by: saving a schedule and setting it again changes
+    nothing, a new handle's included."""
+    h = mi_llt.Handle()
+    assert batched.get_config(h) == (3, 0, True)  # the default of both precisions
+    batched.set_config(h, *batched.get_config(h))
+    assert batched.get_config(h) == (3, 0, True)
+    batched.set_config(h, 2, 4, False)
+    assert batched.get_config(h) == (2, 4, False)
+
+
 def _fma32(a, b, c):
     """a b + c with one rounding to float32 (a product of two floats is exact in double)."""
     return (a.astype(np.float64) * b.astype(np.float64) + c.astype(np.float64)).astype(np.float32)
