@@ -110,7 +110,9 @@ def get_config(handle: Handle) -> tuple:
     return int(a.value), int(b.value), bool(c.value)
 
 
-CANDIDATES = [(w, g, o) for w in (1, 2, 3, 4) for g in (2, 4) for o in (True, False)]
+CANDIDATES = [(w, 0, o) for w in (1, 2, 3, 4) for o in (True, False)]
+# Part of a cached schedule's key: a schedule timed for another kernel says nothing about this one.
+KERNEL = "groups-of-waves"
 CACHE = os.path.join(os.path.expanduser("~"), ".cache", "mi_llt_vbatched.json")
 
 
@@ -121,9 +123,9 @@ def autotune(vb: VBatch, handle: Handle | None = None, candidates=None, reps: in
     Each candidate (wg_per_cu, group, longest_first) runs ``reps`` times on a scratch copy
     of the batch (``restore`` re-creates the inputs; by default the flat buffers are copied
     back before each run) and is timed with events; the best median wins.  Returns
-    ``{"config": best, "times_ms": {candidate: median}}``; cached per batch signature."""
+    ``{"config": best, "times_ms": {candidate: median}}``; cached per batch signature and kernel."""
     h = handle.bind_stream() if handle else default_handle()
-    key = vb.signature()
+    key = f"{vb.signature()}-{KERNEL}"
     if cache and os.path.exists(cache):
         try:
             table = json.load(open(cache))

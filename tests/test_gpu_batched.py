@@ -5,6 +5,8 @@ and LLT::_solve_impl (oracle/llt_oracle.c) on the same input: the factor within 
 relative to ||L||, solve backward error <= 1e-14 (FP64); FP32 against the FP64 oracle within
 FP32 bounds.  Failing pivots, argument errors, the upper triangle left untouched, the
 longest-first schedule, graph replay and the autotuner are covered too."""
+import json
+
 import numpy as np
 import pytest
 import torch
@@ -237,6 +239,19 @@ def test_vbatched_schedule_round_trip(dev):
     assert batched.get_config(h) == (3, 0, True)
     batched.set_config(h, 2, 4, False)
     assert batched.get_config(h) == (2, 4, False)
+
+
+def test_vbatched_autotune_ignores_another_kernels_cache(dev, tmp_path):
+    """A schedule cached under the batch's signature alone was timed for an earlier kernel: it is not
+    applied, and the new one is kept under a key of its own."""
+    vb = batched.gram_batch(16, nmin=8, nmax=64, seed=3)
+    path = tmp_path / "tune.json"
+    path.write_text(json.dumps({vb.signature(): {"config": [1, 4, False], "times_ms": {}}}))
+    h = mi_llt.Handle()
+    out = batched.autotune(vb, h, candidates=[(2, 0, True)], reps=1, cache=str(path))
+    assert out["config"] == [2, 0, True] and batched.get_config(h) == (2, 0, True)
+    assert len(json.loads(path.read_text())) == 2
+    assert len(batched.CANDIDATES) == len({(w, o) for w, _, o in batched.CANDIDATES})  # group: no effect
 
 
 def _fma32(a, b, c):
