@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256, MI_FACTOR_WG_PER_CU) void factor_step_kernel(S
         uint32_t *helped = tickets + (kSyncHelped - kSyncFactorTickets);
         if constexpr (sizeof(S) == 8) {
             if (t >= 1 && t <= nh) {
-                diag_helper(t - 1, A, lda, n, kp, helped, epoch);
+                diag_helper(t - 1, A, lda, n, kp, Wleaf, helped, epoch);
                 return;
             }
         }

@@ -168,6 +168,13 @@ __device__ __forceinline__ void image_store(double *p, double v)
 // 1979, 1850 and 1735 us.
 constexpr int kPart1 = 4, kPart2 = 6;
 
+// Where diag_helper leaves tile (i, j), i >= j, of the updated diagonal block in the panel image (lane
+// order: elements l + 64 r): the places that L's tile and leaf j's inverse take when panel j is stored.
+__device__ __forceinline__ constexpr int helper_tile(int i, int j)
+{
+    return i == j ? (int)kLeafOffset + 256 * j : 256 * ((i * (i - 1)) / 2 + j);
+}
+
 // Cholesky of the 128 x 128 lower block in S (all 256 threads), in eight 16-column panels with
 // a one-panel lookahead inside the block.  After panel p is factored, with T = 7-p tile rows
 // below it and their operands P_x = tile (p+1+x, p), x < T:
@@ -184,19 +191,19 @@ constexpr int kPart1 = 4, kPart2 = 6;
 // to no use (a test of the failure in each panel took longer).  xs: 2 x 256 doubles of LDS, s_fail: an
 // LDS int.
 //
-// Akk: null when S holds the whole block; else S has tile columns 0 and 1 of it, and the others are
-// read from Akk (ld lda, order bs, identity beyond), each one phase ahead, columns 2, 3 and 4 .. 7 once
-// helped[0] and helped[1] have reached `epoch` (diag_helper).
-__device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, double *__restrict__ W, uint32_t *flag,
-                                            const double *Akk, int64_t lda, int bs, const uint32_t *helped,
-                                            uint32_t epoch, int *status)
+// helped: null when S holds the whole block; else S has tile columns 0 and 1 of it, and the others are
+// read from the image (helper_tile), each one phase ahead, columns 2, 3 and 4 .. 7 once helped[0] and
+// helped[1] have reached `epoch` (diag_helper).  Tile (i, j) is read in B(j - 3) and used in B(j - 2), so
+// the panel's own tile can take its place in B(j).
+__device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, double *W, uint32_t *flag,
+                                            const uint32_t *helped, uint32_t epoch, int *status)
 {
     const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = lane_id();
     double *Xl = W + kLeafOffset;
     double lv[16];
     double next[3][4];  // waves 2 and 3: this wave's tiles (i, j), i = j + w - 2, + 2, + 4, of the next column
     auto fetch = [&](int j) {
-        if (Akk && (j == 2 || j == 4)) {
+        if (helped && (j == 2 || j == 4)) {
             uint32_t spins = 0;
             while (__hip_atomic_load(helped + (j == 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < epoch) {
                 __builtin_amdgcn_s_sleep(1);
@@ -211,13 +218,9 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, 
         for (int x = 0; x < 3; ++x) {
             const int i = j + w - 2 + 2 * x;
             if (i < 8) {
-                if (Akk) {
-                    const int gi = 16 * i + (l & 15), ci = gi < bs ? gi : bs - 1;
+                if (helped) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int gj = 16 * j + 4 * r + (l >> 4), cj = gj < bs ? gj : bs - 1;
-                        next[x][r] = coherent_load(Akk + ci + (int64_t)cj * lda);
-                    }
+                    for (int r = 0; r < 4; ++r) next[x][r] = coherent_load(W + helper_tile(i, j) + l + 64 * r);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) next[x][r] = S[256 * ((i * (i + 1)) / 2 + j) + l + 64 * r];
@@ -275,10 +278,7 @@ __device__ __forceinline__ int potrf_in_lds(double *S, double *xs, int *s_fail, 
 #pragma unroll
             for (int x = 0; x < 3; ++x)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int gi = 16 * (i0 + 2 * x) + (l & 15), gj = 16 * j + 4 * r + (l >> 4);
-                    C[x][r] = !Akk || (gi < bs && gj < bs) ? next[x][r] : gi == gj ? 1.0 : 0.0;
-                }
+                for (int r = 0; r < 4; ++r) C[x][r] = next[x][r];
             // Panel p to the image, tile rows p + 1 + w - 2, + 2, ..., and its leaf's inverse; then the next
             // column's loads.  In front of the products, so that the next phase, which waits for all of
             // them when it takes up `next`, finds them done.
@@ -520,12 +520,12 @@ __device__ __forceinline__ void trsm_rows(double *smem, int *s_seen, T *__restri
 }
 
 // FP64 update of tile columns [C0, C1) of the diagonal block, A_kk - P_0 P_0^T, for tile rows W and
-// 7-W, their tiles at and left of the diagonal, with acc starting from A_kk: to S (identity beyond bs; a
-// diagonal tile is written whole, its upper entries are never read as data) for C0 = 0, written
-// through to A_kk (its lower entries) for the others.
+// 7-W, their tiles at and left of the diagonal, with acc starting from A_kk: to S for C0 = 0, to the panel
+// image (helper_tile, written through) for the others.  Identity beyond bs; a diagonal tile is written
+// whole, its upper entries are never read as data.
 template <int W, int C0, int C1>
-__device__ __forceinline__ void diag_update_f64(double *S, double *__restrict__ Akk, const double *__restrict__ P0,
-                                                int64_t lda, int bs)
+__device__ __forceinline__ void diag_update_f64(double *S, const double *__restrict__ Akk,
+                                                const double *__restrict__ P0, int64_t lda, int bs)
 {
     constexpr uint32_t kCols = ((1u << C1) - 1u) & ~((1u << C0) - 1u);
     constexpr uint32_t kActive = (((1u << (W + 1)) - 1u) & kCols) | ((((1u << (8 - W)) - 1u) & kCols) << 8);
@@ -543,20 +543,21 @@ __device__ __forceinline__ void diag_update_f64(double *S, double *__restrict__ 
 #pragma unroll
         for (int b = 0; b < 8; ++b)
             if (t.on(a, b)) {
-                double *C = S + 256 * ((ti * (ti + 1)) / 2 + b) + l;
+                double *C = S + (C0 == 0 ? 256 * ((ti * (ti + 1)) / 2 + b) : helper_tile(ti, b)) + l;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = 16 * ti + (l & 15), j = 16 * b + 4 * r + (l >> 4);
+                    const double v = (i < bs && j < bs) ? t.acc[a][b][r] : (i == j ? 1.0 : 0.0);
                     if (C0 == 0)
-                        C[64 * r] = (i < bs && j < bs) ? t.acc[a][b][r] : (i == j ? 1.0 : 0.0);
-                    else if (i < bs && j <= i)
-                        image_store(Akk + i + (int64_t)j * lda, t.acc[a][b][r]);
+                        C[64 * r] = v;
+                    else
+                        image_store(C + 64 * r, v);
                 }
             }
     }
 }
 template <int C0, int C1>
-__device__ __forceinline__ void diag_update_columns(int w, double *S, double *__restrict__ Akk,
+__device__ __forceinline__ void diag_update_columns(int w, double *S, const double *__restrict__ Akk,
                                                     const double *__restrict__ P0, int64_t lda, int bs)
 {
     switch (w) {
@@ -610,6 +611,27 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
     }
 }
 
+// Helper h of the diagonal role (FP64, k0 > 0): tile columns 2, 3 (h = 0) or 4 .. 7 of A_kk - P_0 P_0^T
+// to the panel image (A_kk itself stays as it is until the block is factored, also when a pivot fails), then
+// helped[h] = epoch.  The update's 36 tiles are 18400 cycles of MFMA on one CU, in front
+// of everything else on the chain; the diagonal role computes the 15 tiles of columns 0 and 1 and needs
+// column 2 a panel's time later, column 4 three panels' time.
+__device__ __forceinline__ void diag_helper(int h, const double *__restrict__ A, int64_t lda, int64_t n, int64_t k0,
+                                            double *__restrict__ Wleaf, uint32_t *helped, uint32_t epoch)
+{
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int bs = (int)((n - k0) < 128 ? (n - k0) : 128);
+    const double *Akk = A + k0 + k0 * lda;
+    const double *P0 = A + k0 + (k0 - 128) * lda;
+    double *Wp = Wleaf + (size_t)(k0 / 128) * kPanelDoubles;
+    if (h == 0)
+        diag_update_columns<2, 4>(w, Wp, Akk, P0, lda, bs);
+    else
+        diag_update_columns<4, 8>(w, Wp, Akk, P0, lda, bs);
+    global_barrier();  // every wave's stores are in memory
+    if (threadIdx.x == 0) __hip_atomic_store(helped + h, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // The panel role of one block step; g is the role from the ticket, less the nh helpers' (diag_helper):
 //   role 0   : C = A_kk - P_0 P_0^T straight into LDS, Cholesky in LDS, the panel image
 //              (L11's strictly lower tiles and the leaf inverses) to the workspace, published by
@@ -623,25 +645,6 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
 // (the diagonal factor and the panel solve are FP64 for every T).  With T = double the row
 // role keeps its rows in registers from the update to the store; with T = float the update
 // is rounded to FP32 storage first (as the mixed-precision trailing updates are) and read back.
-// Helper h of the diagonal role (FP64, k0 > 0): tile columns 2, 3 (h = 0) or 4 .. 7 of A_kk - P_0 P_0^T
-// into A_kk, then helped[h] = epoch.  The update's 36 tiles are 18400 cycles of MFMA on one CU, in front
-// of everything else on the chain; the diagonal role computes the 15 tiles of columns 0 and 1 and needs
-// column 2 a panel's time later, column 4 three panels' time.
-__device__ __forceinline__ void diag_helper(int h, double *__restrict__ A, int64_t lda, int64_t n, int64_t k0,
-                                            uint32_t *helped, uint32_t epoch)
-{
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int bs = (int)((n - k0) < 128 ? (n - k0) : 128);
-    double *Akk = A + k0 + k0 * lda;
-    const double *P0 = A + k0 + (k0 - 128) * lda;
-    if (h == 0)
-        diag_update_columns<2, 4>(w, nullptr, Akk, P0, lda, bs);
-    else
-        diag_update_columns<4, 8>(w, nullptr, Akk, P0, lda, bs);
-    global_barrier();  // every wave's stores are in memory
-    if (threadIdx.x == 0) __hip_atomic_store(helped + h, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 template <typename T, int PREC>
 __device__ __forceinline__ void panel_role(int g, int nh, double *smem, int *s_ok, T *__restrict__ A,
                                            int64_t lda, int64_t n, int64_t k0, double *__restrict__ Wleaf, int *info,
@@ -670,9 +673,7 @@ __device__ __forceinline__ void panel_role(int g, int nh, double *smem, int *s_o
         } else {
             block_to_lds(smem, Ck, lda, bs);
         }
-        const double *Akk = nullptr;
-        if constexpr (sizeof(T) == 8) Akk = nh ? Ck : nullptr;
-        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag, Akk, lda, bs, helped, epoch, status);  // a barrier first
+        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag, nh ? helped : nullptr, epoch, status);  // a barrier first
         if (f >= 0 && tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
         global_barrier();  // every wave's stores of the image are in memory
         if (tid == 0) __hip_atomic_store(flag, 8 * epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

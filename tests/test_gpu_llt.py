@@ -266,6 +266,28 @@ def test_l1_norm_tiles(dev, n, uplo, dtype):
 
 
 
+@pytest.mark.parametrize("n,col", [(300, 200), (300, 129), (256, 255), (200, 150), (130, 129)])
+@pytest.mark.parametrize("count", [1, 16, 17])
+def test_failing_block_keeps_its_input(dev, n, col, count):
+    """A pivot that fails in the second block column leaves that column (its diagonal block and the rows
+    below, to which no earlier launch writes) as it came, for one system and for any batch: the diagonal
+    role's helpers work on a copy."""
+    say(f"[gpu] failing block n={n} column {col} batch {count}")
+    a = workloads.indefinite_at(n, col, seed=n + col)
+    da = mi_llt.colmajor_batched(torch.from_numpy(np.repeat(a[None], count, 0)).to(dev))
+    info = torch.zeros(count, dtype=torch.int32, device=dev)
+    mi_llt.potrf_batched_async_(da, info)
+    torch.cuda.synchronize()
+    assert info.tolist() == [col + 1] * count
+    block = np.tril(a)[128:, 128:256]
+    for m in da.cpu().numpy():
+        np.testing.assert_array_equal(np.tril(m)[128:, 128:256], block)
+    if count == 1:
+        m, i = gpu_factor(a, dev)
+        assert i == col + 1
+        np.testing.assert_array_equal(np.tril(m)[128:, 128:256], block)
+
+
 def test_llt_object_mirror(dev):
     say("[gpu] LLT object")
     n = 260
