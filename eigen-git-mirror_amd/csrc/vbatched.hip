@@ -627,7 +627,8 @@ __global__ __launch_bounds__(256, kVbPerCu<T>) void vb_persistent_kernel(const V
 }
 
 // Plan: every system's arguments checked (its info set), the valid ones sorted into the queues,
-// longest first within a queue (lpt: the tail of the launch stays short) or in the given order.
+// longest first within a queue (lpt: the tail of the launch stays short) or in the given order; systems of
+// one bucket keep the given order in both.
 // Two launches of one workgroup per kVbPlan systems: each counts its systems per bucket (tile
 // count, longest first; lpt = 0: per mode), then each places its own behind the earlier workgroups'.
 constexpr int kVbBuckets = kVbMaxT + 1;
@@ -675,7 +676,7 @@ __global__ __launch_bounds__(kVbPlan) void vb_place_kernel(int64_t batch, const 
                                                            VbDesc *__restrict__ desc, VbQueue *__restrict__ queue,
                                                            int lpt)
 {
-    __shared__ int total[kVbBuckets], before[kVbBuckets], start[kVbBuckets + 1];
+    __shared__ int total[kVbBuckets], before[kVbBuckets], start[kVbBuckets + 1], waves[kVbPlan / 64][kVbBuckets];
     const int tid = threadIdx.x;
     if (tid < kVbBuckets) total[tid] = before[tid] = 0;
     __syncthreads();
@@ -704,20 +705,33 @@ __global__ __launch_bounds__(kVbPlan) void vb_place_kernel(int64_t batch, const 
         if (tid < 3 * 8) queue->next[tid / 8][tid % 8][0] = 0;
     }
     if (tid < kVbBuckets) before[tid] += start[tid];
-    __syncthreads();
     const int64_t i = (int64_t)blockIdx.x * kVbPlan + tid;
-    if (i >= batch) return;
     VbDesc d;
-    d.n = d_n[i];
-    d.lda = d_lda[i];
-    d.nrhs = d_nrhs[i];
-    d.ldb = d_ldb[i];
-    if (vb_check(d.n, d.lda, d.nrhs, d.ldb)) return;
-    d.a = (uint64_t)(uintptr_t)d_A[i];
-    d.b = (uint64_t)(uintptr_t)d_B[i];
-    d.index = (int)i;
-    d.pad[0] = d.pad[1] = d.pad[2] = 0;
-    desc[atomicAdd(&before[vb_bucket(d.n, lpt)], 1)] = d;
+    int bucket = -1;  // none: past the end, or arguments out of range
+    if (i < batch) {
+        d.n = d_n[i];
+        d.lda = d_lda[i];
+        d.nrhs = d_nrhs[i];
+        d.ldb = d_ldb[i];
+        d.a = (uint64_t)(uintptr_t)d_A[i];
+        d.b = (uint64_t)(uintptr_t)d_B[i];
+        d.index = (int)i;
+        d.pad[0] = d.pad[1] = d.pad[2] = 0;
+        if (!vb_check(d.n, d.lda, d.nrhs, d.ldb)) bucket = vb_bucket(d.n, lpt);
+    }
+    // the systems of the bucket in front of this one: in its wave, then in the earlier waves
+    const int l = lane_id(), w = tid >> 6;
+    int rank = 0;
+#pragma unroll
+    for (int b = 0; b < kVbBuckets; ++b) {
+        const uint64_t same = __ballot(bucket == b);
+        if (bucket == b) rank = __popcll(same & ((1ull << l) - 1));
+        if (l == b) waves[w][b] = __popcll(same);
+    }
+    __syncthreads();
+    if (bucket < 0) return;
+    for (int v = 0; v < w; ++v) rank += waves[v][bucket];
+    desc[before[bucket] + rank] = d;
 }
 
 constexpr int64_t kVbQueueBytes = ((int64_t)sizeof(VbQueue) + 255) / 256 * 256;

@@ -5,6 +5,7 @@ and LLT::_solve_impl (oracle/llt_oracle.c) on the same input: the factor within 
 relative to ||L||, solve backward error <= 1e-14 (FP64); FP32 against the FP64 oracle within
 FP32 bounds.  Failing pivots, argument errors, the upper triangle left untouched, the
 longest-first schedule, graph replay and the autotuner are covered too."""
+import ctypes
 import json
 
 import numpy as np
@@ -239,6 +240,39 @@ def test_vbatched_schedule_round_trip(dev):
     assert batched.get_config(h) == (3, 0, True)
     batched.set_config(h, 2, 4, False)
     assert batched.get_config(h) == (2, 4, False)
+
+
+@pytest.mark.parametrize("batch", [1, 63, 1024, 1025, 5000])
+@pytest.mark.parametrize("lpt", [0, 1])
+def test_vbatched_queue_keeps_given_order(dev, batch, lpt):
+    """The plan's queues (the last batch x 48 bytes of the plan, a system's index at byte 32): systems of
+    one size class -- with longest first, of one tile count -- stand in the given order, and systems with
+    bad arguments in none."""
+    rng = np.random.default_rng(batch)
+    ns = rng.integers(0, 257, size=batch)
+    vb = batched.VBatch(ns, rng.integers(0, 3, size=batch))
+    vb.a_flat.fill_(0.0)
+    for i in range(batch):  # identity matrices
+        vb.A(i).diagonal().fill_(1.0) if ns[i] else None
+    bad = rng.random(batch) < 0.1
+    n_arg = torch.from_numpy(np.where(bad, -1, ns).astype(np.int32)).to(dev)
+    L = mi_llt.lib()
+    plan_bytes = getattr(L, "_ZN2mi13vb_plan_bytesEl")  # mi::vb_plan_bytes, mi::launch_vbatched<double>
+    plan_bytes.restype, plan_bytes.argtypes = ctypes.c_int64, [ctypes.c_int64]
+    launch = getattr(L, "_ZN2mi15launch_vbatchedIdEEvlPKiPKPT_S2_S2_S6_S2_PiPviiP12ihipStream_t")
+    vp = ctypes.c_void_p
+    launch.restype, launch.argtypes = None, [ctypes.c_int64] + [vp] * 8 + [ctypes.c_int] * 2 + [vp]
+    plan = torch.zeros(plan_bytes(batch), dtype=torch.uint8, device=dev)
+    launch(batch, *(vp(t.data_ptr()) for t in (n_arg, vb.d_A, vb.d_lda, vb.d_nrhs, vb.d_B, vb.d_ldb, vb.d_info, plan)),
+           min(batch, 256), lpt, vp(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    nt = (ns + 15) // 16
+    key = -nt if lpt else np.digitize(-nt, [-8, -4], right=False)  # orders up to 256, 128, 64
+    good = np.nonzero(~bad)[0]
+    want = good[np.argsort(key[good], kind="stable")]
+    got = plan.cpu().numpy()[-48 * batch:].reshape(batch, 48)[:len(good), 32:36].copy().view(np.int32)[:, 0]
+    np.testing.assert_array_equal(got, want)
+    assert vb.d_info.tolist() == np.where(bad, -1, 0).tolist()
 
 
 def test_vbatched_autotune_ignores_another_kernels_cache(dev, tmp_path):
