@@ -29,8 +29,9 @@
 //
 // The first workgroups and those past the tiles are the panel's: they take its roles from a ticket
 // counter, the first to start the diagonal role (the critical path, always running before anyone waits
-// for it), the next two its helpers (FP64), the others the row roles -- which wait for the diagonal block, so they come last in the
-// grid and do not hold CUs while it is being factored.  The workgroups between are the trailing
+// for it), the next two its helpers (FP64, up to 64 systems), the others the row roles -- which wait for
+// the diagonal block, so they come last in the grid and do not hold CUs while it is being factored.  The
+// workgroups between are the trailing
 // update's tiles, by their place in the grid: with a ticket for each, the last of the 512 that start
 // together came 9 us late (17.5 ns an atomic on one address), 6282 against 6120 us at n = 8192 and
 // 14.2 against 13.85 ms in the FP32-storage factor at n = 16384.  (Raised wave priorities for the
@@ -288,10 +289,13 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
                         hipStream_t s, uint32_t *grid_out, int prec, __bf16 *Wsplit, const Batch &bt)
 {
     const int64_t below = n - kp - kNB;  // rows below the panel's diagonal block
-    // Helpers of the diagonal role (diag_helper), while the launch waits for one system's panel: a large
-    // batch's diagonal roles fill the chip by themselves (120 systems of order 512: 1600 us for the
-    // Gaussian processes without, 1665 with).
-    const int nh = sizeof(S) == 8 && kp > 0 && bt.count <= 16 ? 2 : 0;
+    // Helpers of the diagonal role (diag_helper), while each diagonal role and helper has a CU of its own:
+    // three a system, so the chip holds those of 85.  A factorization in us, without and with them:
+    //   systems     1          16         32         64         96
+    //   n = 256     77  72     79  74     79  74     76  73     86  92
+    //   n = 512    158 141    162 143    169 151    206 195    260 274
+    //   n = 1024   299 262    382 350    515 512    878 866   1213 1226
+    const int nh = sizeof(S) == 8 && kp > 0 && bt.count <= 64 ? 2 : 0;
     const int Gp = kp < 0 ? 0 : 1 + nh + (below > 0 ? (int)((below + 64 * kRowTiles - 1) / (64 * kRowTiles)) : 0);
     int c0 = 0, nsyrk = 0, K = k >= 1 ? 256 : 128, KQ = 0, cq0 = 0, co0 = 0, nko = 0;
     int64_t slab = k >= 1 ? (k - 1) * kNB : 0, slabq = 0, slabo = 0;

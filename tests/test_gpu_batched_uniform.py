@@ -218,6 +218,22 @@ def test_large_batch_factor_is_the_single_one(dev, n):
         assert torch.equal(one, l[z]), z
 
 
+@pytest.mark.parametrize("batch", [17, 64, 65])
+@pytest.mark.parametrize("n", [130, 300])
+def test_factor_with_and_without_helpers(dev, n, batch):
+    """Up to 64 systems the diagonal roles have helpers, beyond none: every system of both is the
+    single-system factor, bit for bit."""
+    say(f"[gpu] batched factor n={n} batch={batch}")
+    a, mats = stack(n, batch, seed=3 * n)
+    info = torch.full((batch,), 99, dtype=torch.int32, device=dev)
+    mi_llt.potrf_batched_async_(a, info)
+    assert info.tolist() == [0] * batch
+    for z in range(batch):
+        l1 = mi_llt.colmajor(torch.from_numpy(mats[z]).to(dev))
+        assert mi_llt.potrf_(l1) == 0
+        assert torch.equal(a[z], l1), f"factor of system {z} differs"
+
+
 def test_batched_argument_errors(dev):
     h = mi_llt.default_handle()
     L = mi_llt.lib()

@@ -267,7 +267,7 @@ def test_l1_norm_tiles(dev, n, uplo, dtype):
 
 
 @pytest.mark.parametrize("n,col", [(300, 200), (300, 129), (256, 255), (200, 150), (130, 129)])
-@pytest.mark.parametrize("count", [1, 16, 17])
+@pytest.mark.parametrize("count", [1, 16, 17, 64, 65])
 def test_failing_block_keeps_its_input(dev, n, col, count):
     """A pivot that fails in the second block column leaves that column (its diagonal block and the rows
     below, to which no earlier launch writes) as it came, for one system and for any batch: the diagonal
