@@ -30,9 +30,9 @@ struct mi_llt_context {
     size_t ws_bytes = 0;
     int *d_info = nullptr;    // device int for the synchronous entry points
     // synchronisation words (status, solve and rank-update tickets, factor tickets, panel flag
-    // at the mi::kSync* offsets, each group on its own cache line); zeroed on the handle's stream when allocated; the ticket and flag words of a solve or a
-    // factorization are reset on the stream at its start, so every call (and every replay of a
-    // captured call) counts from zero
+    // at the mi::kSync* offsets, each group on its own cache line); zeroed on the handle's stream
+    // when allocated; the ticket and flag words of a solve or a factorization are reset on the
+    // stream at its start, so every call (and every replay of a captured call) counts from zero
     uint32_t *sync = nullptr;
     size_t sync_words = 0;
     double *ypk = nullptr;       // the solve's packed copies of finished blocks (grow-only)

@@ -17,8 +17,8 @@
 
 namespace mi {
 
-// Zeroes the ticket counter and the panel flag (sync[kSyncFactorTickets], sync[kSyncFlag]) on
-// the stream: a kernel, not a memset, so that a captured factorization replays it
+// Zeroes the ticket counter, the helpers' words and the panel flag (sync[kSyncFactorTickets],
+// [kSyncHelped], [kSyncFlag]) on the stream: a kernel, not a memset, so that a captured factorization replays it
 // (factor_step.hip).
 void launch_factor_reset(uint32_t *sync, hipStream_t s, const Batch &bt = Batch());
 
@@ -50,8 +50,8 @@ inline double panel_flops(int64_t n, int64_t k0, int64_t NB)
 }
 
 // Queues the factorization of the lower triangle of A (n x n, ld lda) on stream s.
-// sync: the synchronisation words whose ticket counter and panel flag the factorization uses
-// (at kSyncFactorTickets, kSyncFlag); status: the status word; wleaf: the panel images
+// sync: the synchronisation words whose ticket counter, helpers' words and panel flag the factorization
+// uses (at kSyncFactorTickets, kSyncHelped, kSyncFlag); status: the status word; wleaf: the panel images
 // (kPanelDoubles per 128-block).  each(flops, launch) runs every step's launch (the tracing
 // hook of the handle API); the ticket bases and flag epochs count from the reset, so every
 // call and every replay of a captured call has the same accounting.  bt: a batch of systems of
@@ -87,12 +87,12 @@ void enqueue_factorization(hipStream_t s, T *A, int64_t lda, int64_t n, double *
         if (kp < 0 && fl_upd == 0.0) break;
         const double fl = (kp >= 0 ? panel_flops(n, kp, NB) : 0.0) + fl_upd;
         const uint32_t epoch = (kp >= 0) ? ++epoch_now : epoch_now;
-        uint32_t grid = 0;
+        uint32_t drawn = 0;
         each(fl, [&] {
             launch_factor_step<T>(A, lda, n, kp, k, wleaf, d_info, sync + kSyncFactorTickets, tickets, sync + kSyncFlag,
-                                  epoch, status, s, &grid, prec, wsplit, bt);
+                                  epoch, status, s, &drawn, prec, wsplit, bt);
         });
-        tickets += grid;
+        tickets += drawn;
     }
 }
 

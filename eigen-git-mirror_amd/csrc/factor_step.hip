@@ -286,7 +286,7 @@ static void launch_prec(dim3 grid, hipStream_t s, int K, int KQ, S *A, int64_t l
 template <typename S>
 void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, double *Wleaf, int *info,
                         uint32_t *tickets, uint32_t ticket_base, uint32_t *flag, uint32_t epoch, int *status,
-                        hipStream_t s, uint32_t *grid_out, int prec, __bf16 *Wsplit, const Batch &bt)
+                        hipStream_t s, uint32_t *drawn, int prec, __bf16 *Wsplit, const Batch &bt)
 {
     const int64_t below = n - kp - kNB;  // rows below the panel's diagonal block
     // Helpers of the diagonal role (diag_helper), while each diagonal role and helper has a CU of its own:
@@ -320,7 +320,7 @@ void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, dou
     const int halves = (prec != kPrecBF16x3 && prec != kPrecBF16x6) && 2 * (int64_t)nsyrk * bt.count <= 256 ? 1 : 0;
     nsyrk <<= halves;
     const unsigned grid = (unsigned)(Gp + nsyrk);
-    *grid_out = (uint32_t)Gp;  // tickets drawn
+    *drawn = (uint32_t)Gp;
     if (grid == 0) return;
     const dim3 g(grid, 1, bt.count);
     const int64_t slot = split_slot_elems(n, prec == kPrecBF16x6 ? 3 : 2);

@@ -14,13 +14,14 @@ constexpr int kNB = 128;
 //             (tile (ti, tj), ti > tj, at 256 * (ti(ti-1)/2 + tj), each column-major), then at
 //             kLeafOffset the 8 inverses of its 16 x 16 diagonal leaves (column-major).  The
 //             factorization's diagonal role publishes it for the panel solve, which copies it
-//             to LDS as it is.
+//             to LDS as it is.  Before a panel is stored, the diagonal role's helpers leave the
+//             updated tiles of A in its places (helper_tile).
 //   Winv[b] : L_bb^{-T}, 128 x 128, ld 128 (built for the solve)
 constexpr int64_t kPanelDoubles = 36 * 256;
 constexpr int64_t kLeafOffset = 28 * 256;
-// Per diagonal block b, six 128 x 128 matrices (ld 128): X_b^T, X_b (X_b = L_bb^{-1}), then the
+// Per diagonal block b, eight 128 x 128 matrices (ld 128): X_b^T, X_b (X_b = L_bb^{-1}), then the
 // couplings of the solve M_b = X_b L_{b,b-1}, N_b = X_b^T L_{b+1,b}^T, M2_b = X_b L_{b,b-2},
-// N2_b = X_b^T L_{b+2,b}^T (zero where undefined).
+// N2_b = X_b^T L_{b+2,b}^T, M3_b and N3_b (zero where undefined).
 constexpr int64_t kInvDoubles = 8 * 128 * 128;
 constexpr int64_t kInvX = 128 * 128, kInvM = 2 * 128 * 128, kInvN = 3 * 128 * 128;  // offsets
 constexpr int64_t kInvM2 = 4 * 128 * 128, kInvN2 = 5 * 128 * 128;
@@ -60,27 +61,27 @@ constexpr int MI_PANEL_TIMEOUT = 2;
 constexpr int MI_FACTOR_TICKET = 4;  // a factorization workgroup drew a ticket outside its launch
 
 // Launch k of the factorization: panel of block column kp (or none, kp < 0) + the trailing
-// update by panels k-1, k of the block columns k+2, k+4, ... (none for k < 0).  Writes the grid
-// size (= tickets drawn) to *grid_out.  tickets/flag: persistent words of the handle,
+// update by panels k-1, k of the block columns k+2, k+4, ... (none for k < 0).  Writes the number
+// of tickets that it draws (a panel's workgroups; tiles draw none) to *drawn.  tickets/flag: persistent words of the handle,
 // ticket_base = number of tickets drawn before this launch, epoch = this step's flag value.
 // S = double: FP64 throughout (prec ignored); S = float: FP32 storage, FP64 diagonal factor
 // and panel solve, trailing updates in the MFMA arithmetic `prec` (kPrecF32/BF16/BF16x3);
 // with kPrecBF16x3 / kPrecBF16x6 and Wsplit given, the trailing update reads panels split once
-// into 2 / 3 BF16 parts by the panel solve (4 * split_slot_elems(n, parts) elements, no other
+// into 2 / 3 BF16 parts by the panel solve (kSplitRing * split_slot_elems(n, parts) elements, no other
 // contents needed); without Wsplit, kPrecBF16x6 runs its trailing update on FP32 MFMAs.
 template <typename S>
 void launch_factor_step(S *A, int64_t lda, int64_t n, int64_t kp, int64_t k, double *Wleaf, int *info,
                         uint32_t *tickets, uint32_t ticket_base, uint32_t *flag, uint32_t epoch, int *status,
-                        hipStream_t s, uint32_t *grid_out, int prec, __bf16 *Wsplit = nullptr,
+                        hipStream_t s, uint32_t *drawn, int prec, __bf16 *Wsplit = nullptr,
                         const Batch &bt = Batch());
 // BF16 elements of one part (n rows rounded up to 128, x 128 columns) and of one slot (2 parts
-// for kPrecBF16x3, 3 for kPrecBF16x6) of the split-panel ring (Wsplit, 4 slots).
+// for kPrecBF16x3, 3 for kPrecBF16x6) of the split-panel ring (Wsplit).
 __host__ __device__ inline int64_t split_part_elems(int64_t n) { return ((n + 127) / 128 * 128) * 128; }
 // Slots of the ring of split panels: launch k writes panel k+1's slot while its trailing update
 // reads panels k-7..k (the 2-part split schedule), so 9 are in use at once.
 constexpr int kSplitRing = 16;
 __host__ __device__ inline int64_t split_slot_elems(int64_t n, int parts) { return parts * split_part_elems(n); }
-// Winv[b] = {X_b^T, X_b, M_b, N_b, M2_b, N2_b}, X_b = L_bb^{-1}, for every diagonal block
+// Winv[b] = {X_b^T, X_b, M_b, N_b, M2_b, N2_b, M3_b, N3_b}, X_b = L_bb^{-1}, for every diagonal block
 // (Wleaf: the factorization's panel images, or null for a factor without them).
 // couplings = false: X_b^T and X_b only (for users of Winv other than the solve).
 template <typename T>

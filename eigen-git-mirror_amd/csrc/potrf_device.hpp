@@ -19,15 +19,15 @@ __device__ __forceinline__ int sl(int r, int c)
     const int ti = r >> 4, tj = c >> 4;
     return 256 * ((ti * (ti + 1)) / 2 + tj) + (r & 15) + 16 * (c & 15);
 }
-// Panel p (columns c0..c0+15 of the 128 x 128 block in S, tiled: sl), waves 0 and 1 (2 and 3 are
-// meanwhile busy with the previous panel's deferred update, see potrf_in_lds).  Each row of 16
+// Panel p (columns c0..c0+15 of the 128 x 128 block in S, tiled: sl), waves 0 and 1 (2 and 3
+// meanwhile store the previous panel and update a later column, see potrf_in_lds).  Each row of 16
 // lanes holds the whole 16 x 16 leaf in u (leaf_device.hpp), so its broadcasts need no barrier and
 // no scalar registers; v holds one more row per lane, which takes the same column operations: the
 // up to 112 rows below the leaf (row c0+16+64w+l), for which they are the panel solve A_ip
 // L_pp^{-T}, and in the last 16 lanes of wave 1 (never a row below) the rows of the 16 x 16
 // identity, which become L_pp^{-T}, i.e. column i of X_pp = L_pp^{-1} in lane 48+i, written to xleaf
 // (LDS) column-major.  (With readlane broadcasts and the leaf in lanes 0..15, three waves took a panel in
-// 4300 cycles; this form takes 2900, and two waves are left for the deferred updates.)
+// 4300 cycles; this form takes 2900, and two waves are left for the updates.)
 //
 // Returns the failing panel column or -1, the same in both waves.  The factored leaf is left in u:
 // it is written back to S only after a barrier, since the other wave reads the unfactored leaf from
@@ -633,9 +633,10 @@ __device__ __forceinline__ void diag_helper(int h, const double *__restrict__ A,
 }
 
 // The panel role of one block step; g is the role from the ticket, less the nh helpers' (diag_helper):
-//   role 0   : C = A_kk - P_0 P_0^T straight into LDS, Cholesky in LDS, the panel image
-//              (L11's strictly lower tiles and the leaf inverses) to the workspace, published by
-//              `flag` in three parts, then L11 into A;
+//   role 0   : C = A_kk - P_0 P_0^T straight into LDS (with helpers its tile columns 0 and 1, the others
+//              as the helpers leave them), Cholesky in LDS, the panel image (L11's strictly lower tiles
+//              and the leaf inverses) to the workspace, published by `flag` in three parts, then L11
+//              into A;
 //   role g>0 : the g-th 64 kRowTiles rows below the block: C = A_gk - P_g P_0^T, then rows <-
 //              rows * L11^{-T} with the published image as it comes, stored once.
 // The diagonal role publishes even on a failing pivot, so that no waiter is left behind;

@@ -6,7 +6,7 @@
 //   * the 128 x 128 block is held in LDS and factored in 16-column panels: two waves run the
 //     column loop of LLT.h:320-334 (pivot test, sqrt, scale, rank-1 update) in registers on the
 //     row broadcast, which leaves the inverse of the 16 x 16 leaf too, while the other two
-//     apply the previous panel's rank-16 update to the rest of the block with FP64 MFMA;
+//     store the previous panel and bring the column after next up to date with FP64 MFMA;
 //   * the pivot test is Eigen's `x <= 0 -> fail at column k` (LLT.h:327-330), so a NaN
 //     pivot passes as in Eigen; the first failing column goes to `info` (LAPACK k+1); a last
 //     block narrower than 128 is padded with the identity (L_pad = [L 0; 0 I]);

@@ -159,7 +159,8 @@ int mi_spotrs(mi_llt_handle h, char uplo, int64_t n, int64_t nrhs, const float *
               int64_t ldb);
 
 /* m_l1_norm of LLT::compute (LLT.h:442-453): max column sum of |.| of the symmetric matrix
- * whose `uplo` triangle is stored at dA.  Writes one double to the device pointer d_norm. */
+ * whose `uplo` triangle is stored at dA.  Writes one double to the device pointer d_norm.  Takes
+ * n ceil(n/64) doubles of the handle's workspace (n^2/8 bytes: 537 MB at n = 65536). */
 int mi_dsy_l1norm(mi_llt_handle h, char uplo, int64_t n, const double *dA, int64_t lda,
                   double *d_norm);
 /* The same for float storage (summed in FP64). */
@@ -232,9 +233,10 @@ int mi_dposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n,
 int mi_sposv_vbatched(mi_llt_handle h, char uplo, int64_t batch, const int *d_n, float *const *d_A,
                       const int *d_lda, const int *d_nrhs, float *const *d_B, const int *d_ldb, int *d_info);
 /* Schedule of the batched launch (no reference counterpart; set by the autotuner in
- * mi_llt.batched): workgroups of 4 waves launched per CU (1..64; 3 until it is set), a register-block size (0, 2 or 4; accepted and kept, the kernel's
- * blocks are fixed per precision), and longest-first ordering within the size classes (1) or the
- * given order (0). */
+ * mi_llt.batched): workgroups of 4 waves launched per CU (1..64; 3 until it is set), a
+ * register-block size (0, 2 or 4; accepted and kept, the kernel's blocks are fixed), and
+ * longest-first ordering (1) or the given order (0) within the size classes (n <= 64, 128, 256),
+ * which are taken from the largest on. */
 int mi_llt_set_vbatched_config(mi_llt_handle h, int wg_per_cu, int group, int longest_first);
 int mi_llt_get_vbatched_config(mi_llt_handle h, int *wg_per_cu, int *group, int *longest_first);
 
