@@ -24,7 +24,7 @@
 // left-looking by single tile columns: 26.6 GB a launch of 20,000 systems, 5.7 TB/s beyond L2):
 // with 64-column blocks held by the group a factor of 256 reads its finished columns about twice,
 // and a CU has 2 to 12 systems in flight instead of 8 of any size.  20,000 systems, n ~ U[8, 256]:
-// FP64 4.6 -> 3.1 ms, FP32 3.0 -> 1.9 ms; 700 systems FP64 0.60 -> 0.20 ms.  What bounds it now is
+// FP64 4.6 -> 3.1 ms, FP32 3.0 -> 1.9 ms; 700 systems FP64 0.60 -> 0.19 ms.  What bounds it now is
 // the chain of a system's steps (about 6k cycles per 16 columns with two workgroups on a CU: leaf,
 // two barriers, panel, update; then 3.5k per step of each substitution), not memory: one workgroup
 // per CU takes 4.8 ms.
@@ -371,6 +371,7 @@ struct VbGroup {
 #pragma unroll
                     for (int m = 0; m < 16; ++m) v[m] = m == own ? one : zero;
                     const int f = leaf_factor(u, v);
+                    __builtin_amdgcn_s_setprio(0);
                     lds_order();
                     sy->fail = f >= 0 ? k0 + f + 1 : 0;
                     if (l < 16) {
@@ -431,6 +432,11 @@ struct VbGroup {
                     if (h == 1) {
                         subtract(a, c + 1, 1);
                         give_leaf(a, c + 1);
+                        // The next leaf is the system's chain: until it is done, its wave goes ahead of the
+                        // other workgroup's on its SIMD.  It pays where the largest systems share a CU with
+                        // one other (FP64, 520 systems 203 -> 184 us, 700 202 -> 191, 850 209 -> 198; 1000
+                        // 274 -> 286); 300 and 20,000 take as long without.
+                        if (w == ((c + 1) & (W - 1))) __builtin_amdgcn_s_setprio(2);
                     }
                 }
 #pragma unroll
