@@ -165,7 +165,7 @@ __device__ __forceinline__ void image_store(double *p, double v)
 // as the diagonal role for the rest, and are left with 12 of their 144 MFMAs a row tile when the block
 // is done.  One part, two, and three with diag_helper and half tiles (syrk_tile): 41, 38 and 33 us a
 // launch in FP64 at n <= 1024; factor and solve at n = 3001 1330, 1230 and 1123 us, FP32 at n = 4001
-// 1979, 1850 and 1735 us.
+// 1979, 1850 and 1735 us.  (30 and 1057 us with the helpers' tiles in the image.)
 constexpr int kPart1 = 4, kPart2 = 6;
 
 // Where diag_helper leaves tile (i, j), i >= j, of the updated diagonal block in the panel image (lane
@@ -615,7 +615,8 @@ __device__ __forceinline__ void diag_update_lowp(double *S, const T *__restrict_
 // to the panel image (A_kk itself stays as it is until the block is factored, also when a pivot fails), then
 // helped[h] = epoch.  The update's 36 tiles are 18400 cycles of MFMA on one CU, in front
 // of everything else on the chain; the diagonal role computes the 15 tiles of columns 0 and 1 and needs
-// column 2 a panel's time later, column 4 three panels' time.
+// column 2 a panel's time later, column 4 three panels' time.  A tile is contiguous in the image, so stores
+// and loads need no bounds: a launch at n = 1024 takes 30 us, 33 with the tiles written to A.
 __device__ __forceinline__ void diag_helper(int h, const double *__restrict__ A, int64_t lda, int64_t n, int64_t k0,
                                             double *__restrict__ Wleaf, uint32_t *helped, uint32_t epoch)
 {
@@ -674,7 +675,9 @@ __device__ __forceinline__ void panel_role(int g, int nh, double *smem, int *s_o
         } else {
             block_to_lds(smem, Ck, lda, bs);
         }
-        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag, nh ? helped : nullptr, epoch, status);  // a barrier first
+        const uint32_t *from_helpers = nullptr;
+        if constexpr (sizeof(T) == 8) from_helpers = nh ? helped : nullptr;
+        const int f = potrf_in_lds(smem, xs, s_ok, Wp, flag, from_helpers, epoch, status);  // a barrier first
         if (f >= 0 && tid == 0) atomicCAS(info, 0, (int)(k0 + f + 1));
         global_barrier();  // every wave's stores of the image are in memory
         if (tid == 0) __hip_atomic_store(flag, 8 * epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
